@@ -150,6 +150,12 @@ __device__ __forceinline__ bool claim_vertex(u32* mark, int32_t v, u32 stamp) {
   return atomicExch(&mark[v], stamp) != stamp;
 }
 
+// Appends claimed vertices to the touched list of the iteration whose stamp
+// is `stamp` (the list's length is kept by that iteration's parity).
+__device__ __forceinline__ void touch(const KP& P, bool claimed, int32_t v, u32 stamp) {
+  wave_append<int32_t>(claimed, v, &P.ctl->tcount[stamp & 1u].v, P.touched);
+}
+
 // A wave-uniform pointer into global memory pinned to scalar registers, so
 // accesses through it use the SGPR-base + 32-bit lane-offset addressing form
 // (one VGPR per access instead of a 64-bit per-lane address).
@@ -387,7 +393,7 @@ __device__ __forceinline__ void expand_lanes(const KP& P, int32_t u, int32_t e0,
   load_masks<W>(P, u, bfs_on, dense_t, thr, rshift, bm, sm, far, any_s, t);
   if (lead) {
     const bool c = postpone<W, SPARSE>(P, u, far, stamp, t);
-    if (SPARSE) wave_append<int32_t>(c, u, &P.ctl->tcount.v, P.touched);
+    if (SPARSE) touch(P, c, u, stamp);
   }
   bool any_b = false;
 #pragma unroll
@@ -407,7 +413,7 @@ __device__ __forceinline__ void expand_lanes(const KP& P, int32_t u, int32_t e0,
     }
     ++t.edges;
     const bool claimed = relax_edge<W, SPARSE>(P, u, v, wv, bm, sm, stamp, rshift, thr, t);
-    if (SPARSE) wave_append<int32_t>(claimed, v, &P.ctl->tcount.v, P.touched);
+    if (SPARSE) touch(P, claimed, v, stamp);
   }
 }
 
@@ -467,7 +473,7 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
   }
   {
     const bool c = have && postpone<W, SPARSE>(P, u, far, stamp, t);
-    if (SPARSE) wave_append<int32_t>(c, u, &P.ctl->tcount.v, P.touched);
+    if (SPARSE) touch(P, c, u, stamp);
   }
   const bool work = have && (any_b || any_s);
   const int32_t e0 = work ? P.off[u] : 0;
@@ -507,7 +513,7 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
       ++t.edges;
       claimed = relax_edge<W, SPARSE>(P, uj, v, wv, bj, sj, stamp, rshift, thr, t);
     }
-    if (SPARSE) wave_append<int32_t>(claimed, v, &P.ctl->tcount.v, P.touched);
+    if (SPARSE) touch(P, claimed, v, stamp);
   }
 }
 
@@ -583,7 +589,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
               atomicOr(&P.next[nxt_at<W>(uk, wk)], fm);
             }
           }
-          if (SPARSE) wave_append<int32_t>(claimed, uk, &P.ctl->tcount.v, P.touched);
+          if (SPARSE) touch(P, claimed, uk, stamp);
         }
       }
     }
@@ -694,7 +700,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
             const int wk = __builtin_amdgcn_readlane(myword, k0 + k);
             if (atomicOr(&P.next[nxt_at<W>(vk, wk)], m) == 0) claimed = claim_vertex(P.mark, vk, stamp);
           }
-          wave_append<int32_t>(claimed, vk, &P.ctl->tcount.v, P.touched);
+          touch(P, claimed, vk, stamp);
         }
       }
       // Dense mode: lane k0+k owns edge k0+k's next-word update, one masked
@@ -864,7 +870,7 @@ __device__ __forceinline__ void expand_flat_dense_tab(const KP& P, u32 base, u32
                 ++t.nnew;
                 if (atomicOr(&P.next[nxt_at<W>(vk, wp)], m) == 0) claimed = claim_vertex(P.mark, vk, stamp);
               }
-              wave_append<int32_t>(claimed, vk, &P.ctl->tcount.v, P.touched);
+              touch(P, claimed, vk, stamp);
             }
           }
         }
@@ -987,7 +993,7 @@ __device__ __forceinline__ void expand_flat_narrow(const KP& P, u32 base, u32 n,
             ++t.nnew;
             if (atomicOr(&P.next[nxt_at<W>(myv, myword)], (u64)mg) == 0) claimed = claim_vertex(P.mark, myv, stamp);
           }
-          wave_append<int32_t>(claimed, myv, &P.ctl->tcount.v, P.touched);
+          touch(P, claimed, myv, stamp);
         }
       }
     };
@@ -1208,14 +1214,14 @@ __device__ __forceinline__ void advance_push_body(const KP& P, u32* s_item, Tall
       const int32_t v = P.pull_hi[i];
       bool claimed = false;
       if (pull_vertex_wave<W, SPARSE>(P, v, bb, stamp, t) && lane == 0) claimed = true;
-      if (SPARSE) wave_append<int32_t>(claimed, v, &C->tcount.v, P.touched);
+      if (SPARSE) touch(P, claimed, v, stamp);
     }
     const int64_t nLo = P.n_pull_lo;
     for (int64_t base = (int64_t)blockIdx.x * BS; base < nLo; base += (int64_t)gridDim.x * BS) {
       const int64_t i = base + threadIdx.x;
       const int32_t v = i < nLo ? P.pull_lo[i] : 0;
       const bool claimed = i < nLo && pull_vertex<W, SPARSE>(P, v, bb, stamp, t);
-      if (SPARSE) wave_append<int32_t>(claimed, v, &C->tcount.v, P.touched);
+      if (SPARSE) touch(P, claimed, v, stamp);
     }
   }
 }
@@ -1229,8 +1235,9 @@ __device__ __forceinline__ void flush_near_far(const KP& P, const Tally& t, u32 
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) fm = min(fm, (u32)__shfl_xor((int)fm, d, 64));
   if (lane_id() == 0) {
-    if (anyn) atomicOr(&P.ctl->near_new, 1u);
-    if (fm != INF) atomicMin(&P.ctl->far_min, fm);
+    Stripe& st = P.ctl->stripe[blockIdx.x % NSTRIPE];
+    if (anyn) atomicOr(&st.near_new, 1u);
+    if (fm != INF) atomicMin(&st.far_min, fm);
   }
 }
 
@@ -1265,7 +1272,7 @@ __global__ __launch_bounds__(BS) void k_adv_dense(KP P) {
   const u32 iter = C->iter, p = iter & 1u;
   const u32 nD = C->bcount[p][3].v;
   if (nD == 0) return;
-  if (threadIdx.x == 0) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     const u64 now = (u64)wall_clock64();
     atomicMin(&C->adv_t0, now);
     atomicMin(&C->den_t0, now);
@@ -1304,9 +1311,10 @@ __global__ __launch_bounds__(BS) void k_adv_dense(KP P) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    Stripe& st = C->stripe[blockIdx.x % NSTRIPE];
     const u64 now = (u64)wall_clock64();
-    atomicMax(&C->adv_t1, now);
-    atomicMax(&C->den_t1, now);
+    atomicMax(&st.adv_t1, now);
+    atomicMax(&st.den_t1, now);
   }
 }
 
@@ -1319,7 +1327,7 @@ __global__ __launch_bounds__(BLOCK) void k_adv_narrow(KP P) {
   const u32 iter = C->iter, p = iter & 1u;
   const u32 nN = C->bcount[p][4].v;
   if (nN == 0) return;
-  if (threadIdx.x == 0) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
     const u64 now = (u64)wall_clock64();
     atomicMin(&C->adv_t0, now);
     atomicMin(&C->den_t0, now);
@@ -1343,9 +1351,10 @@ __global__ __launch_bounds__(BLOCK) void k_adv_narrow(KP P) {
   }
   __syncthreads();
   if (threadIdx.x == 0) {
+    Stripe& st = C->stripe[blockIdx.x % NSTRIPE];
     const u64 now = (u64)wall_clock64();
-    atomicMax(&C->adv_t1, now);
-    atomicMax(&C->den_t1, now);
+    atomicMax(&st.adv_t1, now);
+    atomicMax(&st.den_t1, now);
   }
 }
 
@@ -1417,7 +1426,7 @@ __device__ __forceinline__ void pull_sssp_item(const KP& P, u64 item, int rshift
   }
   if (SPARSE) {
     const bool c = lane == 0 && claimed && claim_vertex(P.mark, v, stamp);
-    wave_append<int32_t>(c, v, &P.ctl->tcount.v, P.touched);
+    touch(P, c, v, stamp);
   }
 }
 
@@ -1425,7 +1434,7 @@ template <int W>
 __global__ __launch_bounds__(BLOCK) void k_pull_sssp(KP P) {
   Ctl* C = P.ctl;
   if (C->finished || !C->sssp_pull) return;
-  if (threadIdx.x == 0) atomicMin(&C->adv_t0, (u64)wall_clock64());
+  if (blockIdx.x == 0 && threadIdx.x == 0) atomicMin(&C->adv_t0, (u64)wall_clock64());
   const u32 iter = C->iter, p = iter & 1u;
   const u32 stamp = C->stamp_base + iter + 1;
   const int rshift = P.cfg->rshift;
@@ -1448,7 +1457,7 @@ __global__ __launch_bounds__(BLOCK) void k_pull_sssp(KP P) {
     prof_add(P, PF_NEW_WORDS, t.nnew);
   }
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&C->adv_t1, (u64)wall_clock64());
+  if (threadIdx.x == 0) atomicMax(&C->stripe[blockIdx.x % NSTRIPE].adv_t1, (u64)wall_clock64());
 }
 
 // (vertex << 32 | chunk) items of every vertex with edges, PCHUNK edges each
@@ -1478,14 +1487,18 @@ __global__ __launch_bounds__(BS) void k_adv_push(KP P) {
   Ctl* C = P.ctl;
   if (C->finished) return;
   __shared__ u32 s_item;
-  if (threadIdx.x == 0) atomicMin(&C->adv_t0, (u64)wall_clock64());
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    atomicMin(&C->adv_t0, (u64)wall_clock64());
+    C->f_iter = C->iter;
+    C->f_scan = C->dense_mode;
+  }
   Tally t;
   if (C->dense_mode) advance_push_body<W, false, BS>(P, &s_item, t);
   else advance_push_body<W, true, BS>(P, &s_item, t);
   flush_near_far(P, t, C->thr);
   if (P.profile) flush_tally(P, t);
   __syncthreads();
-  if (threadIdx.x == 0) atomicMax(&C->adv_t1, (u64)wall_clock64());
+  if (threadIdx.x == 0) atomicMax(&C->stripe[blockIdx.x % NSTRIPE].adv_t1, (u64)wall_clock64());
 }
 
 // ------------------------------------------------------------------ seed
@@ -1499,6 +1512,10 @@ __global__ __launch_bounds__(BLOCK) void k_seed(KP P, const int32_t* slot_src, i
   // Stamp of the iteration whose filter settles the seeds (stamp_base itself
   // for the batch seeding pass, which runs at iteration 0xFFFFFFFF).
   const u32 stamp = C->stamp_base + C->iter + 1u;
+  if (s == 0) {
+    C->f_iter = C->iter;
+    C->f_scan = C->dense_mode;
+  }
   bool claimed = false;
   int32_t v = 0;
   if (s < nslots && slot_src[s] >= 0) {
@@ -1507,11 +1524,11 @@ __global__ __launch_bounds__(BLOCK) void k_seed(KP P, const int32_t* slot_src, i
     atomicOr(&P.next[nxt_at<W>(v, w)], 1ull << q);
     if ((P.cfg->val_bits[w] >> q) & 1ull) {
       P.vals[vrow(P.V, w, v, P.cfg->rshift) + q] = 0u;
-      atomicOr(&C->near_new, 1u);  // a source at value 0 is below any threshold
+      atomicOr(&C->stripe[0].near_new, 1u);  // a source at value 0 is below any threshold
     }
     claimed = claim_vertex(P.mark, v, stamp);
   }
-  wave_append<int32_t>(claimed, v, &C->tcount.v, P.touched);
+  touch(P, claimed, v, stamp);
 }
 
 // ------------------------------------------------------------------ filter
@@ -1556,11 +1573,18 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   if (C->finished) return;
   __shared__ int s_last;
   __shared__ u32 s_res[(BLOCK / 64 + 1) * 5];
-  if (threadIdx.x == 0) atomicMin(&C->flt_t0, (u64)wall_clock64());
   const Cfg* cfg = P.cfg;
-  const u32 iter = C->iter, p = iter & 1u, np = p ^ 1u;
-  const bool scan = C->dense_mode != 0;
-  const u32 n = scan ? (u32)P.scan_v : C->tcount.v;
+  const u32 iter = C->f_iter, p = iter & 1u, np = p ^ 1u;
+  const u32 stamp = C->stamp_base + iter + 1u;
+  const bool scan = C->f_scan != 0;
+  const u32 n = scan ? (u32)P.scan_v : C->tcount[stamp & 1u].v;
+  // Workgroups with vertices to look at; the others leave at once (with one
+  // touched vertex the launch took 50 us on 777 777 vertices and 52 us on
+  // RMAT-22 while all workgroups reported; 12 and 8 us since).
+  const u32 active = max(1u, min(gridDim.x, (n + BLOCK * FK - 1) / (BLOCK * FK)));
+  if (blockIdx.x >= active) return;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    __hip_atomic_store(&C->flt_t0, (u64)wall_clock64(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const int rshift = cfg->rshift, dense_t = cfg->dense_t;
   const int lane = lane_id();
   u64 bb[W], vb[W], un[W];
@@ -1578,8 +1602,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   // bin counters are single addresses every workgroup contends for (one
   // reservation per 256 vertices cost about 0.3 ms per dense iteration on
   // RMAT-22).
-  constexpr int FK = 4;
-  const u32 gstride = gridDim.x * BLOCK * FK;
+  const u32 gstride = active * BLOCK * FK;
   // The next iteration's bin lists, picked once (indexing the argument's
   // arrays with np inside the loop made the compiler copy the whole
   // argument block to scratch memory).
@@ -1727,89 +1750,134 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       }
     }
   }
-  // Frontier statistics: wave sums, then one atomic per workgroup and counter.
+  // Frontier statistics: wave sums, combined per workgroup into its line of
+  // P.fstat, which the last workgroup adds up.  (One atomic per workgroup and
+  // counter took 145-175 us per scan of RMAT-22's vertices, whatever it found.)
+  constexpr int NW = BLOCK / 64;
+  __shared__ u64 s_st[NW * FSTAT];
+  __shared__ u64 s_red[(BLOCK / FSTAT) * FSTAT];
+  __shared__ u64 s_tot[FSTAT];
+  __shared__ u32 s_cnt[10];  // the five lists' lengths: next frontier, consumed frontier
+  __shared__ Stripe s_stripe;
+  const int tid = (int)threadIdx.x;
+  static_assert(NSUM + MAXW <= FSTAT && FSTAT <= 64, "a statistics line is written by one wave");
   {
-    constexpr int NS = 6;  // sums per wave before the union words
-    __shared__ u64 s_st[(BLOCK / 64) * (NS + MAXW)];
-    const int wave = (int)(threadIdx.x >> 6);
-    u64 sums[NS] = {pairs, epairs, fedges, apairs, averts, aqedges};
+    u64 sums[NSUM] = {pairs, epairs, fedges, apairs, averts, aqedges};
 #pragma unroll
-    for (int i = 0; i < NS; ++i) sums[i] = wave_sum64(sums[i]);
+    for (int i = 0; i < NSUM; ++i) sums[i] = wave_sum64(sums[i]);
     u64 unw[W];
 #pragma unroll
     for (int w = 0; w < W; ++w) unw[w] = wave_or64(un[w]);
     if (lane == 0) {
-      u64* r = s_st + wave * (NS + MAXW);
+      u64* r = s_st + (tid >> 6) * FSTAT;
 #pragma unroll
-      for (int i = 0; i < NS; ++i) r[i] = sums[i];
+      for (int i = 0; i < NSUM; ++i) r[i] = sums[i];
 #pragma unroll
-      for (int w = 0; w < W; ++w) r[NS + w] = unw[w];
+      for (int w = 0; w < W; ++w) r[NSUM + w] = unw[w];
     }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      u64 tot[NS], tu[W];
-#pragma unroll
-      for (int i = 0; i < NS; ++i) tot[i] = 0;
-#pragma unroll
-      for (int w = 0; w < W; ++w) tu[w] = 0;
-      for (int wv = 0; wv < BLOCK / 64; ++wv) {
-        const u64* r = s_st + wv * (NS + MAXW);
-#pragma unroll
-        for (int i = 0; i < NS; ++i) tot[i] += r[i];
-#pragma unroll
-        for (int w = 0; w < W; ++w) tu[w] |= r[NS + w];
+  }
+  __syncthreads();
+  if (tid < 64) {
+    if (tid < NSUM + W) {
+      u64 x = s_st[tid];
+      for (int wv = 1; wv < NW; ++wv) {
+        const u64 y = s_st[wv * FSTAT + tid];
+        x = tid < NSUM ? x + y : x | y;
       }
-      if (tot[0]) atomicAdd(&C->bfs_pairs[np], tot[0]);
-      if (tot[1]) atomicAdd(&C->bfs_edges[np], tot[1]);
-      if (tot[2]) atomicAdd(&C->fedges[np], tot[2]);
-      if (tot[3]) atomicAdd(&C->npairs[np], tot[3]);
-      if (tot[4]) atomicAdd(&C->nverts[np], tot[4]);
-      if (tot[5]) atomicAdd(&C->nqedges[np], tot[5]);
-#pragma unroll
-      for (int w = 0; w < W; ++w)
-        if (tu[w]) atomicOr(&C->union_[w], tu[w]);
+      __hip_atomic_store(&P.fstat[(size_t)blockIdx.x * FSTAT + tid], x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    // The line is in memory (agent-scope stores complete there) before this
+    // wave counts its workgroup as done; nothing else that other workgroups
+    // read in this launch is left by plain stores.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (tid == 0) {
+      // Many workgroups count on NSTRIPE lines first, the last of each line on
+      // the common one.
+      if (active <= 2 * NSTRIPE) {
+        s_last = atomicAdd(&C->done[NSTRIPE].v, 1u) == active - 1;
+      } else {
+        const u32 st = blockIdx.x % NSTRIPE;
+        const u32 members = (active - st + NSTRIPE - 1) / NSTRIPE;
+        s_last = atomicAdd(&C->done[st].v, 1u) == members - 1 && atomicAdd(&C->done[NSTRIPE].v, 1u) == NSTRIPE - 1;
+      }
     }
   }
-  // Last workgroup: advance the state machine.
   __syncthreads();
-  if (threadIdx.x == 0) {
-    __threadfence();
-    const u32 t = atomicAdd(&C->done_blocks.v, 1u);
-    s_last = (t == gridDim.x - 1);
+  if (!s_last) return;
+  // Last workgroup: advance the state machine.  Its threads collect what the
+  // iteration left, and reset the consumed counters, side by side; then one
+  // thread decides.
+  {
+    // Thread (g, k): entry k of every (BLOCK / FSTAT)-th line.
+    const int k = tid % FSTAT, g = tid / FSTAT;
+    u64 x = 0;
+    if (k < NSUM + W)
+      for (u32 b = (u32)g; b < active; b += BLOCK / FSTAT) {
+        const u64 y =
+            __hip_atomic_load(&P.fstat[(size_t)b * FSTAT + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        x = k < NSUM ? x + y : x | y;
+      }
+    s_red[g * FSTAT + k] = x;
+  }
+  if (tid < 10) {
+    Ctr& c = C->bcount[tid < 5 ? np : p][tid % 5];
+    s_cnt[tid] = __hip_atomic_load(&c.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (tid >= 5) c.v = 0;
+  } else if (tid < 10 + 7) {
+    C->fetch[p][tid - 10].v = 0;
+  } else if (tid < 17 + NSTRIPE + 1) {
+    C->done[tid - 17].v = 0;
+  } else if (tid == 17 + NSTRIPE + 1) {
+    C->tcount[(stamp & 1u) ^ 1u].v = 0;  // filled next; this iteration's is reset by the next filter
+  }
+  if (tid >= 64 && tid < 128) {
+    // One wave combines the stripes.
+    const int i = tid - 64;
+    Stripe x{0, 0, INF, 0};
+    if (i < NSTRIPE) {
+      x = C->stripe[i];
+      C->stripe[i] = Stripe{0, 0, INF, 0};
+    }
+#pragma unroll
+    for (int d = NSTRIPE / 2; d >= 1; d >>= 1) {
+      const u64 a1 = shfl64(x.adv_t1, lane ^ d), d1 = shfl64(x.den_t1, lane ^ d);
+      x.adv_t1 = max(x.adv_t1, a1);
+      x.den_t1 = max(x.den_t1, d1);
+      x.far_min = min(x.far_min, (u32)__shfl_xor((int)x.far_min, d, 64));
+      x.near_new |= (u32)__shfl_xor((int)x.near_new, d, 64);
+    }
+    if (i == 0) s_stripe = x;
+  } else if (tid >= 128 && tid < 128 + 5 * NSHARD) {
+    C->shard[p][(tid - 128) / NSHARD][(tid - 128) % NSHARD].v = 0;
   }
   __syncthreads();
-  if (s_last && threadIdx.x == 0) {
-    __threadfence();
-    const u32 total = atomicAdd(&C->bcount[np][0].v, 0u) + atomicAdd(&C->bcount[np][1].v, 0u) +
-                      atomicAdd(&C->bcount[np][2].v, 0u) + atomicAdd(&C->bcount[np][3].v, 0u) +
-                      atomicAdd(&C->bcount[np][4].v, 0u);
-    const u64 fp = atomicAdd(&C->bfs_pairs[np], 0ull), fe = atomicAdd(&C->bfs_edges[np], 0ull);
-    const u64 fall = atomicAdd(&C->fedges[np], 0ull);
-    const u64 napairs = atomicAdd(&C->npairs[np], 0ull), naverts = atomicAdd(&C->nverts[np], 0ull),
-              naqedges = atomicAdd(&C->nqedges[np], 0ull);
-    C->dense_mode = fall >= cfg->dense_fedges_thr ? 1u : 0u;
-    C->fedges[p] = 0;
-    C->npairs[p] = C->nverts[p] = C->nqedges[p] = 0;
+  if (tid < FSTAT) {
+    u64 x = 0;
+    for (int g = 0; g < BLOCK / FSTAT; ++g) {
+      const u64 y = s_red[g * FSTAT + tid];
+      x = tid < NSUM ? x + y : x | y;
+    }
+    s_tot[tid] = x;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const u32 total = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3] + s_cnt[4];
+    const u32 cur_items = s_cnt[5] + s_cnt[6] + s_cnt[7] + s_cnt[8] + s_cnt[9];
+    const u64 fp = s_tot[0], fe = s_tot[1], fall = s_tot[2];
+    const u64 napairs = s_tot[3], naverts = s_tot[4], naqedges = s_tot[5];
+    const u32 cur_pull = C->bfs_pull, cur_spull = C->sssp_pull;
+    const u32 dense = fall >= cfg->dense_fedges_thr ? 1u : 0u;
+    C->dense_mode = dense;
     u64 consumed[MAXW];
     for (int w = 0; w < MAXW; ++w) {
       consumed[w] = C->last_union[w];
-      C->last_union[w] = atomicAnd(&C->union_[w], 0ull);
+      C->last_union[w] = w < W ? s_tot[NSUM + w] : 0ull;
     }
-    const u32 cur_items = C->bcount[p][0].v + C->bcount[p][1].v + C->bcount[p][2].v + C->bcount[p][3].v + C->bcount[p][4].v;
-    C->tcount.v = 0;
-    C->bcount[p][0].v = C->bcount[p][1].v = C->bcount[p][2].v = C->bcount[p][3].v = C->bcount[p][4].v = 0;
-    for (int k = 0; k < 7; ++k) C->fetch[p][k].v = 0;
-    for (int k = 0; k < 5; ++k)
-      for (int s = 0; s < NSHARD; ++s) C->shard[p][k][s].v = 0;
-    C->bfs_pairs[p] = 0;
-    C->bfs_edges[p] = 0;
-    C->done_blocks.v = 0;
-    const u32 cur_pull = C->bfs_pull;
     u32 pull = 0;
     if (fp > 0) {
       if (cfg->pull_policy == 1) pull = 1;
       else if (cfg->pull_policy == 2) {
-        if (C->bfs_pull) pull = fp >= cfg->push_pairs_thr ? 1u : 0u;
+        if (cur_pull) pull = fp >= cfg->push_pairs_thr ? 1u : 0u;
         else pull = (fp >= cfg->pull_pairs_thr || fe >= cfg->pull_edges_thr) ? 1u : 0u;
       }
     }
@@ -1817,7 +1885,6 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     // SSSP pull for the next iteration, on the same ratios applied to the
     // SSSP (vertex, query) pairs of the next frontier (every pair that is
     // not BFS: WCC queries have no frontier) and their degree-weighted count.
-    const u32 cur_spull = C->sssp_pull;
     u32 spull = 0;
     {
       const u64 sp = napairs - fp, se = naqedges - fe;
@@ -1833,20 +1900,19 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     // Near-far: when no SSSP pair below the threshold is left, move it to
     // the smallest pending value plus delta (skipping empty buckets).
     if (cfg->delta != 0) {
-      const u32 fm = C->far_min;
-      if (C->near_new == 0 && fm != INF) {
+      const u32 fm = s_stripe.far_min;
+      if (s_stripe.near_new == 0 && fm != INF) {
         const u64 nt = (u64)fm + (u64)cfg->delta;
         C->thr = nt >= (u64)INF ? INF : (u32)nt;
         ++C->bumps;
       }
-      C->near_new = 0;
-      C->far_min = INF;
     }
     // Launch timing and the iteration record: the advance of this iteration
     // ran iff iter != seeding.
     if (iter != 0xFFFFFFFFu) {
-      const u64 at = C->adv_t1 - C->adv_t0, ft = (u64)wall_clock64() - C->flt_t0;
-      const u64 dt = C->den_t1 > C->den_t0 ? C->den_t1 - C->den_t0 : 0ull;
+      const u64 den_t0 = C->den_t0, now = (u64)wall_clock64();
+      const u64 at = s_stripe.adv_t1 - C->adv_t0, ft = now - __hip_atomic_load(&C->flt_t0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const u64 dt = s_stripe.den_t1 > den_t0 ? s_stripe.den_t1 - den_t0 : 0ull;
       C->adv_ticks += at;
       C->adv_launches += 1;
       C->flt_ticks += ft;
@@ -1871,7 +1937,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
         r.next_vertices = naverts;
         r.next_qedges = naqedges;
         r.edges_scanned = C->prof[PF_PUSH_EDGES] + C->prof[PF_DENSE_EDGES] + C->prof[PF_PULL_EDGES];
-        r.t_end = (u64)wall_clock64();
+        r.t_end = now;
         for (int w = 0; w < MAXW; ++w) r.fr_union[w] = consumed[w];
       }
     } else {
@@ -1883,10 +1949,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       C->t_start = (u64)wall_clock64();
     }
     C->adv_t0 = ~0ull;
-    C->adv_t1 = 0;
     C->den_t0 = ~0ull;
-    C->den_t1 = 0;
-    C->flt_t0 = ~0ull;
     const u32 next_iter = iter + 1u;
     C->iter = next_iter;
     if (total == 0 || (C->max_iter != 0 && next_iter >= C->max_iter)) {
@@ -1894,9 +1957,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     } else {
       if (pull || spull) ++C->pull_iters;
       else ++C->push_iters;
-      if (C->dense_mode) ++C->dense_iters;
+      if (dense) ++C->dense_iters;
     }
-    __threadfence();
   }
 }
 
@@ -2843,14 +2905,9 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
       add_depth_planes(en, W, 4, false);  // depths below 16
     }
     // Control block.
-    Ctl& c = *en->h_ctl;
-    std::memset(&c, 0, sizeof(Ctl));
+    Ctl& c = en->fresh_ctl();
     c.iter = 0xFFFFFFFFu;
     c.thr = cfg.delta ? cfg.delta : INF;
-    c.far_min = INF;
-    c.adv_t0 = ~0ull;
-    c.den_t0 = ~0ull;
-    c.flt_t0 = ~0ull;
     if (en->stamp_epoch > 0xF0000000u) {
       HIP_CHECK(hipMemsetAsync(en->mark.p, 0, (size_t)V * 4, en->s));
       en->stamp_epoch = 1;
@@ -3529,6 +3586,7 @@ cgp_status cgp_engine_create(const cgp_graph* g, const cgp_engine_opts* opts, cg
     HIP_CHECK(hipEventCreateWithFlags(&en->ev_join, hipEventDisableTiming));
     HIP_CHECK(hipMalloc((void**)&en->d_ctl, sizeof(Ctl)));
     HIP_CHECK(hipMalloc((void**)&en->d_cfg, sizeof(Cfg)));
+    HIP_CHECK(hipMalloc((void**)&en->d_fstat, (size_t)en->grid_filter() * FSTAT * sizeof(u64)));
     HIP_CHECK(hipHostMalloc((void**)&en->h_ctl, sizeof(Ctl), hipHostMallocDefault));
     HIP_CHECK(hipHostMalloc((void**)&en->h_cfg, sizeof(Cfg), hipHostMallocDefault));
     HIP_CHECK(hipMemset(en->d_ctl, 0, sizeof(Ctl)));
@@ -3557,6 +3615,7 @@ void cgp_engine_destroy(cgp_engine* en) {
   for (hipEvent_t e : en->ev_pool) (void)hipEventDestroy(e);
   if (en->d_ctl) (void)hipFree(en->d_ctl);
   if (en->d_cfg) (void)hipFree(en->d_cfg);
+  if (en->d_fstat) (void)hipFree(en->d_fstat);
   if (en->h_ctl) (void)hipHostFree(en->h_ctl);
   if (en->h_cfg) (void)hipHostFree(en->h_cfg);
   if (en->h_stage) (void)hipHostFree(en->h_stage);

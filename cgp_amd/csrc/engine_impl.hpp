@@ -148,6 +148,7 @@ struct cgp_engine {
   cgpi::DevBuf pull_items;  // SSSP pull items of the graph, built on first use
   int64_t n_pull_items = 0;
   Ctl* d_ctl = nullptr;
+  u64* d_fstat = nullptr;   // statistics lines of the filter's workgroups
   Cfg* d_cfg = nullptr;
   Ctl* h_ctl = nullptr;     // pinned
   Cfg* h_cfg = nullptr;     // pinned
@@ -222,6 +223,7 @@ struct cgp_engine {
     P.ctl = d_ctl;
     P.cfg = d_cfg;
     P.iters = (cgpk::IterRec*)iters.p;
+    P.fstat = d_fstat;
     P.bin_small = opts.bin_small;
     P.bin_large = opts.bin_large;
     // Serving seeds queries into running iterations, where a full scan must
@@ -257,9 +259,11 @@ struct cgp_engine {
     return (int)std::max<int64_t>(cus, std::min<int64_t>(want, (int64_t)cus * 8));
   }
   int grid_advance() const { return (int)((int64_t)advance_blocks() * 256 / std::max(128, opts.block_size)); }
+  // Filter workgroups: no more than have vertices to look at (each looks at
+  // BLOCK * FK per step), at most four per CU.
   int grid_filter() const {
-    int64_t need = ((int64_t)g->V + BLOCK - 1) / BLOCK;
-    return (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cus * 8));
+    int64_t need = ((int64_t)g->V + BLOCK * cgpk::FK - 1) / (BLOCK * cgpk::FK);
+    return (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cus * 4));
   }
 
   void ensure_words(int W) {
@@ -286,6 +290,15 @@ struct cgp_engine {
       }
     }
     if (moved) drop_graphs();
+  }
+
+  // Zeroed control block in h_ctl with the fields whose start is not zero.
+  Ctl& fresh_ctl() {
+    Ctl& c = *h_ctl;
+    std::memset((void*)&c, 0, sizeof(Ctl));
+    c.adv_t0 = c.den_t0 = c.flt_t0 = ~0ull;
+    for (cgpk::Stripe& x : c.stripe) x.far_min = INF;
+    return c;
   }
 
   void ensure_pull_items();  // engine.hip

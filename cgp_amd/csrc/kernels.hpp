@@ -60,6 +60,16 @@ constexpr int PCHUNK = 256;        // edges per SSSP pull item
 // spread over NSHARD lines instead of one.
 constexpr int NSHARD = 8;
 enum : int { SH_M = 0, SH_S, SH_D, SH_N, SH_P };
+// Workgroups spread their end-of-launch atomics over NSTRIPE lines (by
+// workgroup index); the filter's last workgroup combines them.  One line takes
+// about 12 ns per atomic whoever sends it, so 2048 workgroups on one line were
+// 25 us per counter.
+constexpr int NSTRIPE = 16;
+constexpr int FK = 4;              // vertices per thread and step of the filter
+// Frontier statistics a filter workgroup leaves for the last one, in u64s of
+// one 128-byte line per workgroup: six sums, then the union of each word.
+constexpr int FSTAT = 16;
+constexpr int NSUM = 6;
 
 // Per-batch slot configuration (device resident, rewritten per pass).
 struct Cfg {
@@ -105,6 +115,14 @@ struct alignas(256) Ctr {
   u32 v;
 };
 
+// What a workgroup contributes at the end of a launch: its end time (advance
+// and lane-per-query launch), and the near-far state of its SSSP improvements.
+struct alignas(256) Stripe {
+  u64 adv_t1, den_t1;
+  u32 far_min;   // min value of the pairs postponed or improved to >= thr this iteration
+  u32 near_new;  // nonzero when this iteration produced an SSSP pair below thr
+};
+
 // Device control block: counters and the iteration state machine.
 struct Ctl {
   u32 iter;         // iteration of the current run (0xFFFFFFFF during seeding)
@@ -119,38 +137,35 @@ struct Ctl {
   u32 dense_iters;
   u32 thr;          // SSSP near-far threshold: frontier pairs with value >= thr are postponed
                     // (INF: every pair expands, Bellman-Ford frontier)
-  u32 far_min;      // min value of the pairs postponed or improved to >= thr this iteration
-  u32 near_new;     // nonzero when this iteration produced an SSSP pair below thr
   u32 bumps;        // threshold raises so far
-  u32 pad;
-  u64 bfs_pairs[2];           // BFS frontier (vertex, query) pairs, by parity
-  u64 bfs_edges[2];           // ... weighted by degree
-  u64 fedges[2];              // summed degree of the next frontier's vertices
-  u64 union_[MAXW];           // OR of next words in the running filter
+  // The running iteration as its filter sees it, written by the kernel before
+  // it (advance or seeding): the filter's last workgroup moves iter and
+  // dense_mode on while workgroups without work may not have started yet.
+  u32 f_iter;
+  u32 f_scan;       // that iteration's dense_mode
   u64 last_union[MAXW];       // OR of the frontier words the last filter produced
   u64 prof[NPROF];            // work counters (profile mode)
-  // Device-clock launch timing (wall_clock64 ticks): first workgroup start
-  // and last workgroup end of the running advance / filter, and the sums
-  // over the launches of the run that did work.
-  u64 adv_t0, adv_t1, flt_t0, den_t0, den_t1;
+  // Device-clock launch timing (wall_clock64 ticks): start of the running
+  // advance / filter (its first workgroup), and the sums over the launches of
+  // the run that did work; the ends are in the stripes.
+  u64 adv_t0, flt_t0, den_t0;
   u64 adv_ticks, flt_ticks, adv_launches, den_ticks, den_launches;
-  // Frontier statistics of the filter being run (all kinds): (vertex, query)
-  // pairs, distinct vertices and query-weighted degree of the next frontier;
-  // the seeding filter's values are kept as the sizes of frontier 0.
-  u64 npairs[2], nverts[2], nqedges[2];
+  // Sizes of frontier 0 (from the seeding filter): (vertex, query) pairs,
+  // distinct vertices, their summed degree and the query-weighted degree.
   u64 seed_pairs, seed_verts, seed_edges, seed_qedges;
   u64 t_start;  // device clock at the end of the seeding filter
   // Counters hit by atomics from every wave or workgroup, each on its own
   // line (the host never reads them: it copies back only the fields above).
-  Ctr tcount;                 // touched-list length
-  Ctr done_blocks;            // filter last-workgroup detection
+  Stripe stripe[NSTRIPE];     // by workgroup index
+  Ctr tcount[2];              // touched-list length, by parity of the iteration that fills it
+  Ctr done[NSTRIPE + 1];      // filter last-workgroup detection: by workgroup index, then all
   Ctr bcount[2][5];           // [parity][small, medium, large items, dense items, narrow dense items]
   Ctr fetch[2][7];            // [parity] work cursors of the advance without shards (L, D, unused,
                               // unused, pull-high, unused, unused)
   Ctr shard[2][5][NSHARD];    // [parity][M, S, unused, N, SSSP pull] per-shard work cursors
 };
 // Bytes of Ctl the host reads back after a run of iterations.
-constexpr size_t CTL_HOST_BYTES = offsetof(Ctl, tcount);
+constexpr size_t CTL_HOST_BYTES = offsetof(Ctl, stripe);
 
 // Per-iteration record, written by the filter's last workgroup into a ring
 // of ITER_RING entries (index = iteration % ITER_RING), no host sync.
@@ -204,6 +219,7 @@ struct KP {
   Ctl* ctl;
   const Cfg* cfg;
   IterRec* iters;
+  u64* fstat;  // FSTAT words per filter workgroup
   int32_t bin_small;
   int32_t bin_large;
   // Vertices a full compaction scan visits: [0, scan_v).  On a symmetric

@@ -449,18 +449,13 @@ cgp_status cgp_serve_start(cgp_engine* en, const cgp_serve_opts* so) {
     cfg.dense_t = en->opts.dense_threshold;
     cfg.delta = (u32)en->opts.sssp_delta;
     cfg.dense_fedges_thr = std::max<u64>(1, (u64)V / (u64)en->opts.frontier_dense_div);
-    Ctl& c = *en->h_ctl;
-    std::memset(&c, 0, sizeof(Ctl));
-    c.iter = 0;
+    Ctl& c = en->fresh_ctl();
     c.thr = cfg.delta ? cfg.delta : INF;
-    c.far_min = INF;
     if (en->stamp_epoch > 0xE0000000u) {
       HIP_CHECK(hipMemsetAsync(en->mark.p, 0, (size_t)V * 4, en->s));
       en->stamp_epoch = 1;
     }
     c.stamp_base = en->stamp_epoch;
-    c.adv_t0 = ~0ull;
-    c.flt_t0 = ~0ull;
     HIP_CHECK(hipMemcpyAsync(en->d_cfg, &cfg, sizeof(Cfg), hipMemcpyHostToDevice, en->s));
     HIP_CHECK(hipMemcpyAsync(en->d_ctl, &c, sizeof(Ctl), hipMemcpyHostToDevice, en->s));
     HIP_CHECK(hipStreamSynchronize(en->s));

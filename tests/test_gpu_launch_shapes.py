@@ -1,0 +1,59 @@
+"""GPU parity at the sizes where a launch changes shape: the edges of a
+workgroup's share of vertices, edges and work items, and lists shorter and
+longer than the launch has waves.  Every row is compared with the oracle."""
+import numpy as np
+import pytest
+
+import cgp_amd
+import oracle_lib as O
+from cgp_amd import BFS, SSSP, WCC
+
+pytestmark = pytest.mark.gpu
+
+
+def ring_graph(V, hub_degree=0, seed=1, chords=3, directed=False):
+    """A ring of V vertices with random chords; vertex V // 2 is joined to
+    hub_degree others."""
+    rng = np.random.RandomState(seed)
+    a, b = [np.arange(V)], [(np.arange(V) + 1) % max(V, 1)]
+    if V > 4:
+        a.append(rng.randint(0, V, chords * V))
+        b.append(rng.randint(0, V, chords * V))
+    if hub_degree:
+        a.append(np.full(hub_degree, V // 2))
+        b.append(rng.choice(V, hub_degree, replace=False))
+    a, b = np.concatenate(a), np.concatenate(b)
+    a, b = a[a != b], b[a != b]
+    if not directed:
+        a, b = np.concatenate([a, b]), np.concatenate([b, a])
+    key = np.unique(a.astype(np.int64) * V + b)
+    src, dst = key // V, key % V
+    lo, hi = np.minimum(src, dst), np.maximum(src, dst)
+    wt = ((lo * 7919 + hi * 104729 + seed) % 97 + 1).astype(np.uint32)
+    off = np.zeros(V + 1, np.int64)
+    np.add.at(off, src + 1, 1)
+    return np.cumsum(off).astype(np.int32), dst.astype(np.int32), wt
+
+
+def check(off, idx, wt, kinds, sources, runs=1, **opts):
+    """Batches of the queries, the sources rotated from run to run on one
+    engine (so captured launches are replayed), against the oracle."""
+    V = len(off) - 1
+    en = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, idx, wt), **opts)
+    og = O.G(off, idx, wt)
+    for r in range(runs):
+        src = [(s + 37 * r) % V for s in sources]
+        got = en.run_batch(kinds, src)[0]
+        for i, (k, s) in enumerate(zip(kinds, src)):
+            assert np.array_equal(got[i], O.expected(og, k, s)), (r, i, k, s)
+
+
+# A filter workgroup looks at 1024 vertices per step; from 33 workgroups on
+# their completion is counted on several lines first.
+@pytest.mark.parametrize("V", [1, 2, 1023, 1024, 1025, 32 * 1024, 32 * 1024 + 1, 40 * 1024 + 7])
+@pytest.mark.parametrize("opts", [dict(frontier_dense_div=1), dict(frontier_dense_div=1 << 20),
+                                  dict(sssp_delta=60)], ids=["sparse", "dense", "near_far"])
+def test_filter_workgroups(gpu, V, opts):
+    off, idx, wt = ring_graph(V, hub_degree=min(V // 2, 700))
+    kinds = [BFS] * 3 + [SSSP] * 5 + [WCC]
+    check(off, idx, wt, kinds, [0, V // 2, V - 1, V - 1, V // 3, 0, V // 2, V // 5, 0], runs=3, **opts)
