@@ -156,6 +156,21 @@ __device__ __forceinline__ void touch(const KP& P, bool claimed, int32_t v, u32 
   wave_append<int32_t>(claimed, v, &P.ctl->tcount[stamp & 1u].v, P.touched);
 }
 
+// Whether the lane that saw a next word of v empty (its atomicOr returned 0)
+// claims v for this iteration.  With one word per vertex that lane is the only
+// one; with several, one lane per word can be, and the stamp decides.
+template <int W>
+__device__ __forceinline__ bool claim_first(u32* mark, int32_t v, u32 stamp) {
+  return W == 1 || claim_vertex(mark, v, stamp);
+}
+
+// A wave-uniform value held in scalar registers.
+__device__ __forceinline__ int32_t uniform32(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ u64 uniform64(u64 x) {
+  return ((u64)(u32)__builtin_amdgcn_readfirstlane((int)(u32)(x >> 32)) << 32) |
+         (u32)__builtin_amdgcn_readfirstlane((int)(u32)x);
+}
+
 // A wave-uniform pointer into global memory pinned to scalar registers, so
 // accesses through it use the SGPR-base + 32-bit lane-offset addressing form
 // (one VGPR per access instead of a 64-bit per-lane address).
@@ -231,91 +246,154 @@ __device__ __forceinline__ void note_improved(Tally& t, u32 c, u32 thr) {
   else t.fmin = min(t.fmin, c);
 }
 
-// Relaxes edge (u -> v, weight wv) for every active BFS bit (bitmask
-// first-write against visited) and every sparse SSSP bit; sets the new bits
-// in next[v].  Sparse mode returns whether this lane made the vertex's first
-// claim of the iteration.
-template <int W, bool SPARSE>
-__device__ __forceinline__ bool relax_edge(const KP& P, int32_t u, int32_t v, u32 wv,
-                                           const u64 (&bm)[W], const u64 (&sm)[W], u32 stamp,
-                                           int rshift, u32 thr, Tally& t) {
-  bool first = false;
-  const size_t vb = vis_at<W>(v, 0);
-  // All W visited and W next words of v in one go (one contiguous record),
-  // issued before any of them is used.  In dense mode an edge with no BFS
-  // bit needs neither: its improved SSSP bits go to next[v] by a
-  // fire-and-forget atomicOr, so the record's line is touched only for an
-  // improvement, not for every edge scanned.  (A per-vertex byte of "BFS
-  // words every running query has visited", kept by the filter to skip the
-  // record read too, cut the visited tests of the RMAT-22 mixed batch by
-  // 39 % but not its traffic: the skipped records were cache hits, and the
-  // extra dependent load made 160 BFS 0.5 ms slower.)
-  bool any_b = false;
-#pragma unroll
-  for (int w = 0; w < W; ++w) any_b |= bm[w] != 0;
-  u64 nx[W], vis[W];
+// Relaxes N edges u[i] -> v[i] of weight wv[i] per lane (those with ok[i]) for
+// every active BFS bit (bitmask first-write against visited) and every sparse
+// SSSP bit, and sets the new bits in next[v[i]].  bm(i, w) and sm(i, w) are the
+// active BFS and SSSP bits of edge i's source in word w; a v[i] without ok[i]
+// is still a vertex.  Each step does its memory accesses for all N edges
+// before it uses any: the records, then the values, then the updates, so a
+// lane waits once per step and not once per edge.
+//
+// In dense mode edges without BFS bits (any_b false) read no record: their
+// improved SSSP bits go to next by a fire-and-forget atomicOr, so the record's
+// line is touched only for an improvement, not for every edge scanned.  (A
+// per-vertex byte of "BFS words every running query has visited", kept by the
+// filter to skip the record read too, cut the visited tests of the RMAT-22
+// mixed batch by 39 % but not its traffic: the skipped records were cache
+// hits, and the extra dependent load made 160 BFS 0.5 ms slower.)
+//
+// The step is as much bound by instruction issue as by memory (a 64-edge step
+// of a BFS scan of RMAT-22 has about 1600 cycles of its SIMD, and 100 vector
+// instructions are 400 of them), so what can be known per unit of work is
+// decided by the caller: any_b and any_s, wave-uniform, say whether some edge
+// has BFS or sparse SSSP bits, and the work counters of edges and queries are
+// kept per vertex.
+template <int W, bool SPARSE, int N, class BM, class SM>
+__device__ __forceinline__ void relax_edges(const KP& P, const int32_t (&u)[N], const int32_t (&v)[N],
+                                            const u32 (&wv)[N], const bool (&ok)[N], BM bm, SM sm, bool any_b,
+                                            bool any_s, u32 stamp, int rshift, u32 thr, Tally& t) {
+  // nx: bits that next[v] already has; add: bits to set there.
+  u64 nx[N][W], add[N][W];
   if (SPARSE || any_b) {
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      nx[w] = P.next[vb + W + w];
-      vis[w] = P.visited[vb + w];
+    for (int i = 0; i < N; ++i) {
+      const size_t vb = vis_at<W>(v[i], 0);
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        nx[i][w] = P.next[vb + W + w];
+        add[i][w] = P.visited[vb + w];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+#pragma unroll
+      for (int w = 0; w < W; ++w) add[i][w] = bm(i, w) & ~(add[i][w] | nx[i][w]);
     }
   } else {
 #pragma unroll
-    for (int w = 0; w < W; ++w) nx[w] = vis[w] = 0;
-  }
+    for (int i = 0; i < N; ++i) {
 #pragma unroll
-  for (int w = 0; w < W; ++w) {
-    if (!(bm[w] | sm[w])) continue;
-    u64 add = 0;
-    if (bm[w]) {
-      ++t.bfs;
-      add = bm[w] & ~vis[w];
+      for (int w = 0; w < W; ++w) nx[i][w] = add[i][w] = 0;
     }
-    u64 s = sm[w];
-    if (s) {
-      ++t.swords;
-      const size_t ub = vrow(P.V, w, u, rshift), vr = vrow(P.V, w, v, rshift);
-      while (s) {
-        // Up to 4 active queries per round, their 8 value loads in flight together.
-        int q[4];
-        bool a[4];
-        u32 du[4], cur[4];
+  }
+  if (any_s) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          // Unused slots of the batch re-read the first slot's values (same
-          // lines), never a line no active query needs.
-          a[i] = s != 0;
-          q[i] = a[i] ? __ffsll((long long)s) - 1 : q[0];
-          if (a[i]) s &= s - 1;
-          du[i] = P.vals[ub + q[i]];
-          cur[i] = P.vals[vr + q[i]];
+    for (int w = 0; w < W; ++w) {
+      // Up to QB active queries of the word per edge and round, their value
+      // loads in flight together.
+      constexpr int QB = N >= 4 ? 1 : N == 2 ? 2 : 4;
+      u64 s[N], left = 0;
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        s[i] = ok[i] ? sm(i, w) : 0ull;
+        left |= s[i];
+      }
+      while (left) {
+        int q[N][QB];
+        bool a[N][QB];
+        u32 du[N][QB], cur[N][QB];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          const size_t ub = vrow(P.V, w, u[i], rshift), vr = vrow(P.V, w, v[i], rshift);
+#pragma unroll
+          for (int k = 0; k < QB; ++k) {
+            // Unused slots of the round re-read an active query's values (the
+            // same lines), never a line that no query needs.
+            a[i][k] = s[i] != 0;
+            q[i][k] = a[i][k] ? __ffsll((long long)s[i]) - 1 : k ? q[i][0] : 0;
+            if (k || a[i][k]) {
+              s[i] &= s[i] - 1;
+              du[i][k] = P.vals[ub + q[i][k]];
+              cur[i][k] = P.vals[vr + q[i][k]];
+            }
+          }
         }
+        left = 0;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (!a[i]) continue;
-          ++t.sssp;
-          const u32 cand = du[i] + wv;
-          if (cand < du[i]) continue;  // saturate: never wrap past CGP_INF
-          if (cand < cur[i]) {
-            atomicMin(&P.vals[vr + q[i]], cand);
-            add |= 1ull << q[i];
-            ++t.imp;
-            note_improved(t, cand, thr);
+        for (int i = 0; i < N; ++i) {
+          left |= s[i];
+#pragma unroll
+          for (int k = 0; k < QB; ++k) {
+            // Saturating add: a path past CGP_INF stays unreachable.
+            const u32 cand = __builtin_elementwise_add_sat(du[i][k], wv[i]);
+            if (a[i][k] && cand < cur[i][k]) {
+              atomicMin(&P.vals[vrow(P.V, w, v[i], rshift) + q[i][k]], cand);
+              add[i][w] |= (1ull << q[i][k]) & ~nx[i][w];
+              ++t.imp;
+              note_improved(t, cand, thr);
+            }
           }
         }
       }
     }
-    if (add & ~nx[w]) {
+  }
+  bool first[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    first[i] = false;
+    u64 some = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) some |= add[i][w];
+    if (!ok[i] || !some) continue;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      if (!add[i][w]) continue;
       ++t.nnew;
+      u64* const x = &P.next[nxt_at<W>(v[i], w)];
       if (SPARSE) {
-        if (atomicOr(&P.next[vb + W + w], add) == 0) first = true;
+        if (atomicOr(x, add[i][w]) == 0) first[i] = true;
       } else {
-        atomicOr(&P.next[vb + W + w], add);
+        atomicOr(x, add[i][w]);
       }
     }
   }
-  return SPARSE && first && claim_vertex(P.mark, v, stamp);
+  if (SPARSE) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) touch(P, first[i] && claim_first<W>(P.mark, v[i], stamp), v[i], stamp);
+  }
+}
+
+// Work counters of d edges of a vertex with BFS bits bm and sparse SSSP bits
+// sm, and, once per vertex or chunk (`item`), of the vertex itself.
+template <int W>
+__device__ __forceinline__ void count_edges(Tally& t, const u64 (&bm)[W], const u64 (&sm)[W], u32 d, bool item,
+                                            bool weighted) {
+  u32 nb = 0, ns = 0, nq = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    nb += bm[w] ? 1u : 0u;
+    ns += sm[w] ? 1u : 0u;
+    nq += (u32)__popcll(sm[w]);
+  }
+  t.edges += d;
+  t.bfs += d * nb;
+  t.swords += d * ns;
+  t.sssp += (u64)d * nq;
+  if (ns && weighted) t.wedges += d;
+  if (item) {
+    ++t.items;
+    t.src += nq;
+  }
 }
 
 // Frontier masks of vertex u: BFS bits, and the sparse SSSP bits (popcount
@@ -379,41 +457,104 @@ __device__ __forceinline__ bool postpone(const KP& P, int32_t u, const u64 (&far
       atomicOr(&P.next[nxt_at<W>(u, w)], far[w]);
     }
   }
-  return SPARSE && first && claim_vertex(P.mark, u, stamp);
+  return SPARSE && first && claim_first<W>(P.mark, u, stamp);
 }
 
-// Expands frontier vertex u over edges [e0, e1) with lanes striding by
-// `stride` from `first` (lane-per-edge): BFS bits and sparse SSSP words.
+// Lane k's value of a per-lane word, as a wave-uniform scalar.
+__device__ __forceinline__ u64 lane64(u64 x, int k) {
+  return ((u64)(u32)__builtin_amdgcn_readlane((int)(u32)(x >> 32), k) << 32) |
+         (u32)__builtin_amdgcn_readlane((int)(u32)x, k);
+}
+
+// Expands up to 64 (vertex, edge range) units with the whole wave, lane = edge:
+// lane k < cnt holds unit k, vertex u with edges [e0, e1) (empty ranges
+// allowed), and `lead` in the part of a vertex that postpones its far pairs and
+// counts its queries.  The units' masks are fetched by their lanes in parallel
+// and each unit's are then wave-uniform, in scalar registers; N steps of 64
+// edges are relaxed together, and the columns and weights of the next step, of
+// the next unit too, are on their way while a step is relaxed.
 template <int W, bool SPARSE>
-__device__ __forceinline__ void expand_lanes(const KP& P, int32_t u, int32_t e0, int32_t e1,
-                                             int32_t first, int32_t stride, bool bfs_on, int dense_t,
-                                             int rshift, u32 stamp, u32 thr, bool lead, Tally& t) {
+__device__ __forceinline__ void expand_units(const KP& P, int cnt, int32_t u, int32_t e0, int32_t e1, bool lead,
+                                             bool bfs_on, int dense_t, int rshift, u32 stamp, u32 thr, Tally& t) {
+  // Steps in flight: as many as leave the kernel three waves per SIMD (four at
+  // W = 1).  One RMAT-18 SSSP query at N = 1 / 4: 980 / 820 us; 160 BFS on
+  // RMAT-22 (W = 4) at 1 / 2 / 4: 9.2 / 9.5 / 11.6 ms.
+  constexpr int N = W == 1 ? 4 : W == 2 ? 2 : 1;
+  const int lane = lane_id();
+  const bool have = lane < cnt && e0 < e1;
   u64 bm[W], sm[W], far[W];
-  bool any_s;
-  load_masks<W>(P, u, bfs_on, dense_t, thr, rshift, bm, sm, far, any_s, t);
-  if (lead) {
-    const bool c = postpone<W, SPARSE>(P, u, far, stamp, t);
+  bool any_s = false, any_b = false;
+  if (have) load_masks<W>(P, u, bfs_on, dense_t, thr, rshift, bm, sm, far, any_s, t);
+#pragma unroll
+  for (int w = 0; w < W; ++w) {
+    if (!have) bm[w] = sm[w] = far[w] = 0;
+    any_b |= bm[w] != 0;
+  }
+  if (thr != INF) {
+    const bool c = have && lead && postpone<W, SPARSE>(P, u, far, stamp, t);
     if (SPARSE) touch(P, c, u, stamp);
   }
-  bool any_b = false;
-#pragma unroll
-  for (int w = 0; w < W; ++w) any_b |= (bm[w] != 0);
-  if (!any_b && !any_s) return;
-  if (first == e0) {
-    ++t.items;
-#pragma unroll
-    for (int w = 0; w < W; ++w) t.src += (u64)__popcll(sm[w]);
-  }
-  for (int32_t e = first; e < e1; e += stride) {
-    const int32_t v = P.idx[e];
-    u32 wv = 1;
-    if (any_s && P.wt) {
-      wv = P.wt[e];
-      ++t.wedges;
+  if (!any_b && !any_s) e1 = e0;
+  else if (P.profile) count_edges<W>(t, bm, sm, (u32)(e1 - e0), lead, P.wt != nullptr);
+  const u64 units = __ballot(have && e0 < e1), weighted_units = P.wt ? __ballot(any_s) : 0ull;
+  struct Step {
+    int k;  // unit
+    int32_t v[N];
+    u32 wv[N];
+    bool ok[N];
+  };
+  u64 left = units;
+  int k = 0;
+  int32_t eb = 0, end = 0;
+  // The next step's columns and weights; false when the units are exhausted.
+  const auto fetch = [&](Step& st) {
+    if (eb >= end) {
+      if (!left) return false;
+      k = __builtin_ctzll(left);
+      left &= left - 1;
+      eb = __builtin_amdgcn_readlane(e0, k);
+      end = __builtin_amdgcn_readlane(e1, k);
     }
-    ++t.edges;
-    const bool claimed = relax_edge<W, SPARSE>(P, u, v, wv, bm, sm, stamp, rshift, thr, t);
-    if (SPARSE) touch(P, claimed, v, stamp);
+    st.k = k;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      // Lanes past the end re-read the last edge (a line already wanted).
+      const int32_t e = eb + i * 64 + lane;
+      st.ok[i] = e < end;
+      const int32_t ec = min(e, end - 1);
+      st.v[i] = P.idx[ec];
+      st.wv[i] = (weighted_units >> k) & 1ull ? P.wt[ec] : 1u;
+    }
+    eb += 64 * N;
+    return true;
+  };
+  Step cur, nxt;
+  bool more = fetch(cur);
+  int ku = -1;  // unit whose masks are in scalar registers
+  int32_t uk = 0;
+  u64 bk[W], sk[W];
+  bool k_b = false, k_s = false;
+  while (more) {
+    more = fetch(nxt);
+    if (cur.k != ku) {
+      ku = cur.k;
+      uk = __builtin_amdgcn_readlane(u, ku);
+      k_b = k_s = false;
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        bk[w] = lane64(bm[w], ku);
+        sk[w] = lane64(sm[w], ku);
+        k_b |= bk[w] != 0;
+        k_s |= sk[w] != 0;
+      }
+    }
+    int32_t uu[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) uu[i] = uk;
+    relax_edges<W, SPARSE, N>(
+        P, uu, cur.v, cur.wv, cur.ok, [&](int, int w) { return bk[w]; }, [&](int, int w) { return sk[w]; }, k_b, k_s,
+        stamp, rshift, thr, t);
+    cur = nxt;
   }
 }
 
@@ -455,13 +596,18 @@ __device__ __forceinline__ int wave_upper_bound(u32 incl, u32 f) {
 // grids and meshes consecutive ids are neighbours whose rows share cache
 // lines, and mixing measured slower (4096^2 grid, 512 SSSP: push 1067 -> 1195
 // ms per batch).
+//
+// Groups shorter than 64 (lists with fewer than 64 entries per wave of the
+// launch) are gsz consecutive entries, or gsz / 8 runs.  N windows of 64 edges
+// are relaxed together.
 template <int W, bool SPARSE>
-__device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t* list, u32 g, u32 ng, u32 n,
+__device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t* list, u32 g, u32 ng, u32 gsz, u32 n,
                                                      bool bfs_on, int dense_t, int rshift, u32 stamp,
                                                      u32 thr, Tally& t) {
+  constexpr int N = W == 1 ? 2 : 1;
   const int lane = lane_id();
-  const u32 e = P.mix_small ? (g + (u32)(lane >> 3) * ng) * 8u + (u32)(lane & 7) : g * 64u + (u32)lane;
-  const bool have = e < n;
+  const u32 e = P.mix_small && gsz >= 8 ? (g + (u32)(lane >> 3) * ng) * 8u + (u32)(lane & 7) : g * gsz + (u32)lane;
+  const bool have = (u32)lane < gsz && e < n;
   const int32_t u = have ? list[e] : 0;
   u64 bm[W], sm[W], far[W];
   bool any_s = false, any_b = false;
@@ -471,49 +617,58 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
     if (!have) bm[w] = sm[w] = far[w] = 0;
     any_b |= bm[w] != 0;
   }
-  {
+  if (thr != INF) {
     const bool c = have && postpone<W, SPARSE>(P, u, far, stamp, t);
     if (SPARSE) touch(P, c, u, stamp);
   }
   const bool work = have && (any_b || any_s);
   const int32_t e0 = work ? P.off[u] : 0;
   const u32 d = work ? (u32)(P.off[u + 1] - e0) : 0u;
-  if (work) {
-    ++t.items;
-#pragma unroll
-    for (int w = 0; w < W; ++w) t.src += (u64)__popcll(sm[w]);
-  }
+  if (work && P.profile) count_edges<W>(t, bm, sm, d, true, P.wt != nullptr);
   const u32 incl = wave_incl_scan(d);
   // Wave-uniform (scalar) so the loops below branch on the scalar unit and
   // the per-step row indices stay in scalar registers.
   const u32 total = (u32)__builtin_amdgcn_readlane((int)incl, 63);
-  for (u32 win = 0; win < total; win += 64) {
-    const u32 f = win + (u32)lane;
-    const int j = wave_upper_bound(incl, f);
-    const int32_t uj = __shfl(u, j, 64);
-    const u32 exj = (u32)__shfl((int)(incl - d), j, 64);
-    const int32_t ej = __shfl(e0, j, 64) + (int32_t)(f - exj);
-    u64 bj[W], sj[W];
-    bool sj_any = false;
+  const bool wave_b = __ballot(any_b) != 0, wave_s = __ballot(any_s) != 0, weighted = wave_s && P.wt;
+  // The columns and weights of the next windows are on their way while the
+  // current ones are relaxed.
+  int jn[N];
+  int32_t vn[N];
+  u32 wn[N];
+  const auto fetch = [&](u32 win) {
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      bj[w] = shfl64(bm[w], j);
-      sj[w] = shfl64(sm[w], j);
-      sj_any |= sj[w] != 0;
+    for (int i = 0; i < N; ++i) {
+      const u32 f = min(win + (u32)i * 64u + (u32)lane, total - 1);  // lanes past the end re-read the last edge
+      jn[i] = wave_upper_bound(incl, f);
+      const u32 exj = (u32)__shfl((int)(incl - d), jn[i], 64);
+      const int32_t ej = __shfl(e0, jn[i], 64) + (int32_t)(f - exj);
+      vn[i] = P.idx[ej];
+      wn[i] = weighted ? P.wt[ej] : 1u;
     }
-    bool claimed = false;
-    int32_t v = 0;
-    if (f < total) {
-      v = P.idx[ej];
-      u32 wv = 1;
-      if (sj_any && P.wt) {
-        wv = P.wt[ej];
-        ++t.wedges;
+  };
+  if (total) fetch(0);
+  for (u32 win = 0; win < total; win += 64 * N) {
+    int32_t uj[N], v[N];
+    u32 wv[N];
+    bool ok[N];
+    u64 bj[N][W], sj[N][W];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int j = jn[i];
+      ok[i] = win + (u32)i * 64u + (u32)lane < total;
+      uj[i] = __shfl(u, j, 64);
+      v[i] = vn[i];
+      wv[i] = wn[i];
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        bj[i][w] = wave_b ? shfl64(bm[w], j) : 0ull;
+        sj[i][w] = wave_s ? shfl64(sm[w], j) : 0ull;
       }
-      ++t.edges;
-      claimed = relax_edge<W, SPARSE>(P, uj, v, wv, bj, sj, stamp, rshift, thr, t);
     }
-    if (SPARSE) touch(P, claimed, v, stamp);
+    if (win + 64 * N < total) fetch(win + 64 * N);
+    relax_edges<W, SPARSE, N>(
+        P, uj, v, wv, ok, [&](int i, int w) { return bj[i][w]; }, [&](int i, int w) { return sj[i][w]; }, wave_b,
+        wave_s, stamp, rshift, thr, t);
   }
 }
 
@@ -584,7 +739,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
           if (lane == 0) {
             ++t.nnew;
             if (SPARSE) {
-              if (atomicOr(&P.next[nxt_at<W>(uk, wk)], fm) == 0) claimed = claim_vertex(P.mark, uk, stamp);
+              if (atomicOr(&P.next[nxt_at<W>(uk, wk)], fm) == 0) claimed = claim_first<W>(P.mark, uk, stamp);
             } else {
               atomicOr(&P.next[nxt_at<W>(uk, wk)], fm);
             }
@@ -698,7 +853,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
           if (lane == 0) {
             ++t.nnew;
             const int wk = __builtin_amdgcn_readlane(myword, k0 + k);
-            if (atomicOr(&P.next[nxt_at<W>(vk, wk)], m) == 0) claimed = claim_vertex(P.mark, vk, stamp);
+            if (atomicOr(&P.next[nxt_at<W>(vk, wk)], m) == 0) claimed = claim_first<W>(P.mark, vk, stamp);
           }
           touch(P, claimed, vk, stamp);
         }
@@ -868,7 +1023,7 @@ __device__ __forceinline__ void expand_flat_dense_tab(const KP& P, u32 base, u32
               bool claimed = false;
               if (lane == 0) {
                 ++t.nnew;
-                if (atomicOr(&P.next[nxt_at<W>(vk, wp)], m) == 0) claimed = claim_vertex(P.mark, vk, stamp);
+                if (atomicOr(&P.next[nxt_at<W>(vk, wp)], m) == 0) claimed = claim_first<W>(P.mark, vk, stamp);
               }
               touch(P, claimed, vk, stamp);
             }
@@ -991,7 +1146,7 @@ __device__ __forceinline__ void expand_flat_narrow(const KP& P, u32 base, u32 n,
           bool claimed = false;
           if (own && mg) {
             ++t.nnew;
-            if (atomicOr(&P.next[nxt_at<W>(myv, myword)], (u64)mg) == 0) claimed = claim_vertex(P.mark, myv, stamp);
+            if (atomicOr(&P.next[nxt_at<W>(myv, myword)], (u64)mg) == 0) claimed = claim_first<W>(P.mark, myv, stamp);
           }
           touch(P, claimed, myv, stamp);
         }
@@ -1056,7 +1211,7 @@ __device__ __forceinline__ bool pull_vertex(const KP& P, int32_t v, const u64 (&
       }
     }
   }
-  return SPARSE && first && claim_vertex(P.mark, v, stamp);
+  return SPARSE && first && claim_first<W>(P.mark, v, stamp);
 }
 
 // Bottom-up step for a high-degree vertex v with the whole wave: each step
@@ -1108,7 +1263,7 @@ __device__ __forceinline__ bool pull_vertex_wave(const KP& P, int32_t v, const u
         }
       }
     }
-    first = SPARSE && first && claim_vertex(P.mark, v, stamp);
+    first = SPARSE && first && claim_first<W>(P.mark, v, stamp);
   }
   return first;
 }
@@ -1119,43 +1274,90 @@ __device__ __forceinline__ u32 wave_fetch(u32* ctr, u32 n) {
   return (u32)__shfl((int)i, 0, 64);
 }
 
-// Wave-level claims of `chunk` units from NSHARD contiguous shards of [0, n):
-// shard s covers [n*s/NSHARD, n*(s+1)/NSHARD) and has cursor cur[s] (units
-// handed out so far).  A wave starts at its workgroup's shard and moves to the
-// next when that one is exhausted (cursors only grow, so an exhausted shard
-// stays exhausted); after NSHARD exhausted shards every unit has been claimed.
-// Claims never cross a shard's end.  All state is wave-uniform.
+// Wave-level claims of the units [0, n), in NSHARD contiguous shards: shard s
+// covers [n*s/NSHARD, n*(s+1)/NSHARD) and belongs to the workgroups with
+// blockIdx % NSHARD == s, one XCD.  Each of a shard's waves owns its first
+// units without any atomic (`chunk` units by its rank); what is left is handed
+// out through the shard's cursor, and a wave whose shard is exhausted looks at
+// all cursors with one load before it claims from another (cursors only grow).
+// A list that the first claims cover costs no atomic at all.  (Every wave used
+// to find each shard exhausted by an atomic of its own: 16 per wave and
+// launch, 16 us at 1024 waves and 93 us at 8192 with one unit of work.)
+// The claims get shorter towards a shard's end.  Claims never cross a shard's
+// end.  All state is wave-uniform.  `turn` (0 to 3) rotates which waves come
+// first, so that the short lists of consecutive phases go to different waves.
 struct ShardFetch {
-  int s, left;
-  __device__ __forceinline__ ShardFetch() : s((int)(blockIdx.x % NSHARD)), left(NSHARD) {}
-  __device__ __forceinline__ bool next(Ctr* cur, u32 n, u32 chunk, u32& lo, u32& hi) {
-    while (left > 0) {
-      const u32 b = (u32)(((u64)n * (u32)s) / NSHARD), e = (u32)(((u64)n * (u32)(s + 1)) / NSHARD);
-      if (b < e) {
+  u32 n, chunk, wpb;
+  int s;
+  bool first, strided;
+  u32 rank;  // first claim: this wave's place in its shard
+  __device__ __forceinline__ ShardFetch(u32 n_, u32 chunk_, u32 turn, bool strided_ = false)
+      : n(n_), chunk(chunk_), first(true), strided(strided_) {
+    wpb = blockDim.x / 64u;
+    s = (int)(blockIdx.x % NSHARD);
+    const u32 nw = waves(s);
+    rank = (blockIdx.x / NSHARD) * wpb + (u32)uniform32((int32_t)(threadIdx.x >> 6)) + turn * (nw / 4u);
+    if (rank >= nw) rank -= nw;
+  }
+  __device__ __forceinline__ u32 waves(int sh) const { return (gridDim.x - (u32)sh + NSHARD - 1) / NSHARD * wpb; }
+  __device__ __forceinline__ u32 begin(int sh) const { return (u32)(((u64)n * (u32)sh) / NSHARD); }
+  __device__ __forceinline__ u32 size(int sh) const {
+    return strided ? (n + NSHARD - 1u - (u32)sh) / NSHARD : begin(sh + 1) - begin(sh);
+  }
+  // Unit i of the shard the last claim was from.
+  __device__ __forceinline__ u32 unit(u32 i) const { return strided ? i * NSHARD + (u32)s : begin(s) + i; }
+  // Units of a shard beyond its waves' first claims.
+  __device__ __forceinline__ u32 shared(int sh) const {
+    const u32 all = size(sh), own = waves(sh) * chunk;
+    return all > own ? all - own : 0u;
+  }
+  __device__ __forceinline__ bool next(Ctr* cur, u32& lo, u32& hi) {
+    if (first) {
+      first = false;
+      lo = rank * chunk;
+      hi = min(size(s), lo + chunk);
+      if (lo < hi) return true;
+    }
+    while (true) {
+      const u32 sz = shared(s);
+      if (sz) {
+        // Towards the end a claim is one unit: the last claims bound the
+        // launch's end.
         const u32 i = wave_fetch(&cur[s].v, chunk);
-        if (i < e - b) {
-          lo = b + i;
-          hi = min(e, lo + chunk);
+        if (i < sz) {
+          lo = waves(s) * chunk + i;
+          hi = min(size(s), lo + chunk);
           return true;
         }
       }
-      s = s + 1 == NSHARD ? 0 : s + 1;
-      --left;
+      const int k = lane_id() % NSHARD;
+      const u32 szk = shared(k);
+      const bool more =
+          szk && __hip_atomic_load(&cur[k].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < szk;
+      const u32 m = (u32)__ballot(more) & ((1u << NSHARD) - 1u);
+      if (!m) return false;
+      const u32 up = m >> s;  // the next shard with units left, cyclically
+      s = up ? s + __builtin_ctz(up) : __builtin_ctz(m);
     }
-    return false;
   }
 };
 
-// Body of the advance for one frontier mode; workgroups pull work
-// dynamically, heaviest first:
-//   L  one workgroup per LCHUNK-edge chunk of a high-degree vertex
-//   D  64 (vertex, dense SSSP word, DCHUNK-edge chunk) items per wave,
-//      edges flattened, lane = query
-//   M  one wave per medium-degree vertex, lane = edge
-//   S  64 low-degree vertices per wave, edges flattened, lane = edge
+// Units per claim of a list of n units on nw waves: several when every wave
+// has many to take (each claim is an atomic on a line that an eighth of the
+// waves share), one when the claims would leave waves without work.
+__device__ __forceinline__ u32 claim_units(u32 n, u32 nw) {
+  return n >= 16u * nw ? 8u : n >= 8u * nw ? 4u : n >= 4u * nw ? 2u : 1u;
+}
+
+// Body of the advance for one frontier mode; waves take work heaviest first:
+//   L  one wave per part of an LCHUNK-edge chunk of a high-degree vertex
+//   M  one wave per medium-degree vertex, lane = edge; several waves share a
+//      vertex when the list is shorter than the launch has waves
+//   S  up to 64 low-degree vertices per wave, edges flattened, lane = edge
 //   P  (pull iterations) one lane per vertex of the whole graph
+// (D, the lane-per-query rows of dense SSSP words, is k_adv_dense.)
 template <int W, bool SPARSE, int BS>
-__device__ __forceinline__ void advance_push_body(const KP& P, u32* s_item, Tally& t) {
+__device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   Ctl* C = P.ctl;
   const u32 iter = C->iter, p = iter & 1u;
   const bool bfs_on = C->bfs_pull == 0;
@@ -1164,42 +1366,61 @@ __device__ __forceinline__ void advance_push_body(const KP& P, u32* s_item, Tall
   // In an SSSP pull iteration every vertex gathers its SSSP values itself: a
   // threshold of 0 leaves no SSSP word to the push phases.
   const int rshift = P.cfg->rshift, dense_t = C->sssp_pull ? 0 : P.cfg->dense_t;
+  const u32 nw = gridDim.x * (BS / 64);
   const int lane = lane_id();
-  // Phase L.
-  const u32 nL = C->bcount[p][2].v;
-  while (nL) {
-    __syncthreads();
-    if (threadIdx.x == 0) *s_item = atomicAdd(&C->fetch[p][0].v, 1u);
-    __syncthreads();
-    const u32 i = *s_item;
-    if (i >= nL) break;
-    const u64 item = P.large[p][i];
-    const int32_t u = (int32_t)(item >> 32);
-    const int32_t e0 = P.off[u] + (int32_t)((u32)item * LCHUNK);
-    const int32_t e1 = min(P.off[u + 1], e0 + LCHUNK);
-    expand_lanes<W, SPARSE>(P, u, e0, e1, e0 + (int32_t)threadIdx.x, BS, bfs_on, dense_t, rshift,
-                            stamp, thr, (u32)item == 0 && threadIdx.x == 0, t);
-  }
-  // Work cursors are single addresses every wave contends for, so each
-  // fetch claims several units (FETCH_M medium vertices, FETCH_S groups of
-  // 64 small vertices).
-  constexpr u32 FETCH_M = 4, FETCH_S = 4;
-  // Phase M.
-  const u32 nM = C->bcount[p][1].v;
   u32 lo, hi;
-  for (ShardFetch sf; nM && sf.next(C->shard[p][SH_M], nM, FETCH_M, lo, hi);) {
-    for (u32 i = lo; i < hi; ++i) {
-      const int32_t u = P.medium[p][i];
-      const int32_t e0 = P.off[u], e1 = P.off[u + 1];
-      expand_lanes<W, SPARSE>(P, u, e0, e1, e0 + lane, 64, bfs_on, dense_t, rshift, stamp, thr, lane == 0, t);
+  // Phase L.  A chunk is two units, or up to 32 of 128 edges while that leaves
+  // every unit a wave of its own.
+  const u32 nL = C->bcount[p][2].v;
+  if (nL) {
+    u32 sh = 1;
+    while (sh < 5 && (nL << (sh + 1)) <= nw) ++sh;
+    const u32 n = nL << sh;
+    ShardFetch sf(n, claim_units(n, nw), 0, P.mix_small);
+    while (sf.next(C->shard[p][SH_L], lo, hi)) {
+      const u32 i = sf.unit(min(lo + (u32)lane, hi - 1));
+      const u64 item = P.large[p][i >> sh];
+      const u32 part = i & ((1u << sh) - 1u);
+      const int32_t u = (int32_t)(item >> 32);
+      const int32_t e0 = P.off[u] + (int32_t)((u32)item * LCHUNK + part * ((u32)LCHUNK >> sh));
+      const int32_t e1 = min(P.off[u + 1], e0 + (LCHUNK >> sh));
+      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, (u32)item == 0 && part == 0, bfs_on, dense_t, rshift,
+                              stamp, thr, t);
     }
   }
-  // Phase S: groups of 64 entries (expand_flat_vertices).
+  // Phase M.  With fewer vertices than waves, 2, 4 or 8 waves take equal parts
+  // of each vertex's edges: a medium vertex has up to bin_large edges, eight
+  // rounds of a wave, and one such vertex used to be the length of a small
+  // graph's whole launch.
+  const u32 nM = C->bcount[p][1].v;
+  if (nM) {
+    u32 sh = 0;
+    while (sh < 3 && (nM << (sh + 1)) <= nw) ++sh;
+    const u32 n = nM << sh;
+    ShardFetch sf(n, claim_units(n, nw), 1, P.mix_small);
+    while (sf.next(C->shard[p][SH_M], lo, hi)) {
+      const u32 i = sf.unit(min(lo + (u32)lane, hi - 1));
+      const int32_t u = P.medium[p][i >> sh];
+      const int32_t b = P.off[u], d = P.off[u + 1] - b;
+      const u32 part = i & ((1u << sh) - 1u);
+      // Parts of whole 64-edge steps.
+      const int32_t len = (int32_t)((((u32)d + 63u) / 64u + (1u << sh) - 1u) >> sh) * 64;
+      const int32_t e0 = b + (int32_t)part * len, e1 = min(b + d, e0 + len);
+      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, part == 0, bfs_on, dense_t, rshift, stamp, thr, t);
+    }
+  }
+  // Phase S.  Groups of 64 entries, halved down to 4 while that leaves every
+  // group a wave of its own.
   const u32 nS = C->bcount[p][0].v;
-  const u32 ngS = (nS + 63u) / 64u;
-  for (ShardFetch sf; nS && sf.next(C->shard[p][SH_S], ngS, FETCH_S, lo, hi);) {
-    for (u32 g = lo; g < hi; ++g)
-      expand_flat_vertices<W, SPARSE>(P, P.small[p], g, ngS, nS, bfs_on, dense_t, rshift, stamp, thr, t);
+  if (nS) {
+    u32 gsz = 64;
+    while (gsz > 4 && nS <= (gsz / 2) * nw) gsz /= 2;
+    const u32 ng = (nS + gsz - 1) / gsz;
+    ShardFetch sf(ng, claim_units(ng, nw), 2);
+    while (sf.next(C->shard[p][SH_S], lo, hi)) {
+      for (u32 g = lo; g < hi; ++g)
+        expand_flat_vertices<W, SPARSE>(P, P.small[p], sf.unit(g), ng, gsz, nS, bfs_on, dense_t, rshift, stamp, thr, t);
+    }
   }
   // Phase P: high-degree vertices one wave each (64 neighbours per step,
   // early exit on a wave-wide OR), then the rest one lane each.
@@ -1337,9 +1558,9 @@ __global__ __launch_bounds__(BLOCK) void k_adv_narrow(KP P) {
   const bool sparse = C->dense_mode == 0;
   Tally t;
   u32 lo, hi;
-  for (ShardFetch sf; sf.next(C->shard[p][SH_N], nN, 64u, lo, hi);) {
-    if (sparse) expand_flat_narrow<W, true>(P, lo, hi, rshift, stamp, t);
-    else expand_flat_narrow<W, false>(P, lo, hi, rshift, stamp, t);
+  for (ShardFetch sf(nN, 64u, 0); sf.next(C->shard[p][SH_N], lo, hi);) {
+    if (sparse) expand_flat_narrow<W, true>(P, sf.unit(lo), sf.unit(hi), rshift, stamp, t);
+    else expand_flat_narrow<W, false>(P, sf.unit(lo), sf.unit(hi), rshift, stamp, t);
   }
   if (P.profile) {
     prof_add(P, PF_DENSE_ITEMS, t.ditems);
@@ -1425,7 +1646,7 @@ __device__ __forceinline__ void pull_sssp_item(const KP& P, u64 item, int rshift
     }
   }
   if (SPARSE) {
-    const bool c = lane == 0 && claimed && claim_vertex(P.mark, v, stamp);
+    const bool c = lane == 0 && claimed && claim_first<W>(P.mark, v, stamp);
     touch(P, c, v, stamp);
   }
 }
@@ -1443,10 +1664,10 @@ __global__ __launch_bounds__(BLOCK) void k_pull_sssp(KP P) {
   Tally t;
   constexpr u32 FETCH_P = 16;
   u32 lo, hi;
-  for (ShardFetch sf; sf.next(C->shard[p][SH_P], n, FETCH_P, lo, hi);) {
+  for (ShardFetch sf(n, FETCH_P, 0); sf.next(C->shard[p][SH_P], lo, hi);) {
     for (u32 i = lo; i < hi; ++i) {
-      if (sparse) pull_sssp_item<W, true, 8>(P, P.pull_items[i], rshift, stamp, t);
-      else pull_sssp_item<W, false, 8>(P, P.pull_items[i], rshift, stamp, t);
+      if (sparse) pull_sssp_item<W, true, 8>(P, P.pull_items[sf.unit(i)], rshift, stamp, t);
+      else pull_sssp_item<W, false, 8>(P, P.pull_items[sf.unit(i)], rshift, stamp, t);
     }
   }
   if (P.profile) {
@@ -1486,15 +1707,14 @@ template <int W, int BS>
 __global__ __launch_bounds__(BS) void k_adv_push(KP P) {
   Ctl* C = P.ctl;
   if (C->finished) return;
-  __shared__ u32 s_item;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     atomicMin(&C->adv_t0, (u64)wall_clock64());
     C->f_iter = C->iter;
     C->f_scan = C->dense_mode;
   }
   Tally t;
-  if (C->dense_mode) advance_push_body<W, false, BS>(P, &s_item, t);
-  else advance_push_body<W, true, BS>(P, &s_item, t);
+  if (C->dense_mode) advance_push_body<W, false, BS>(P, t);
+  else advance_push_body<W, true, BS>(P, t);
   flush_near_far(P, t, C->thr);
   if (P.profile) flush_tally(P, t);
   __syncthreads();
@@ -1532,6 +1752,11 @@ __global__ __launch_bounds__(BLOCK) void k_seed(KP P, const int32_t* slot_src, i
 }
 
 // ------------------------------------------------------------------ filter
+template <typename T>
+__device__ __forceinline__ T* pick(T* a, T* b, u32 which) {
+  return (T*)((u64)a ^ (((u64)a ^ (u64)b) & (0ull - (u64)which)));
+}
+
 // Vertex i of the filter's list (i < n: the scan's i, or touched[i]), its next
 // words and CSR offsets; zeros past the end.  The W next words of a record
 // are contiguous and 16-byte aligned (W >= 2).
@@ -1603,14 +1828,14 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   // reservation per 256 vertices cost about 0.3 ms per dense iteration on
   // RMAT-22).
   const u32 gstride = active * BLOCK * FK;
-  // The next iteration's bin lists, picked once (indexing the argument's
-  // arrays with np inside the loop made the compiler copy the whole
-  // argument block to scratch memory).
-  int32_t* const l_small = np ? P.small[1] : P.small[0];
-  int32_t* const l_medium = np ? P.medium[1] : P.medium[0];
-  u64* const l_large = np ? P.large[1] : P.large[0];
-  u64* const l_dense = np ? P.dense[1] : P.dense[0];
-  u64* const l_dense_n = np ? P.dense_n[1] : P.dense_n[0];
+  // The next iteration's bin lists, picked once, by arithmetic: indexing the
+  // argument's arrays with np, or selecting between their entries, makes the
+  // compiler copy the whole argument block (240 bytes a lane) to scratch memory.
+  int32_t* const l_small = pick(P.small[0], P.small[1], np);
+  int32_t* const l_medium = pick(P.medium[0], P.medium[1], np);
+  u64* const l_large = pick(P.large[0], P.large[1], np);
+  u64* const l_dense = pick(P.dense[0], P.dense[1], np);
+  u64* const l_dense_n = pick(P.dense_n[0], P.dense_n[1], np);
   for (u32 base = blockIdx.x * BLOCK * FK; base < n; base += gstride) {
     int32_t vv[FK], o0[FK], o1[FK];
     u64 nwk[FK][W];

@@ -57,3 +57,28 @@ def test_filter_workgroups(gpu, V, opts):
     off, idx, wt = ring_graph(V, hub_degree=min(V // 2, 700))
     kinds = [BFS] * 3 + [SSSP] * 5 + [WCC]
     check(off, idx, wt, kinds, [0, V // 2, V - 1, V - 1, V // 3, 0, V // 2, V // 5, 0], runs=3, **opts)
+
+
+# Push work lists: vertices of at most 64 edges go 64 (or fewer) to a wave, of
+# at most 2048 one to a wave or part of one, larger ones in chunks of 4096
+# edges split into parts.  advance_blocks sets how many waves share the lists:
+# one workgroup makes every list longer than the launch has waves.
+@pytest.mark.parametrize("hub", [63, 64, 65, 2047, 2049, 4095, 4097, 9000])
+@pytest.mark.parametrize("opts", [dict(), dict(advance_blocks=1), dict(advance_blocks=9, block_size=128),
+                                  dict(advance_blocks=3, block_size=512, frontier_dense_div=1),
+                                  dict(bin_small=1, bin_large=2), dict(sssp_delta=60)],
+                         ids=["default", "one_block", "nine_blocks", "sparse", "all_large", "near_far"])
+def test_push_work_lists(gpu, hub, opts):
+    V = 12007
+    off, idx, wt = ring_graph(V, hub_degree=hub, seed=hub, chords=2)
+    check(off, idx, wt, [BFS, BFS, SSSP, SSSP], [V // 2, 0, V // 2, 5], runs=2, dense_threshold=65, **opts)
+
+
+# The same lists with two and four mask words, and on a directed graph.
+@pytest.mark.parametrize("n", [5, 70, 150])
+@pytest.mark.parametrize("directed", [False, True])
+def test_push_mask_words(gpu, n, directed):
+    V = 3001
+    off, idx, wt = ring_graph(V, hub_degree=2500, seed=n, directed=directed)
+    kinds = [SSSP] * (n // 3) + [BFS] * (n - n // 3)
+    check(off, idx, wt, kinds, [(i * 131) % V for i in range(n)], runs=2, advance_blocks=2)
