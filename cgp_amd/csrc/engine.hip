@@ -672,6 +672,33 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
   }
 }
 
+// Units of the lane-per-query lists: claim c of nc takes g of the n parts of
+// the list's items, an item (a vertex's chunk of DCHUNK edges) having 2^sh
+// parts.  On skewed graphs (mix) a claim's parts are spread over the list,
+// which follows vertex ids and so degrees; else they are consecutive.
+struct DenseClaim {
+  u32 n, g, nc, sh, c;
+  bool mix;
+  // 64 items per claim, halved while the claims would be fewer than four per
+  // wave, and items of fewer than one per wave split down to 16 edges.  64 items
+  // are up to 8192 edges, which a wave takes 1.2 ms for, and that was the
+  // length of a launch on any small graph (with 64 / with this rule: RMAT-14
+  // 11 SSSP 2.6 / 1.0 ms, a 300007-vertex directed graph with 11 SSSP 6.3 /
+  // 2.9 ms, RMAT-20 64 SSSP 7.5 / 6.5 ms, RMAT-22 mixed 256 47.4 / 46.9 ms;
+  // with twelve claims per wave 1.08, 3.0, 6.5 and 47.1 ms).  Consecutive items
+  // on skewed graphs measured 7.1 ms on RMAT-20.
+  __device__ __forceinline__ DenseClaim(u32 items, u32 nw, bool mix_) : g(64), sh(0), c(0), mix(mix_) {
+    while (sh < 3 && (items << (sh + 1)) <= nw) ++sh;
+    n = items << sh;
+    while (g > 1 && n < g * 4u * nw) g /= 2;
+    nc = (n + g - 1) / g;
+  }
+  __device__ __forceinline__ u32 at(int lane) const { return mix ? c + (u32)lane * nc : c * g + (u32)lane; }
+  __device__ __forceinline__ u32 len() const { return (u32)DCHUNK >> sh; }
+  // Index of a part among the parts of its vertex (chunk: its item's).
+  __device__ __forceinline__ u32 part(u32 at, u32 chunk) const { return (chunk << sh) | (at & ((1u << sh) - 1u)); }
+};
+
 // Phase D: a wave takes up to 64 dense (vertex, word, chunk) items at once,
 // flattens their edges as above, and walks them U per step with lane q as
 // query q.  Every value load is unconditional (inactive lanes read a clamped
@@ -679,18 +706,19 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
 // are all in flight together, and the loads of step k+1 are issued before
 // the atomics of step k, so waiting for them never waits on the atomics.
 template <int W, bool SPARSE, int U, bool NF>
-__device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, int rshift, u32 stamp,
+__device__ __forceinline__ void expand_flat_dense(const KP& P, const DenseClaim& dc, int rshift, u32 stamp,
                                                   u32 thr, Tally& t) {
   const int lane = lane_id();
   const int R = 1 << rshift;
   const u32 p = P.ctl->iter & 1u;
-  const bool have = base + (u32)lane < n;
-  const u64 item = have ? P.dense[p][base + lane] : 0ull;
+  const u32 at = dc.at(lane);
+  const bool have = (u32)lane < dc.g && at < dc.n;
+  const u64 item = have ? P.dense[p][at >> dc.sh] : 0ull;
   const int32_t u = (int32_t)(item >> 32);
   const int w = (int)((item >> 24) & 0xFF);
-  const u32 chunk = (u32)(item & 0xFFFFFF);
-  const int32_t e0 = have ? P.off[u] + (int32_t)(chunk * DCHUNK) : 0;
-  const int32_t e1 = have ? min(P.off[u + 1], e0 + DCHUNK) : 0;
+  const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
+  const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
+  const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
   u64 sm = have ? (P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) : 0ull;
   const bool inrow = lane < R;
   // Lane offset inside a value row; every lane reads a valid address of the
@@ -711,7 +739,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
     // item's source row (8 rows in flight); pairs at or above thr are
     // postponed (chunk 0 of the vertex keeps them in the next frontier) and
     // an item left with no near pair scans no edges.
-    const int nit = (int)min(64u, n - base);
+    const int nit = (int)__popcll(__ballot(have));  // a prefix of the lanes
     u64 near = sm;
     for (int i0 = 0; i0 < nit; i0 += 8) {
       u32 dv[8];
@@ -732,7 +760,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
         const u64 fm = __ballot(isfar);
         if (isfar) t.fmin = min(t.fmin, dv[k]);
         if (lane == it) near = sm & ~fm;
-        if (fm && __builtin_amdgcn_readlane((int)chunk, it) == 0) {
+        if (fm && __builtin_amdgcn_readlane((int)part, it) == 0) {
           const int32_t uk = __builtin_amdgcn_readlane(u, it);
           const int wk = __builtin_amdgcn_readlane(w, it);
           bool claimed = false;
@@ -883,18 +911,19 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, u32 base, u32 n, 
 // Steps past the window's last edge read an entry of weight CGP_INF, so they
 // cannot improve anything.
 template <int W, bool SPARSE, int U, bool A64>
-__device__ __forceinline__ void expand_flat_dense_tab(const KP& P, u32 base, u32 n, int rshift, u32 stamp,
+__device__ __forceinline__ void expand_flat_dense_tab(const KP& P, const DenseClaim& dc, int rshift, u32 stamp,
                                                       uint4* tab, u32* wtab, Tally& t) {
   const int lane = lane_id();
   const int R = 1 << rshift;
   const u32 p = P.ctl->iter & 1u;
-  const bool have = base + (u32)lane < n;
-  const u64 item = have ? P.dense[p][base + lane] : 0ull;
+  const u32 at = dc.at(lane);
+  const bool have = (u32)lane < dc.g && at < dc.n;
+  const u64 item = have ? P.dense[p][at >> dc.sh] : 0ull;
   const int32_t u = (int32_t)(item >> 32);
   const int w = (int)((item >> 24) & 0xFF);
-  const u32 chunk = (u32)(item & 0xFFFFFF);
-  const int32_t e0 = have ? P.off[u] + (int32_t)(chunk * DCHUNK) : 0;
-  const int32_t e1 = have ? min(P.off[u + 1], e0 + DCHUNK) : 0;
+  const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
+  const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
+  const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
   const u64 sm = have ? (P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) : 0ull;
   const u32 dlen = sm ? (u32)(e1 - e0) : 0u;
   if (have) {
@@ -1064,17 +1093,18 @@ __device__ __forceinline__ u64 row_bcast64(u64 x) {
 // phase D (no near-far split: the filter routes items here only when
 // postponing is off).
 template <int W, bool SPARSE>
-__device__ __forceinline__ void expand_flat_narrow(const KP& P, u32 base, u32 n, int rshift, u32 stamp,
+__device__ __forceinline__ void expand_flat_narrow(const KP& P, const DenseClaim& dc, int rshift, u32 stamp,
                                                    Tally& t) {
   const int lane = lane_id();
   const u32 p = P.ctl->iter & 1u;
-  const bool have = base + (u32)lane < n;
-  const u64 item = have ? P.dense_n[p][base + lane] : 0ull;
+  const u32 at = dc.at(lane);
+  const bool have = (u32)lane < dc.g && at < dc.n;
+  const u64 item = have ? P.dense_n[p][at >> dc.sh] : 0ull;
   const int32_t u = (int32_t)(item >> 32);
   const int w = (int)((item >> 24) & 0xFF);
-  const u32 chunk = (u32)(item & 0xFFFFFF);
-  const int32_t e0 = have ? P.off[u] + (int32_t)(chunk * DCHUNK) : 0;
-  const int32_t e1 = have ? min(P.off[u + 1], e0 + DCHUNK) : 0;
+  const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
+  const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
+  const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
   const u32 sm = have ? (u32)(P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) & 0xFFFFu : 0u;
   const u32 d = sm ? (u32)(e1 - e0) : 0u;
   if (have) {
@@ -1271,7 +1301,7 @@ __device__ __forceinline__ bool pull_vertex_wave(const KP& P, int32_t v, const u
 __device__ __forceinline__ u32 wave_fetch(u32* ctr, u32 n) {
   u32 i = 0;
   if (lane_id() == 0) i = atomicAdd(ctr, n);
-  return (u32)__shfl((int)i, 0, 64);
+  return (u32)uniform32((int32_t)i);  // lane 0 is active: whole waves come here
 }
 
 // Wave-level claims of the units [0, n), in NSHARD contiguous shards: shard s
@@ -1430,7 +1460,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
     for (int w = 0; w < W; ++w) bb[w] = P.cfg->bfs_bits[w];
     const u32 nH = (u32)P.n_pull_hi;
     while (nH) {
-      const u32 i = wave_fetch(&C->fetch[p][4].v, 1u);
+      const u32 i = wave_fetch(&C->pull_hi[p].v, 1u);
       if (i >= nH) break;
       const int32_t v = P.pull_hi[i];
       bool claimed = false;
@@ -1509,17 +1539,13 @@ __global__ __launch_bounds__(BS) void k_adv_dense(KP P) {
   __shared__ u32 s_wt[TAB == 2 ? BS : 1];
   uint4* tab = s_tab + (TAB ? (threadIdx.x & ~63u) : 0u);
   u32* wtab = s_wt + (TAB == 2 ? (threadIdx.x & ~63u) : 0u);
-  // One group of 64 items per fetch: items carry up to DCHUNK edges each, so
-  // coarser claims leave a long tail (measured 2.5x slower at 4 groups).  A
-  // single cursor: the per-XCD shards of the other phases measured about
-  // 1 ms slower here on the RMAT-22 mixed batch (29.8 against 28.9 ms), the
-  // stealing at the end of the shards lengthening the tail.
-  while (true) {
-    const u32 i = wave_fetch(&C->fetch[p][1].v, 64u);
-    if (i >= nD) break;
-    if (TAB) expand_flat_dense_tab<W, SPARSE, U, TAB == 2>(P, i, nD, rshift, stamp, tab, wtab, t);
-    else if (thr == INF) expand_flat_dense<W, SPARSE, U, false>(P, i, nD, rshift, stamp, thr, t);
-    else expand_flat_dense<W, SPARSE, U, true>(P, i, nD, rshift, stamp, thr, t);
+  DenseClaim dc(nD, gridDim.x * (BS / 64), P.mix_small);
+  u32 lo, hi;
+  for (ShardFetch sf(dc.nc, 1, 0, true); sf.next(C->shard[p][SH_D], lo, hi);) {
+    dc.c = sf.unit(lo);
+    if (TAB) expand_flat_dense_tab<W, SPARSE, U, TAB == 2>(P, dc, rshift, stamp, tab, wtab, t);
+    else if (thr == INF) expand_flat_dense<W, SPARSE, U, false>(P, dc, rshift, stamp, thr, t);
+    else expand_flat_dense<W, SPARSE, U, true>(P, dc, rshift, stamp, thr, t);
   }
   flush_near_far(P, t, thr);
   if (P.profile) {
@@ -1558,9 +1584,11 @@ __global__ __launch_bounds__(BLOCK) void k_adv_narrow(KP P) {
   const bool sparse = C->dense_mode == 0;
   Tally t;
   u32 lo, hi;
-  for (ShardFetch sf(nN, 64u, 0); sf.next(C->shard[p][SH_N], lo, hi);) {
-    if (sparse) expand_flat_narrow<W, true>(P, sf.unit(lo), sf.unit(hi), rshift, stamp, t);
-    else expand_flat_narrow<W, false>(P, sf.unit(lo), sf.unit(hi), rshift, stamp, t);
+  DenseClaim dc(nN, gridDim.x * (BLOCK / 64), P.mix_small);
+  for (ShardFetch sf(dc.nc, 1, 0, true); sf.next(C->shard[p][SH_N], lo, hi);) {
+    dc.c = sf.unit(lo);
+    if (sparse) expand_flat_narrow<W, true>(P, dc, rshift, stamp, t);
+    else expand_flat_narrow<W, false>(P, dc, rshift, stamp, t);
   }
   if (P.profile) {
     prof_add(P, PF_DENSE_ITEMS, t.ditems);
@@ -1994,6 +2022,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
 #pragma unroll
     for (int w = 0; w < W; ++w) unw[w] = wave_or64(un[w]);
     if (lane == 0) {
+  static_assert(128 + NSH * NSHARD <= BLOCK, "one thread per work cursor");
       u64* r = s_st + (tid >> 6) * FSTAT;
 #pragma unroll
       for (int i = 0; i < NSUM; ++i) r[i] = sums[i];
@@ -2048,11 +2077,11 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     Ctr& c = C->bcount[tid < 5 ? np : p][tid % 5];
     s_cnt[tid] = __hip_atomic_load(&c.v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (tid >= 5) c.v = 0;
-  } else if (tid < 10 + 7) {
-    C->fetch[p][tid - 10].v = 0;
-  } else if (tid < 17 + NSTRIPE + 1) {
-    C->done[tid - 17].v = 0;
-  } else if (tid == 17 + NSTRIPE + 1) {
+  } else if (tid == 10) {
+    C->pull_hi[p].v = 0;
+  } else if (tid < 11 + NSTRIPE + 1) {
+    C->done[tid - 11].v = 0;
+  } else if (tid == 11 + NSTRIPE + 1) {
     C->tcount[(stamp & 1u) ^ 1u].v = 0;  // filled next; this iteration's is reset by the next filter
   }
   if (tid >= 64 && tid < 128) {
@@ -2072,7 +2101,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       x.near_new |= (u32)__shfl_xor((int)x.near_new, d, 64);
     }
     if (i == 0) s_stripe = x;
-  } else if (tid >= 128 && tid < 128 + 5 * NSHARD) {
+  } else if (tid >= 128 && tid < 128 + NSH * NSHARD) {
     C->shard[p][(tid - 128) / NSHARD][(tid - 128) % NSHARD].v = 0;
   }
   __syncthreads();

@@ -59,7 +59,7 @@ constexpr int PCHUNK = 256;        // edges per SSSP pull item
 // CSR rows and source rows stay in that XCD's L2, and the cursors' atomics
 // spread over NSHARD lines instead of one.
 constexpr int NSHARD = 8;
-enum : int { SH_M = 0, SH_S, SH_L, SH_N, SH_P };
+enum : int { SH_M = 0, SH_S, SH_L, SH_D, SH_N, SH_P, NSH };
 // Workgroups spread their end-of-launch atomics over NSTRIPE lines (by
 // workgroup index); the filter's last workgroup combines them.  One line takes
 // about 12 ns per atomic whoever sends it, so 2048 workgroups on one line were
@@ -160,9 +160,8 @@ struct Ctl {
   Ctr tcount[2];              // touched-list length, by parity of the iteration that fills it
   Ctr done[NSTRIPE + 1];      // filter last-workgroup detection: by workgroup index, then all
   Ctr bcount[2][5];           // [parity][small, medium, large items, dense items, narrow dense items]
-  Ctr fetch[2][7];            // [parity] work cursors of the advance without shards (unused, D, unused,
-                              // unused, pull-high, unused, unused)
-  Ctr shard[2][5][NSHARD];    // [parity][M, S, L, N, SSSP pull] per-shard work cursors
+  Ctr pull_hi[2];             // [parity] work cursor of the bottom-up step's high-degree vertices
+  Ctr shard[2][NSH][NSHARD];  // [parity][phase] per-shard work cursors
 };
 // Bytes of Ctl the host reads back after a run of iterations.
 constexpr size_t CTL_HOST_BYTES = offsetof(Ctl, stripe);

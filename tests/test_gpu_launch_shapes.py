@@ -82,3 +82,20 @@ def test_push_mask_words(gpu, n, directed):
     off, idx, wt = ring_graph(V, hub_degree=2500, seed=n, directed=directed)
     kinds = [SSSP] * (n // 3) + [BFS] * (n - n // 3)
     check(off, idx, wt, kinds, [(i * 131) % V for i in range(n)], runs=2, advance_blocks=2)
+
+
+# Lane-per-query lists: claims of 1 to 64 items of at most 128 edges, items
+# split down to 16 edges when the launch has more waves than items.  At most 16
+# SSSP queries go to the narrow list (four edges per step), more to the wide
+# one; dense_threshold=1 sends every SSSP word there.
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 70])
+@pytest.mark.parametrize("hub", [15, 127, 129, 3000])
+@pytest.mark.parametrize("opts", [dict(), dict(advance_blocks=1), dict(advance_blocks=9, frontier_dense_div=1),
+                                  dict(dense_wide_addr=1, advance_blocks=2), dict(sssp_delta=60, advance_blocks=2),
+                                  dict(dense_unroll=4)],
+                         ids=["default", "one_block", "sparse", "wide_addr", "near_far", "unroll4"])
+def test_lane_per_query_lists(gpu, n, hub, opts):
+    V = 4099
+    off, idx, wt = ring_graph(V, hub_degree=hub, seed=n, chords=2)
+    check(off, idx, wt, [SSSP] * n + [BFS], [(i * 131) % V for i in range(n)] + [3], runs=2, dense_threshold=1,
+          **opts)
