@@ -99,3 +99,24 @@ def test_lane_per_query_lists(gpu, n, hub, opts):
     off, idx, wt = ring_graph(V, hub_degree=hub, seed=n, chords=2)
     check(off, idx, wt, [SSSP] * n + [BFS], [(i * 131) % V for i in range(n)] + [3], runs=2, dense_threshold=1,
           **opts)
+
+
+# Weak components of directed graphs: below 4096 vertices every edge hooks, from
+# there on after a sample of two out-edges per vertex.  Edges only enter the
+# last vertices, and two parts stay apart.
+@pytest.mark.parametrize("V", [4095, 4096, 4097, 70001])
+def test_wcc_directed(gpu, V):
+    rng = np.random.RandomState(V)
+    half = V // 2
+    top = half * 4 // 5  # no edge leaves the first part's vertices from here on
+    a = np.concatenate([rng.randint(0, top, V), rng.randint(half, V, V // 3)])
+    b = np.concatenate([rng.randint(0, half, V), rng.randint(half, V, V // 3)])
+    keep = (a != b) & ((a < half) == (b < half))
+    key = np.unique(a[keep].astype(np.int64) * V + b[keep])
+    src, dst = key // V, key % V
+    off = np.zeros(V + 1, np.int64)
+    np.add.at(off, src + 1, 1)
+    off = np.cumsum(off).astype(np.int32)
+    got = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, dst.astype(np.int32))).wcc(2)
+    exp = O.expected(O.G(off, dst.astype(np.int32), None), WCC, 0)
+    assert np.array_equal(got[0], exp) and np.array_equal(got[1], exp)
