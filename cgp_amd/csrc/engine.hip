@@ -1510,16 +1510,24 @@ __device__ __forceinline__ void flush_tally(const KP& P, const Tally& t) {
   prof_add(P, PF_SSSP_SRC, t.src);
 }
 
+template <int W, bool SPARSE, int U, int TAB>
+__device__ __forceinline__ void expand_dense_claim(const KP& P, const DenseClaim& dc, int rshift, u32 stamp, u32 thr,
+                                                   uint4* tab, u32* wtab, Tally& t) {
+  if (TAB) expand_flat_dense_tab<W, SPARSE, U, TAB == 2>(P, dc, rshift, stamp, tab, wtab, t);
+  else if (thr == INF) expand_flat_dense<W, SPARSE, U, false>(P, dc, rshift, stamp, thr, t);
+  else expand_flat_dense<W, SPARSE, U, true>(P, dc, rshift, stamp, thr, t);
+}
+
 // The advance of one iteration is two persistent launches of BS-thread
 // workgroups (BS is a tuning parameter: 128, 256 or 512).  k_adv_dense runs
-// the lane-per-query rows of dense SSSP words (phase D) with its own lean
-// register budget, one instantiation per frontier mode (the one that does
-// not match the device-selected mode exits at once); k_adv_push runs phases
-// L, M, S and P.
-template <int W, int BS, bool SPARSE, int U, int TAB>
+// the lane-per-query rows of dense SSSP words (phase D) with its own register
+// budget; k_adv_push runs phases L, M, S and P.  Both frontier modes are in one
+// kernel: they need the same registers (142 and 145 at W = 4, U = 16), and a
+// launch that exits at once still takes 4.5 us of every iteration.
+template <int W, int BS, int U, int TAB>
 __global__ __launch_bounds__(BS) void k_adv_dense(KP P) {
   Ctl* C = P.ctl;
-  if (C->finished || (C->dense_mode == 0) != SPARSE || C->sssp_pull) return;
+  if (C->finished || C->sssp_pull) return;
   const u32 iter = C->iter, p = iter & 1u;
   const u32 nD = C->bcount[p][3].v;
   if (nD == 0) return;
@@ -1539,13 +1547,13 @@ __global__ __launch_bounds__(BS) void k_adv_dense(KP P) {
   __shared__ u32 s_wt[TAB == 2 ? BS : 1];
   uint4* tab = s_tab + (TAB ? (threadIdx.x & ~63u) : 0u);
   u32* wtab = s_wt + (TAB == 2 ? (threadIdx.x & ~63u) : 0u);
+  const bool sparse = C->dense_mode == 0;
   DenseClaim dc(nD, gridDim.x * (BS / 64), P.mix_small);
   u32 lo, hi;
   for (ShardFetch sf(dc.nc, 1, 0, true); sf.next(C->shard[p][SH_D], lo, hi);) {
     dc.c = sf.unit(lo);
-    if (TAB) expand_flat_dense_tab<W, SPARSE, U, TAB == 2>(P, dc, rshift, stamp, tab, wtab, t);
-    else if (thr == INF) expand_flat_dense<W, SPARSE, U, false>(P, dc, rshift, stamp, thr, t);
-    else expand_flat_dense<W, SPARSE, U, true>(P, dc, rshift, stamp, thr, t);
+    if (sparse) expand_dense_claim<W, true, U, TAB>(P, dc, rshift, stamp, thr, tab, wtab, t);
+    else expand_dense_claim<W, false, U, TAB>(P, dc, rshift, stamp, thr, tab, wtab, t);
   }
   flush_near_far(P, t, thr);
   if (P.profile) {
@@ -2014,6 +2022,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   __shared__ Stripe s_stripe;
   const int tid = (int)threadIdx.x;
   static_assert(NSUM + MAXW <= FSTAT && FSTAT <= 64, "a statistics line is written by one wave");
+  static_assert(128 + NSH * NSHARD <= BLOCK, "one thread per work cursor");
   {
     u64 sums[NSUM] = {pairs, epairs, fedges, apairs, averts, aqedges};
 #pragma unroll
@@ -2022,7 +2031,6 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
 #pragma unroll
     for (int w = 0; w < W; ++w) unw[w] = wave_or64(un[w]);
     if (lane == 0) {
-  static_assert(128 + NSH * NSHARD <= BLOCK, "one thread per work cursor");
       u64* r = s_st + (tid >> 6) * FSTAT;
 #pragma unroll
       for (int i = 0; i < NSUM; ++i) r[i] = sums[i];
@@ -2626,25 +2634,17 @@ __global__ __launch_bounds__(BLOCK) void k_reached(const int32_t* off, const int
 // ============================================================== host side
 namespace {
 
-// Both frontier-mode instantiations of the lane-per-query advance (the one
-// not matching the device-selected mode exits at once), U = rows per step.
-// It is wave-level work, so it always runs 256-thread workgroups.
+// The lane-per-query advance, U = rows per step.  It is wave-level work, so it
+// always runs 256-thread workgroups.
 template <int W, int U>
 void launch_dense_u(hipStream_t s, dim3 grid, const KP& P, int tab) {
-  if (tab == 1) {
-    hipLaunchKernelGGL((k_adv_dense<W, BLOCK, false, U, 1>), grid, dim3(BLOCK), 0, s, P);
-    hipLaunchKernelGGL((k_adv_dense<W, BLOCK, true, U, 1>), grid, dim3(BLOCK), 0, s, P);
-  } else if (tab == 2) {
-    hipLaunchKernelGGL((k_adv_dense<W, BLOCK, false, U, 2>), grid, dim3(BLOCK), 0, s, P);
-    hipLaunchKernelGGL((k_adv_dense<W, BLOCK, true, U, 2>), grid, dim3(BLOCK), 0, s, P);
-  } else {
-    hipLaunchKernelGGL((k_adv_dense<W, BLOCK, false, U, 0>), grid, dim3(BLOCK), 0, s, P);
-    hipLaunchKernelGGL((k_adv_dense<W, BLOCK, true, U, 0>), grid, dim3(BLOCK), 0, s, P);
-  }
+  if (tab == 1) hipLaunchKernelGGL((k_adv_dense<W, BLOCK, U, 1>), grid, dim3(BLOCK), 0, s, P);
+  else if (tab == 2) hipLaunchKernelGGL((k_adv_dense<W, BLOCK, U, 2>), grid, dim3(BLOCK), 0, s, P);
+  else hipLaunchKernelGGL((k_adv_dense<W, BLOCK, U, 0>), grid, dim3(BLOCK), 0, s, P);
 }
 
 // Optional advance launches of the current slot configuration: bit 0, the
-// lane-per-query kernels (some word has SSSP slots); bit 1, the narrow
+// wide lane-per-query kernel (some word has SSSP slots); bit 1, the narrow
 // kernel (some word is narrow now, or was when the last filter binned the
 // frontier this advance expands: serving admission can end the narrow
 // regime between a filter and the next advance); bit 2, the SSSP pull
@@ -2654,8 +2654,11 @@ void launch_dense_u(hipStream_t s, dim3 grid, const KP& P, int tab) {
 int launch_set(const cgp_engine* en) {
   const Cfg& c = *en->h_cfg;
   int ls = 0;
-  for (int w = 0; w < MAXW; ++w)
-    if (c.val_bits[w]) ls |= 1;
+  // In a batch run narrow words are all of the SSSP words from the seeding
+  // filter on, and the wide list stays empty.
+  if (!c.narrow_words || en->serve)
+    for (int w = 0; w < MAXW; ++w)
+      if (c.val_bits[w]) ls |= 1;
   if (c.narrow_words || en->narrow_binned) ls |= 2;
   if (c.sssp_pull_policy) ls |= 4;
   return ls;
@@ -2819,6 +2822,7 @@ void compute_wcc(cgp_engine* en) {
   int32_t* parent = (int32_t*)en->parent.p;
   const int gb = en->cus * 16;
   hipLaunchKernelGGL(k_wcc_init, dim3(gb), dim3(BLOCK), 0, en->s, parent, g->V);
+  constexpr int kSample = 2, kProbe = 1024;
   if (!g->symmetric || g->V < 4096) {
     // Directed graphs (weak components need every stored edge) and tiny
     // graphs: a hooking pass over all edges.  On larger graphs every vertex
@@ -2831,7 +2835,6 @@ void compute_wcc(cgp_engine* en) {
                          (const int32_t*)g->idx, g->V, kSample, parent);
       hipLaunchKernelGGL(k_wcc_compress, dim3(gb), dim3(BLOCK), 0, en->s, parent, g->V);
     }
-  constexpr int kSample = 2, kProbe = 1024;
     hipLaunchKernelGGL(k_wcc_hook, dim3(gb), dim3(BLOCK), 0, en->s, (const int32_t*)g->rows,
                        (const int32_t*)g->idx, g->E, parent, g->symmetric ? 1 : 0);
   } else {
