@@ -247,16 +247,20 @@ struct cgp_engine {
   // Grid sizes: persistent-style, sized to the device, independent of the
   // frontier so the launches can be captured once and replayed.
   // Same thread count per launch for every workgroup size.
-  // Advance workgroups: `advance_blocks`, or by default one per 65536 edges
-  // between one and eight per CU.  The persistent advance launches fetch
-  // their work dynamically, so workgroups beyond what the frontier keeps
-  // busy only add start-up and fetch cost (RMAT-20 64 SSSP: 9.5 ms at 2048
-  // workgroups, 8.6 ms at 480; RMAT-22 and the 4096^2 grid are flat between
-  // 1024 and 2048).
+  // Advance workgroups: `advance_blocks`, or by default one per 24576 edges
+  // between one and three per CU.  The advance launches are persistent and
+  // hand their work out, so three per CU, as many as fit (141-146 registers:
+  // three waves per SIMD), is the most that helps: later ones start when the
+  // work is gone and only find that out (at 256 / 512 / 768 / 1024 / 2048
+  // workgroups RMAT-22 mixed 256 takes 78.5 / 51.6 / 45.8 / 47.4 / 47.2 ms and
+  // 160 BFS 10.5 / 8.4 / 8.35 / 8.9 / 8.9 ms).  Below, the frontiers are too
+  // short for more: RMAT-18 (7.5 M edges) one SSSP 844 us at 256, 889 at 512;
+  // 2048^2 grid (17 M) 128 SSSP 151 / 117.5 / 113.8 / 112.4 ms at 256 / 512 /
+  // 640 / 768; RMAT-20 (31 M) 64 SSSP 8.6 / 6.35 / 6.23 / 6.30 ms.
   int advance_blocks() const {
     if (opts.advance_blocks > 0) return opts.advance_blocks;
-    const int64_t want = g->E / 65536;
-    return (int)std::max<int64_t>(cus, std::min<int64_t>(want, (int64_t)cus * 8));
+    const int64_t want = g->E / 24576;
+    return (int)std::max<int64_t>(cus, std::min<int64_t>(want, (int64_t)cus * 3));
   }
   int grid_advance() const { return (int)((int64_t)advance_blocks() * 256 / std::max(128, opts.block_size)); }
   // Filter workgroups: no more than have vertices to look at (each looks at
