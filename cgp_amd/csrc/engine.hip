@@ -1788,11 +1788,6 @@ __global__ __launch_bounds__(BLOCK) void k_seed(KP P, const int32_t* slot_src, i
 }
 
 // ------------------------------------------------------------------ filter
-template <typename T>
-__device__ __forceinline__ T* pick(T* a, T* b, u32 which) {
-  return (T*)((u64)a ^ (((u64)a ^ (u64)b) & (0ull - (u64)which)));
-}
-
 // Vertex i of the filter's list (i < n: the scan's i, or touched[i]), its next
 // words and CSR offsets; zeros past the end.  The W next words of a record
 // are contiguous and 16-byte aligned (W >= 2).
@@ -1864,14 +1859,14 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   // reservation per 256 vertices cost about 0.3 ms per dense iteration on
   // RMAT-22).
   const u32 gstride = active * BLOCK * FK;
-  // The next iteration's bin lists, picked once, by arithmetic: indexing the
-  // argument's arrays with np, or selecting between their entries, makes the
-  // compiler copy the whole argument block (240 bytes a lane) to scratch memory.
-  int32_t* const l_small = pick(P.small[0], P.small[1], np);
-  int32_t* const l_medium = pick(P.medium[0], P.medium[1], np);
-  u64* const l_large = pick(P.large[0], P.large[1], np);
-  u64* const l_dense = pick(P.dense[0], P.dense[1], np);
-  u64* const l_dense_n = pick(P.dense_n[0], P.dense_n[1], np);
+  // The next iteration's bin lists, picked once (indexing the argument's
+  // arrays with np inside the loop made the compiler copy the whole
+  // argument block to scratch memory).
+  int32_t* const l_small = np ? P.small[1] : P.small[0];
+  int32_t* const l_medium = np ? P.medium[1] : P.medium[0];
+  u64* const l_large = np ? P.large[1] : P.large[0];
+  u64* const l_dense = np ? P.dense[1] : P.dense[0];
+  u64* const l_dense_n = np ? P.dense_n[1] : P.dense_n[0];
   for (u32 base = blockIdx.x * BLOCK * FK; base < n; base += gstride) {
     int32_t vv[FK], o0[FK], o1[FK];
     u64 nwk[FK][W];
@@ -2019,7 +2014,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   __shared__ u64 s_red[(BLOCK / FSTAT) * FSTAT];
   __shared__ u64 s_tot[FSTAT];
   __shared__ u32 s_cnt[10];  // the five lists' lengths: next frontier, consumed frontier
-  __shared__ Stripe s_stripe;
+  __shared__ u64 s_adv_t1, s_den_t1;
+  __shared__ u32 s_far_min, s_near_new;
   const int tid = (int)threadIdx.x;
   static_assert(NSUM + MAXW <= FSTAT && FSTAT <= 64, "a statistics line is written by one wave");
   static_assert(128 + NSH * NSHARD <= BLOCK, "one thread per work cursor");
@@ -2039,7 +2035,9 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     }
   }
   __syncthreads();
-  if (tid < 64) {
+  // (A workgroup that was alone has everything in its LDS and reports nothing:
+  // three round trips to memory less on every short frontier.)
+  if (active > 1 && tid < 64) {
     if (tid < NSUM + W) {
       u64 x = s_st[tid];
       for (int wv = 1; wv < NW; ++wv) {
@@ -2064,8 +2062,10 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       }
     }
   }
-  __syncthreads();
-  if (!s_last) return;
+  if (active > 1) {
+    __syncthreads();
+    if (!s_last) return;
+  }
   // Last workgroup: advance the state machine.  Its threads collect what the
   // iteration left, and reset the consumed counters, side by side; then one
   // thread decides.
@@ -2073,7 +2073,9 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     // Thread (g, k): entry k of every (BLOCK / FSTAT)-th line.
     const int k = tid % FSTAT, g = tid / FSTAT;
     u64 x = 0;
-    if (k < NSUM + W)
+    if (active == 1) {
+      if (g < NW && k < NSUM + W) x = s_st[g * FSTAT + k];
+    } else if (k < NSUM + W) {
       for (u32 b = (u32)g; b < active; b += BLOCK / FSTAT) {
         const u64 y =
             __hip_atomic_load(&P.fstat[(size_t)b * FSTAT + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -2095,20 +2097,31 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   if (tid >= 64 && tid < 128) {
     // One wave combines the stripes.
     const int i = tid - 64;
-    Stripe x{0, 0, INF, 0};
+    u64 a1 = 0, d1 = 0;
+    u32 fm = INF, nn = 0;
     if (i < NSTRIPE) {
-      x = C->stripe[i];
-      C->stripe[i] = Stripe{0, 0, INF, 0};
+      Stripe& x = C->stripe[i];
+      a1 = x.adv_t1;
+      d1 = x.den_t1;
+      fm = x.far_min;
+      nn = x.near_new;
+      x.adv_t1 = x.den_t1 = 0;
+      x.far_min = INF;
+      x.near_new = 0;
     }
 #pragma unroll
     for (int d = NSTRIPE / 2; d >= 1; d >>= 1) {
-      const u64 a1 = shfl64(x.adv_t1, lane ^ d), d1 = shfl64(x.den_t1, lane ^ d);
-      x.adv_t1 = max(x.adv_t1, a1);
-      x.den_t1 = max(x.den_t1, d1);
-      x.far_min = min(x.far_min, (u32)__shfl_xor((int)x.far_min, d, 64));
-      x.near_new |= (u32)__shfl_xor((int)x.near_new, d, 64);
+      a1 = max(a1, shfl64(a1, lane ^ d));
+      d1 = max(d1, shfl64(d1, lane ^ d));
+      fm = min(fm, (u32)__shfl_xor((int)fm, d, 64));
+      nn |= (u32)__shfl_xor((int)nn, d, 64);
     }
-    if (i == 0) s_stripe = x;
+    if (i == 0) {
+      s_adv_t1 = a1;
+      s_den_t1 = d1;
+      s_far_min = fm;
+      s_near_new = nn;
+    }
   } else if (tid >= 128 && tid < 128 + NSH * NSHARD) {
     C->shard[p][(tid - 128) / NSHARD][(tid - 128) % NSHARD].v = 0;
   }
@@ -2120,6 +2133,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       x = tid < NSUM ? x + y : x | y;
     }
     s_tot[tid] = x;
+    }
   }
   __syncthreads();
   if (tid == 0) {
@@ -2162,8 +2176,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     // Near-far: when no SSSP pair below the threshold is left, move it to
     // the smallest pending value plus delta (skipping empty buckets).
     if (cfg->delta != 0) {
-      const u32 fm = s_stripe.far_min;
-      if (s_stripe.near_new == 0 && fm != INF) {
+      const u32 fm = s_far_min;
+      if (s_near_new == 0 && fm != INF) {
         const u64 nt = (u64)fm + (u64)cfg->delta;
         C->thr = nt >= (u64)INF ? INF : (u32)nt;
         ++C->bumps;
@@ -2173,8 +2187,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     // ran iff iter != seeding.
     if (iter != 0xFFFFFFFFu) {
       const u64 den_t0 = C->den_t0, now = (u64)wall_clock64();
-      const u64 at = s_stripe.adv_t1 - C->adv_t0, ft = now - __hip_atomic_load(&C->flt_t0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const u64 dt = s_stripe.den_t1 > den_t0 ? s_stripe.den_t1 - den_t0 : 0ull;
+      const u64 at = s_adv_t1 - C->adv_t0, ft = now - __hip_atomic_load(&C->flt_t0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const u64 dt = s_den_t1 > den_t0 ? s_den_t1 - den_t0 : 0ull;
       C->adv_ticks += at;
       C->adv_launches += 1;
       C->flt_ticks += ft;
