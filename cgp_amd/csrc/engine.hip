@@ -271,13 +271,33 @@ __device__ __forceinline__ void note_improved(Tally& t, u32 c, u32 thr) {
 template <int W, bool SPARSE, int N, class BM, class SM>
 __device__ __forceinline__ void relax_edges(const KP& P, const int32_t (&u)[N], const int32_t (&v)[N],
                                             const u32 (&wv)[N], const bool (&ok)[N], BM bm, SM sm, bool any_b,
-                                            bool any_s, u32 stamp, int rshift, u32 thr, Tally& t) {
+                                            bool any_s, const u32* done, u32 stamp, int rshift, u32 thr,
+                                            Tally& t) {
   // nx: bits that next[v] already has; add: bits to set there.
   u64 nx[N][W], add[N][W];
   if (SPARSE || any_b) {
+    // Targets that every BFS query has visited need no record.
+    u32 dn[N];
+    if (done) {
+#pragma unroll
+      for (int i = 0; i < N; ++i) dn[i] = done[(u32)v[i] >> 5];
+#pragma unroll
+      for (int i = 0; i < N; ++i) dn[i] = (dn[i] >> ((u32)v[i] & 31u)) & 1u;
+    } else {
+#pragma unroll
+      for (int i = 0; i < N; ++i) dn[i] = 0;
+    }
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const size_t vb = vis_at<W>(v[i], 0);
+      if (dn[i]) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+          nx[i][w] = 0;
+          add[i][w] = ~0ull;
+        }
+        continue;
+      }
 #pragma unroll
       for (int w = 0; w < W; ++w) {
         nx[i][w] = P.next[vb + W + w];
@@ -475,7 +495,7 @@ __device__ __forceinline__ u64 lane64(u64 x, int k) {
 // the next unit too, are on their way while a step is relaxed.
 template <int W, bool SPARSE>
 __device__ __forceinline__ void expand_units(const KP& P, int cnt, int32_t u, int32_t e0, int32_t e1, bool lead,
-                                             bool bfs_on, int dense_t, int rshift, u32 stamp, u32 thr, Tally& t) {
+                                             const u32* done, bool bfs_on, int dense_t, int rshift, u32 stamp, u32 thr, Tally& t) {
   // Steps in flight: as many as leave the kernel three waves per SIMD (four at
   // W = 1).  One RMAT-18 SSSP query at N = 1 / 4: 980 / 820 us; 160 BFS on
   // RMAT-22 (W = 4) at 1 / 2 / 4: 9.2 / 9.5 / 11.6 ms.
@@ -553,7 +573,7 @@ __device__ __forceinline__ void expand_units(const KP& P, int cnt, int32_t u, in
     for (int i = 0; i < N; ++i) uu[i] = uk;
     relax_edges<W, SPARSE, N>(
         P, uu, cur.v, cur.wv, cur.ok, [&](int, int w) { return bk[w]; }, [&](int, int w) { return sk[w]; }, k_b, k_s,
-        stamp, rshift, thr, t);
+        done, stamp, rshift, thr, t);
     cur = nxt;
   }
 }
@@ -602,7 +622,7 @@ __device__ __forceinline__ int wave_upper_bound(u32 incl, u32 f) {
 // are relaxed together.
 template <int W, bool SPARSE>
 __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t* list, u32 g, u32 ng, u32 gsz, u32 n,
-                                                     bool bfs_on, int dense_t, int rshift, u32 stamp,
+                                                     const u32* done, bool bfs_on, int dense_t, int rshift, u32 stamp,
                                                      u32 thr, Tally& t) {
   constexpr int N = W == 1 ? 2 : 1;
   const int lane = lane_id();
@@ -668,7 +688,7 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
     if (win + 64 * N < total) fetch(win + 64 * N);
     relax_edges<W, SPARSE, N>(
         P, uj, v, wv, ok, [&](int i, int w) { return bj[i][w]; }, [&](int i, int w) { return sj[i][w]; }, wave_b,
-        wave_s, stamp, rshift, thr, t);
+        wave_s, done, stamp, rshift, thr, t);
   }
 }
 
@@ -1397,6 +1417,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   // threshold of 0 leaves no SSSP word to the push phases.
   const int rshift = P.cfg->rshift, dense_t = C->sssp_pull ? 0 : P.cfg->dense_t;
   const u32 nw = gridDim.x * (BS / 64);
+  const u32* const done = C->use_done ? P.done : nullptr;
   const int lane = lane_id();
   u32 lo, hi;
   // Phase L.  A chunk is two units, or up to 32 of 128 edges while that leaves
@@ -1414,8 +1435,8 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
       const int32_t u = (int32_t)(item >> 32);
       const int32_t e0 = P.off[u] + (int32_t)((u32)item * LCHUNK + part * ((u32)LCHUNK >> sh));
       const int32_t e1 = min(P.off[u + 1], e0 + (LCHUNK >> sh));
-      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, (u32)item == 0 && part == 0, bfs_on, dense_t, rshift,
-                              stamp, thr, t);
+      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, (u32)item == 0 && part == 0, done, bfs_on, dense_t,
+                              rshift, stamp, thr, t);
     }
   }
   // Phase M.  With fewer vertices than waves, 2, 4 or 8 waves take equal parts
@@ -1436,7 +1457,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
       // Parts of whole 64-edge steps.
       const int32_t len = (int32_t)((((u32)d + 63u) / 64u + (1u << sh) - 1u) >> sh) * 64;
       const int32_t e0 = b + (int32_t)part * len, e1 = min(b + d, e0 + len);
-      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, part == 0, bfs_on, dense_t, rshift, stamp, thr, t);
+      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, part == 0, done, bfs_on, dense_t, rshift, stamp, thr, t);
     }
   }
   // Phase S.  Groups of 64 entries, halved down to 4 while that leaves every
@@ -1449,7 +1470,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
     ShardFetch sf(ng, claim_units(ng, nw), 2);
     while (sf.next(C->shard[p][SH_S], lo, hi)) {
       for (u32 g = lo; g < hi; ++g)
-        expand_flat_vertices<W, SPARSE>(P, P.small[p], sf.unit(g), ng, gsz, nS, bfs_on, dense_t, rshift, stamp, thr, t);
+        expand_flat_vertices<W, SPARSE>(P, P.small[p], sf.unit(g), ng, gsz, nS, done, bfs_on, dense_t, rshift, stamp, thr, t);
     }
   }
   // Phase P: high-degree vertices one wave each (64 neighbours per step,
@@ -1853,6 +1874,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   const u32 depth_base = iter + 1u;
   u64 pairs = 0, epairs = 0, fedges = 0;
   u64 apairs = 0, averts = 0, aqedges = 0;  // every kind: pairs, vertices, query-weighted degree
+  u64 ndone = 0;  // vertices whose last BFS query this is
   // Each thread takes FK vertices per step (their loads issued together) and
   // the workgroup reserves their bin entries with one atomic per bin: the
   // bin counters are single addresses every workgroup contends for (one
@@ -1894,7 +1916,6 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
           P.front[(size_t)v * W + w] = nw;
         }
         nb[w] = nw & bb[w];
-        if (nb[w]) P.visited[vis_at<W>(v, w)] |= nb[w];
         const u64 s = nw & vb[w];
         if (s && __popcll(s) >= dense_t) (((cfg->narrow_words >> w) & 1u) ? nmask : dmask) |= 1u << w;
         else if (s) need_bin = true;
@@ -1902,6 +1923,26 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
         un[w] |= nw;
         vpairs += (u32)__popcll(nb[w]);
         allp += (u32)__popcll(nw);
+      }
+      bool all = vpairs != 0;
+      if (vpairs) {
+#pragma unroll
+        for (int w = 0; w < W; ++w) {
+          if (!bb[w]) continue;
+          const u64 x = P.visited[vis_at<W>(v, w)] | nb[w];
+          if (nb[w]) P.visited[vis_at<W>(v, w)] = x;
+          all &= (bb[w] & ~x) == 0;
+        }
+      }
+      if (P.done) {
+        ndone += all ? 1u : 0u;
+        if (scan) {
+          // A wave's vertices are 64 consecutive ones, which it alone looks at.
+          const u64 m = __ballot(all);
+          if (m && lane == 0) ((u64*)P.done)[(u32)v >> 6] |= m;
+        } else if (all) {
+          atomicOr(&P.done[(u32)v >> 5], 1u << ((u32)v & 31u));
+        }
       }
       pairs += vpairs;
       epairs += (u64)vpairs * (u64)deg;
@@ -2020,7 +2061,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   static_assert(NSUM + MAXW <= FSTAT && FSTAT <= 64, "a statistics line is written by one wave");
   static_assert(128 + NSH * NSHARD <= BLOCK, "one thread per work cursor");
   {
-    u64 sums[NSUM] = {pairs, epairs, fedges, apairs, averts, aqedges};
+    u64 sums[NSUM] = {pairs, epairs, fedges, apairs, averts, aqedges, ndone};
 #pragma unroll
     for (int i = 0; i < NSUM; ++i) sums[i] = wave_sum64(sums[i]);
     u64 unw[W];
@@ -2081,6 +2122,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
             __hip_atomic_load(&P.fstat[(size_t)b * FSTAT + k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         x = k < NSUM ? x + y : x | y;
       }
+    }
     s_red[g * FSTAT + k] = x;
   }
   if (tid < 10) {
@@ -2133,7 +2175,6 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       x = tid < NSUM ? x + y : x | y;
     }
     s_tot[tid] = x;
-    }
   }
   __syncthreads();
   if (tid == 0) {
@@ -2141,6 +2182,14 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     const u32 cur_items = s_cnt[5] + s_cnt[6] + s_cnt[7] + s_cnt[8] + s_cnt[9];
     const u64 fp = s_tot[0], fe = s_tot[1], fall = s_tot[2];
     const u64 napairs = s_tot[3], naverts = s_tot[4], naqedges = s_tot[5];
+    // The done bits are looked up from the iteration on that has enough of
+    // them to skip records by: the lookup is a load before the others.  (From a
+    // sixteenth, an eighth or a quarter of the vertices on: RMAT-22 one BFS and
+    // WCC 1.87 / 1.96 / 1.95 ms, 2.30 without them; 160 BFS 7.8 / 7.9 / 7.9 ms,
+    // 8.2 without, where the last large iteration went from 1.28 to 0.78 ms.)
+    const u32 dv = C->done_verts + (u32)s_tot[6];
+    C->done_verts = dv;
+    C->use_done = P.done && dv > (u32)P.V / 16u ? 1u : 0u;
     const u32 cur_pull = C->bfs_pull, cur_spull = C->sssp_pull;
     const u32 dense = fall >= cfg->dense_fedges_thr ? 1u : 0u;
     C->dense_mode = dense;
@@ -2952,7 +3001,7 @@ static int bit_length(u64 x) { return x ? 64 - __builtin_clzll(x) : 0; }
 // traversal state, so the early copy is overwritten).  This takes the
 // readback's round trip (about 70 us) off the end of a batch.
 static bool run_iterations(cgp_engine* en, int W, bool no_graph, const std::function<void()>& output) {
-  const KP P = en->kp();
+  const KP P = en->kp(W, !no_graph);
   const bool use_graph = en->opts.use_hip_graph != 0 && !no_graph;
   const int K = use_graph ? std::max(1, en->opts.graph_iterations) : 1;
   const int ls = launch_set(en);
@@ -3116,7 +3165,7 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
     while ((1 << rshift) < R) ++rshift;
     en->ensure_words(W);
     en->ensure_vals((size_t)W * V * R);
-    const KP P = en->kp();
+    const KP P = en->kp(W, !no_alloc);
     // Slot configuration.
     Cfg& cfg = *en->h_cfg;
     std::memset(&cfg, 0, sizeof(Cfg));
@@ -3215,7 +3264,7 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
     }
     // Visited + next records (2W words per vertex) start clear; the layout
     // depends on W, so the whole region is cleared for every pass.
-    fill_u32(en->s, en->visited.p, (size_t)V * W * 4, 0u, en->cus);
+    fill_u32(en->s, en->visited.p, (size_t)V * W * 4 + (no_alloc ? 0 : en->done_bytes() / 4), 0u, en->cus);
     en->next_dirty = false;
     dispatch_seed(en, W, P, (const int32_t*)en->slot_src.p, W * 64);
     en->tick(CAT_INIT, false);

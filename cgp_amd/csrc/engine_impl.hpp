@@ -191,7 +191,9 @@ struct cgp_engine {
   // guarded by the serving module's pool mutex.
   std::vector<uint32_t*> result_pool;
 
-  KP kp() const {
+  // Kernel parameters; keep_done: of a batch pass of W words, whose done bits
+  // lie behind its records.
+  KP kp(int W = 0, bool keep_done = false) const {
     KP P{};
     P.V = g->V;
     P.E = g->E;
@@ -224,6 +226,7 @@ struct cgp_engine {
     P.cfg = d_cfg;
     P.iters = (cgpk::IterRec*)iters.p;
     P.fstat = d_fstat;
+    P.done = keep_done ? (u32*)((char*)visited.p + (size_t)g->V * W * 16) : nullptr;
     P.bin_small = opts.bin_small;
     P.bin_large = opts.bin_large;
     // Serving seeds queries into running iterations, where a full scan must
@@ -270,11 +273,15 @@ struct cgp_engine {
     return (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cus * 4));
   }
 
+  // Bytes of the per-vertex done bits, kept behind the visited + next records
+  // of the running pass's W and cleared with them.
+  size_t done_bytes() const { return ((size_t)g->V + 127) / 128 * 16; }
+
   void ensure_words(int W) {
     const size_t V = (size_t)g->V, E = (size_t)g->E;
     bool moved = false;
     if (W > wcap) {
-      moved |= visited.ensure(V * W * 16);  // visited + next records
+      moved |= visited.ensure(V * W * 16 + done_bytes());  // visited + next records, then the done bits
       moved |= front.ensure(V * W * 8);
       HIP_CHECK(hipMemsetAsync(visited.p, 0, V * W * 16, s));
       for (int k = 0; k < 2; ++k) {

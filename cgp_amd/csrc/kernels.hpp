@@ -67,9 +67,9 @@ enum : int { SH_M = 0, SH_S, SH_L, SH_D, SH_N, SH_P, NSH };
 constexpr int NSTRIPE = 16;
 constexpr int FK = 4;              // vertices per thread and step of the filter
 // Frontier statistics a filter workgroup leaves for the last one, in u64s of
-// one 128-byte line per workgroup: six sums, then the union of each word.
+// one 128-byte line per workgroup: seven sums, then the union of each word.
 constexpr int FSTAT = 16;
-constexpr int NSUM = 6;
+constexpr int NSUM = 7;
 
 // Per-batch slot configuration (device resident, rewritten per pass).
 struct Cfg {
@@ -143,6 +143,8 @@ struct Ctl {
   // dense_mode on while workgroups without work may not have started yet.
   u32 f_iter;
   u32 f_scan;       // that iteration's dense_mode
+  u32 done_verts;   // vertices that every BFS query of the pass has visited
+  u32 use_done;     // the push launch looks a target up in KP::done before its record
   u64 last_union[MAXW];       // OR of the frontier words the last filter produced
   u64 prof[NPROF];            // work counters (profile mode)
   // Device-clock launch timing (wall_clock64 ticks): start of the running
@@ -219,6 +221,9 @@ struct KP {
   const Cfg* cfg;
   IterRec* iters;
   u64* fstat;  // FSTAT words per filter workgroup
+  // Bit v: every BFS query of the pass has visited v (batch runs; null: not
+  // kept).  512 KiB for 2^22 vertices, so it stays in every XCD's L2.
+  u32* done;
   int32_t bin_small;
   int32_t bin_large;
   // Vertices a full compaction scan visits: [0, scan_v).  On a symmetric

@@ -59,6 +59,22 @@ def test_filter_workgroups(gpu, V, opts):
     check(off, idx, wt, kinds, [0, V // 2, V - 1, V - 1, V // 3, 0, V // 2, V // 5, 0], runs=3, **opts)
 
 
+# Batches of different mask widths in turn on one engine: the bits that mark
+# vertices every BFS query has visited lie behind the pass's own records.
+@pytest.mark.parametrize("V", [63, 64, 65, 127, 5001])
+@pytest.mark.parametrize("div", [1, 1 << 20])
+def test_mask_widths_in_turn(gpu, V, div):
+    off, idx, wt = ring_graph(V, hub_degree=V // 3, chords=4)
+    en = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, idx, wt), frontier_dense_div=div)
+    og = O.G(off, idx, wt)
+    for n in (150, 3, 70, 300, 1, 150):
+        kinds = [BFS if i % 7 else SSSP for i in range(n)]
+        src = [(i * 31 + n) % V for i in range(n)]
+        got = en.run_batch(kinds, src)[0]
+        for i, (k, s) in enumerate(zip(kinds, src)):
+            assert np.array_equal(got[i], O.expected(og, k, s)), (n, i, k, s)
+
+
 # Push work lists: vertices of at most 64 edges go 64 (or fewer) to a wave, of
 # at most 2048 one to a wave or part of one, larger ones in chunks of 4096
 # edges split into parts.  advance_blocks sets how many waves share the lists:
