@@ -358,9 +358,10 @@ __device__ __forceinline__ void relax_edges(const KP& P, const int32_t (&u)[N], 
             const u32 cand = __builtin_elementwise_add_sat(du[i][k], wv[i]);
             if (a[i][k] && cand < cur[i][k]) {
               atomicMin(&P.vals[vrow(P.V, w, v[i], rshift) + q[i][k]], cand);
-              add[i][w] |= (1ull << q[i][k]) & ~nx[i][w];
               ++t.imp;
               note_improved(t, cand, thr);
+              if (cand < thr) add[i][w] |= (1ull << q[i][k]) & ~nx[i][w];
+              else atomicOr(&P.far[(size_t)v[i] * W + w], 1ull << q[i][k]);
             }
           }
         }
@@ -417,12 +418,10 @@ __device__ __forceinline__ void count_edges(Tally& t, const u64 (&bm)[W], const 
 }
 
 // Frontier masks of vertex u: BFS bits, and the sparse SSSP bits (popcount
-// below dense_t; denser words go lane-per-query) split at the near-far
-// threshold: pairs whose value is >= thr land in far[] and are not expanded.
+// below dense_t; denser words go lane-per-query).
 template <int W>
-__device__ __forceinline__ void load_masks(const KP& P, int32_t u, bool bfs_on, int dense_t,
-                                           u32 thr, int rshift, u64 (&bm)[W], u64 (&sm)[W],
-                                           u64 (&far)[W], bool& any_w, Tally& t) {
+__device__ __forceinline__ void load_masks(const KP& P, int32_t u, bool bfs_on, int dense_t, u64 (&bm)[W],
+                                           u64 (&sm)[W], bool& any_w) {
   const Cfg* cfg = P.cfg;
   any_w = false;
 #pragma unroll
@@ -431,53 +430,57 @@ __device__ __forceinline__ void load_masks(const KP& P, int32_t u, bool bfs_on, 
     bm[w] = bfs_on ? (f & cfg->bfs_bits[w]) : 0ull;
     u64 s = f & cfg->val_bits[w];
     if (__popcll(s) >= dense_t) s = 0;  // handled lane-per-query
-    far[w] = 0;
-    if (s && thr != INF) {
-      const size_t ub = vrow(P.V, w, u, rshift);
-      u64 x = s;
-      while (x) {
-        int q[4];
-        bool a[4];
-        u32 d[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          a[i] = x != 0;
-          q[i] = a[i] ? __ffsll((long long)x) - 1 : q[0];
-          if (a[i]) x &= x - 1;
-          d[i] = P.vals[ub + q[i]];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          if (a[i] && d[i] >= thr) {
-            far[w] |= 1ull << q[i];
-            t.fmin = min(t.fmin, d[i]);
-          }
-        }
-      }
-      s &= ~far[w];
-    }
     sm[w] = s;
     any_w |= (s != 0);
   }
 }
 
-// Keeps u's postponed SSSP pairs in the next frontier.  Sparse mode returns
-// whether this made the vertex's first claim of the iteration.
+// The raise of the near-far threshold (old -> thr): every pair of the far set
+// with a value in [old, thr) joins the next frontier, pairs at or above thr
+// stay, and pairs below old leave the set: their value was lowered below the
+// threshold after they were put there, which put them into a frontier then.
+// No SSSP pair is expanded in this iteration, so values stand still.
 template <int W, bool SPARSE>
-__device__ __forceinline__ bool postpone(const KP& P, int32_t u, const u64 (&far)[W], u32 stamp,
-                                         Tally& t) {
-  bool first = false;
+__device__ __forceinline__ void raise_far(const KP& P, u32 old, u32 thr, int rshift, u32 stamp, Tally& t) {
+  for (int64_t b = (int64_t)blockIdx.x * blockDim.x; b < P.V; b += (int64_t)gridDim.x * blockDim.x) {
+    const bool have = b + threadIdx.x < P.V;
+    const int32_t v = have ? (int32_t)(b + threadIdx.x) : 0;
+    bool first = false;
+    for (int w = 0; w < W && have; ++w) {
+      const u64 f = P.far[(size_t)v * W + w];
+      if (!f) continue;
+      const size_t vb = vrow(P.V, w, v, rshift);
+      u64 x = f, keep = 0, near = 0;
+      while (x) {
+        int q[4];
+        u32 d[4];
 #pragma unroll
-  for (int w = 0; w < W; ++w) {
-    if (!far[w]) continue;
-    ++t.nnew;
-    if (SPARSE) {
-      if (atomicOr(&P.next[nxt_at<W>(u, w)], far[w]) == 0) first = true;
-    } else {
-      atomicOr(&P.next[nxt_at<W>(u, w)], far[w]);
+        for (int i = 0; i < 4; ++i) {
+          q[i] = x ? __ffsll((long long)x) - 1 : q[0];  // past the last: the first again
+          x &= x - 1;
+          d[i] = P.vals[vb + q[i]];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (d[i] >= thr) keep |= 1ull << q[i];
+          else if (d[i] >= old) near |= 1ull << q[i];
+          if (d[i] >= thr) t.fmin = min(t.fmin, d[i]);
+        }
+      }
+      if (keep != f) P.far[(size_t)v * W + w] = keep;
+      if (near) {
+        ++t.nnear;
+        ++t.nnew;
+        u64* const n = &P.next[nxt_at<W>(v, w)];
+        if (SPARSE) {
+          if (atomicOr(n, near) == 0) first = true;
+        } else {
+          atomicOr(n, near);
+        }
+      }
     }
+    if (SPARSE) touch(P, first && claim_first<W>(P.mark, v, stamp), v, stamp);
   }
-  return SPARSE && first && claim_first<W>(P.mark, u, stamp);
 }
 
 // Lane k's value of a per-lane word, as a wave-uniform scalar.
@@ -488,8 +491,8 @@ __device__ __forceinline__ u64 lane64(u64 x, int k) {
 
 // Expands up to 64 (vertex, edge range) units with the whole wave, lane = edge:
 // lane k < cnt holds unit k, vertex u with edges [e0, e1) (empty ranges
-// allowed), and `lead` in the part of a vertex that postpones its far pairs and
-// counts its queries.  The units' masks are fetched by their lanes in parallel
+// allowed), and `lead` in the part of a vertex that counts it and its queries.
+// The units' masks are fetched by their lanes in parallel
 // and each unit's are then wave-uniform, in scalar registers; N steps of 64
 // edges are relaxed together, and the columns and weights of the next step, of
 // the next unit too, are on their way while a step is relaxed.
@@ -502,17 +505,13 @@ __device__ __forceinline__ void expand_units(const KP& P, int cnt, int32_t u, in
   constexpr int N = W == 1 ? 4 : W == 2 ? 2 : 1;
   const int lane = lane_id();
   const bool have = lane < cnt && e0 < e1;
-  u64 bm[W], sm[W], far[W];
+  u64 bm[W], sm[W];
   bool any_s = false, any_b = false;
-  if (have) load_masks<W>(P, u, bfs_on, dense_t, thr, rshift, bm, sm, far, any_s, t);
+  if (have) load_masks<W>(P, u, bfs_on, dense_t, bm, sm, any_s);
 #pragma unroll
   for (int w = 0; w < W; ++w) {
-    if (!have) bm[w] = sm[w] = far[w] = 0;
+    if (!have) bm[w] = sm[w] = 0;
     any_b |= bm[w] != 0;
-  }
-  if (thr != INF) {
-    const bool c = have && lead && postpone<W, SPARSE>(P, u, far, stamp, t);
-    if (SPARSE) touch(P, c, u, stamp);
   }
   if (!any_b && !any_s) e1 = e0;
   else if (P.profile) count_edges<W>(t, bm, sm, (u32)(e1 - e0), lead, P.wt != nullptr);
@@ -629,17 +628,13 @@ __device__ __forceinline__ void expand_flat_vertices(const KP& P, const int32_t*
   const u32 e = P.mix_small && gsz >= 8 ? (g + (u32)(lane >> 3) * ng) * 8u + (u32)(lane & 7) : g * gsz + (u32)lane;
   const bool have = (u32)lane < gsz && e < n;
   const int32_t u = have ? list[e] : 0;
-  u64 bm[W], sm[W], far[W];
+  u64 bm[W], sm[W];
   bool any_s = false, any_b = false;
-  if (have) load_masks<W>(P, u, bfs_on, dense_t, thr, rshift, bm, sm, far, any_s, t);
+  if (have) load_masks<W>(P, u, bfs_on, dense_t, bm, sm, any_s);
 #pragma unroll
   for (int w = 0; w < W; ++w) {
-    if (!have) bm[w] = sm[w] = far[w] = 0;
+    if (!have) bm[w] = sm[w] = 0;
     any_b |= bm[w] != 0;
-  }
-  if (thr != INF) {
-    const bool c = have && postpone<W, SPARSE>(P, u, far, stamp, t);
-    if (SPARSE) touch(P, c, u, stamp);
   }
   const bool work = have && (any_b || any_s);
   const int32_t e0 = work ? P.off[u] : 0;
@@ -739,7 +734,7 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, const DenseClaim&
   const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
   const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
   const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
-  u64 sm = have ? (P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) : 0ull;
+  const u64 sm = have ? (P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) : 0ull;
   const bool inrow = lane < R;
   // Lane offset inside a value row; every lane reads a valid address of the
   // (always valid) row whether or not its pair is active, so the loads issue
@@ -754,50 +749,6 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, const DenseClaim&
   for (int ww = 0; ww < W; ++ww) lane_words |= (u32)((P.cfg->val_bits[ww] >> lq) & 1ull) << ww;
   if (!inrow) lane_words = 0;
   const u32 lq4 = (u32)lq * 4u;
-  if (NF) {
-    // Near-far split of the wave's items: lane q reads value q of each
-    // item's source row (8 rows in flight); pairs at or above thr are
-    // postponed (chunk 0 of the vertex keeps them in the next frontier) and
-    // an item left with no near pair scans no edges.
-    const int nit = (int)__popcll(__ballot(have));  // a prefix of the lanes
-    u64 near = sm;
-    for (int i0 = 0; i0 < nit; i0 += 8) {
-      u32 dv[8];
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int it = min(i0 + k, nit - 1);
-        const u32 uk = (u32)__builtin_amdgcn_readlane(u, it);
-        const u32 wk = (u32)__builtin_amdgcn_readlane(w, it);
-        dv[k] = uniform_gptr(P.vals + ((size_t)(wk * (u32)P.V + uk) << rshift))[(unsigned)lq];
-      }
-#pragma unroll
-      for (int k = 0; k < 8; ++k) {
-        const int it = i0 + k;
-        if (it >= nit) break;
-        const u64 smk = ((u64)(u32)__builtin_amdgcn_readlane((int)(u32)(sm >> 32), it) << 32) |
-                        (u32)__builtin_amdgcn_readlane((int)(u32)sm, it);
-        const bool isfar = inrow && ((smk >> lane) & 1ull) && dv[k] >= thr;
-        const u64 fm = __ballot(isfar);
-        if (isfar) t.fmin = min(t.fmin, dv[k]);
-        if (lane == it) near = sm & ~fm;
-        if (fm && __builtin_amdgcn_readlane((int)part, it) == 0) {
-          const int32_t uk = __builtin_amdgcn_readlane(u, it);
-          const int wk = __builtin_amdgcn_readlane(w, it);
-          bool claimed = false;
-          if (lane == 0) {
-            ++t.nnew;
-            if (SPARSE) {
-              if (atomicOr(&P.next[nxt_at<W>(uk, wk)], fm) == 0) claimed = claim_first<W>(P.mark, uk, stamp);
-            } else {
-              atomicOr(&P.next[nxt_at<W>(uk, wk)], fm);
-            }
-          }
-          if (SPARSE) touch(P, claimed, uk, stamp);
-        }
-      }
-    }
-    sm = near;
-  }
   const u32 d = sm ? (u32)(e1 - e0) : 0u;
   if (have) {
     ++t.ditems;
@@ -880,19 +831,28 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, const DenseClaim&
         vr_c[k] = vr[k];
       }
       if (k0 + U < cnt) issue(k0 + U);
-      u32 mine_lo = 0, mine_hi = 0;
+      u32 mine_lo = 0, mine_hi = 0, far_lo = 0, far_hi = 0;
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        const u64 m = mk[k];
-        if (m == 0) continue;
-        if ((m >> lane) & 1ull) {
+        const u64 mi = mk[k];
+        if (mi == 0) continue;
+        if ((mi >> lane) & 1ull) {
           __hip_atomic_fetch_min((gu32*)vr_c[k] + (unsigned)lq, c_c[k], __ATOMIC_RELAXED,
                                  __HIP_MEMORY_SCOPE_AGENT);
           note_improved(t, c_c[k], thr);
           ++t.imp;
         }
+        // Values at or above the threshold go to the far set, the others to
+        // the next frontier.
+        const u64 mf = NF ? __ballot(c_c[k] >= thr) & mi : 0ull;
+        const u64 m = mi & ~mf;
+        const bool own = lane == k0 + k;
+        if (NF && mf) {
+          far_lo = own ? (u32)mf : far_lo;
+          far_hi = own ? (u32)(mf >> 32) : far_hi;
+        }
+        if (m == 0) continue;
         if (!SPARSE) {
-          const bool own = lane == k0 + k;
           mine_lo = own ? (u32)m : mine_lo;
           mine_hi = own ? (u32)(m >> 32) : mine_hi;
         } else {
@@ -912,6 +872,8 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, const DenseClaim&
         ++t.nnew;
         atomicOr(&P.next[nxt_at<W>(myv, myword)], ((u64)mine_hi << 32) | mine_lo);
       }
+      if (NF && (far_lo | far_hi))
+        atomicOr(&P.far[(size_t)myv * W + (size_t)myword], ((u64)far_hi << 32) | far_lo);
     }
   }
 }
@@ -1333,8 +1295,7 @@ __device__ __forceinline__ u32 wave_fetch(u32* ctr, u32 n) {
 // A list that the first claims cover costs no atomic at all.  (Every wave used
 // to find each shard exhausted by an atomic of its own: 16 per wave and
 // launch, 16 us at 1024 waves and 93 us at 8192 with one unit of work.)
-// The claims get shorter towards a shard's end.  Claims never cross a shard's
-// end.  All state is wave-uniform.  `turn` (0 to 3) rotates which waves come
+// Claims never cross a shard's end.  All state is wave-uniform.  `turn` (0 to 3) rotates which waves come
 // first, so that the short lists of consecutive phases go to different waves.
 struct ShardFetch {
   u32 n, chunk, wpb;
@@ -1418,6 +1379,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   const int rshift = P.cfg->rshift, dense_t = C->sssp_pull ? 0 : P.cfg->dense_t;
   const u32 nw = gridDim.x * (BS / 64);
   const u32* const done = C->use_done ? P.done : nullptr;
+  if (C->raised) raise_far<W, SPARSE>(P, C->thr_old, thr, rshift, stamp, t);
   const int lane = lane_id();
   u32 lo, hi;
   // Phase L.  A chunk is two units, or up to 32 of 128 edges while that leaves
@@ -2191,8 +2153,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     C->done_verts = dv;
     C->use_done = P.done && dv > (u32)P.V / 16u ? 1u : 0u;
     const u32 cur_pull = C->bfs_pull, cur_spull = C->sssp_pull;
-    const u32 dense = fall >= cfg->dense_fedges_thr ? 1u : 0u;
-    C->dense_mode = dense;
+    u32 dense = fall >= cfg->dense_fedges_thr ? 1u : 0u;
     u64 consumed[MAXW];
     for (int w = 0; w < MAXW; ++w) {
       consumed[w] = C->last_union[w];
@@ -2223,15 +2184,27 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     }
     C->sssp_pull = spull;
     // Near-far: when no SSSP pair below the threshold is left, move it to
-    // the smallest pending value plus delta (skipping empty buckets).
+    // the smallest value of the far set plus delta (skipping empty buckets);
+    // the next advance takes the far set's pairs below it up (raise_far).
+    u32 raised = 0;
     if (cfg->delta != 0) {
-      const u32 fm = s_far_min;
-      if (s_near_new == 0 && fm != INF) {
+      u32 fm = min(C->far_min, s_far_min);
+      // (An empty frontier can follow lowered pairs: on vertices without edges.)
+      if ((s_near_new == 0 || total == 0) && fm != INF) {
         const u64 nt = (u64)fm + (u64)cfg->delta;
+        C->thr_old = C->thr;
         C->thr = nt >= (u64)INF ? INF : (u32)nt;
         ++C->bumps;
+        raised = 1;
+        fm = INF;  // taken again over the pairs that stay
+        // The raise looks at every vertex, and the filter may as well: claiming
+        // and listing what it takes up took 780 us of a 2048^2 grid's raise.
+        dense = 1;
       }
+      C->far_min = fm;
+      C->raised = raised;
     }
+    C->dense_mode = dense;
     // Launch timing and the iteration record: the advance of this iteration
     // ran iff iter != seeding.
     if (iter != 0xFFFFFFFFu) {
@@ -2277,7 +2250,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     C->den_t0 = ~0ull;
     const u32 next_iter = iter + 1u;
     C->iter = next_iter;
-    if (total == 0 || (C->max_iter != 0 && next_iter >= C->max_iter)) {
+    if ((total == 0 && !raised) || (C->max_iter != 0 && next_iter >= C->max_iter)) {
       C->finished = 1;
     } else {
       if (pull || spull) ++C->pull_iters;
@@ -2285,6 +2258,17 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       if (dense) ++C->dense_iters;
     }
   }
+}
+
+// OR of every vertex's far words into ctl->far_union (a serving session asks
+// whether a query still has far pairs).
+__global__ __launch_bounds__(BLOCK) void k_far_union(KP P, int W) {
+  const int64_t n = (int64_t)P.V * W, stride = (int64_t)gridDim.x * BLOCK;
+  // The stride is a multiple of every W, so a thread stays on one word.
+  u64 x = 0;
+  const int64_t i0 = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
+  for (int64_t i = i0; i < n; i += stride) x |= P.far[i];
+  if (x) atomicOr(&P.ctl->far_union[i0 % W], x);
 }
 
 // ------------------------------------------------------------------ utilities
@@ -2826,6 +2810,16 @@ void dispatch_seed(cgp_engine* en, int W, const KP& P, const int32_t* src, int n
   }
 }
 
+void far_union(cgp_engine* en, int W) {
+  const KP P = en->kp(W);
+  fill_u32(en->s, en->d_ctl->far_union, MAXW * 2, 0u, en->cus);
+  hipLaunchKernelGGL(k_far_union, dim3(en->cus * 4), dim3(BLOCK), 0, en->s, P, W);
+  HIP_CHECK(hipGetLastError());
+  HIP_CHECK(hipMemcpyAsync(en->h_ctl->far_union, en->d_ctl->far_union, sizeof(en->h_ctl->far_union),
+                           hipMemcpyDeviceToHost, en->s));
+  HIP_CHECK(hipStreamSynchronize(en->s));
+}
+
 u32 narrow_mask(const Cfg& cfg, int W) {
   // Words whose SSSP slots all sit in lanes 0..15 can relax four edges per
   // lane-per-query step (phase N).  Measured on RMAT-22: worth it when every
@@ -3264,7 +3258,7 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
     }
     // Visited + next records (2W words per vertex) start clear; the layout
     // depends on W, so the whole region is cleared for every pass.
-    fill_u32(en->s, en->visited.p, (size_t)V * W * 4 + (no_alloc ? 0 : en->done_bytes() / 4), 0u, en->cus);
+    fill_u32(en->s, en->visited.p, en->record_bytes(W) / 4, 0u, en->cus);
     en->next_dirty = false;
     dispatch_seed(en, W, P, (const int32_t*)en->slot_src.p, W * 64);
     en->tick(CAT_INIT, false);
@@ -3396,7 +3390,7 @@ struct StaticLayout {
       wcc_rows, wcc_probe, slot_src, qmap, total;
 };
 
-StaticLayout static_layout(const cgp_graph* g, int Wm, int Rm, int nw) {
+StaticLayout static_layout(const cgp_graph* g, size_t record_bytes, int Wm, int Rm, int nw) {
   const size_t V = (size_t)g->V, E = (size_t)g->E;
   StaticLayout L{};
   size_t at = 0;
@@ -3405,12 +3399,11 @@ StaticLayout static_layout(const cgp_graph* g, int Wm, int Rm, int nw) {
     at += (bytes + 255) & ~(size_t)255;
     return r;
   };
-  L.visited = take(V * Wm * 16);
+  L.visited = take(record_bytes);
   L.front = take(V * Wm * 8);
-  for (int k = 0; k < 2; ++k) {
-    L.dense[k] = take((size_t)Wm * (V + E / DCHUNK + 1) * 8);
-    L.dense_n[k] = take((size_t)Wm * (V + E / DCHUNK + 1) * 8);
-  }
+  // A batch pass routes its lane-per-query items to one of the two lists for
+  // its whole length, so they share their memory here.
+  for (int k = 0; k < 2; ++k) L.dense[k] = L.dense_n[k] = take((size_t)Wm * (V + E / DCHUNK + 1) * 8);
   L.mark = take(V * 4 + 4);
   L.touched = take(V * 4 + 4);
   for (int k = 0; k < 2; ++k) {
@@ -3451,7 +3444,7 @@ void engine_run_batch_static(cgp_engine* en, const cgp_query* queries, int32_t n
     while (Rm < std::min(64, first)) Rm <<= 1;
     if (first > 64) Rm = 64;
   }
-  const StaticLayout L = static_layout(g, Wm, Rm, nw);
+  const StaticLayout L = static_layout(g, en->record_bytes(Wm), Wm, Rm, nw);
   if (L.total > (size_t)CGP_STATIC_SCRATCH_BYTES)
     fail(CGP_ECAPACITY, "cgp_run_batch_static: this batch needs " + std::to_string(L.total) +
                             " bytes of device scratch; the static array holds " +

@@ -125,7 +125,7 @@ struct cgp_engine {
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   int cus = 1;
   int wcap = 0;            // words allocated in visited/next/front/dense
-  cgpi::DevBuf visited, front, mark, vals, touched, small[2], medium[2], large[2], dense[2], dense_n[2];  // visited: visited + next records
+  cgpi::DevBuf visited, front, mark, vals, touched, small[2], medium[2], large[2], dense[2], dense_n[2];  // visited: see record_bytes
   cgpi::DevBuf iters;  // per-iteration record ring (ITER_RING entries)
   std::vector<cgpk::IterRec> report;  // records of the last batch run, all passes
   // The rest of the last batch run's report: its queries, each query's slot
@@ -193,7 +193,7 @@ struct cgp_engine {
 
   // Kernel parameters; keep_done: of a batch pass of W words, whose done bits
   // lie behind its records.
-  KP kp(int W = 0, bool keep_done = false) const {
+  KP kp(int W, bool keep_done = false) const {
     KP P{};
     P.V = g->V;
     P.E = g->E;
@@ -226,7 +226,9 @@ struct cgp_engine {
     P.cfg = d_cfg;
     P.iters = (cgpk::IterRec*)iters.p;
     P.fstat = d_fstat;
-    P.done = keep_done ? (u32*)((char*)visited.p + (size_t)g->V * W * 16) : nullptr;
+    char* const behind = (char*)visited.p + (size_t)g->V * W * 16;  // records of a pass of W words
+    P.done = keep_done ? (u32*)behind : nullptr;
+    P.far = opts.sssp_delta != 0 ? (u64*)(behind + done_bytes()) : nullptr;
     P.bin_small = opts.bin_small;
     P.bin_large = opts.bin_large;
     // Serving seeds queries into running iterations, where a full scan must
@@ -273,17 +275,21 @@ struct cgp_engine {
     return (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cus * 4));
   }
 
-  // Bytes of the per-vertex done bits, kept behind the visited + next records
-  // of the running pass's W and cleared with them.
+  // Bytes of the per-vertex done bits.
   size_t done_bytes() const { return ((size_t)g->V + 127) / 128 * 16; }
+  // Bytes of a pass of W words that start at zero: visited + next records, done
+  // bits, and with postponing the far words.
+  size_t record_bytes(int W) const {
+    const size_t V = (size_t)g->V;
+    return V * W * 16 + done_bytes() + (opts.sssp_delta != 0 ? V * W * 8 : 0);
+  }
 
   void ensure_words(int W) {
     const size_t V = (size_t)g->V, E = (size_t)g->E;
     bool moved = false;
+    moved |= visited.ensure(record_bytes(W));
     if (W > wcap) {
-      moved |= visited.ensure(V * W * 16 + done_bytes());  // visited + next records, then the done bits
       moved |= front.ensure(V * W * 8);
-      HIP_CHECK(hipMemsetAsync(visited.p, 0, V * W * 16, s));
       for (int k = 0; k < 2; ++k) {
         moved |= dense[k].ensure((size_t)W * (V + E / DCHUNK + 1) * 8);
         moved |= dense_n[k].ensure((size_t)W * (V + E / DCHUNK + 1) * 8);
@@ -308,6 +314,7 @@ struct cgp_engine {
     Ctl& c = *h_ctl;
     std::memset((void*)&c, 0, sizeof(Ctl));
     c.adv_t0 = c.den_t0 = c.flt_t0 = ~0ull;
+    c.far_min = INF;
     for (cgpk::Stripe& x : c.stripe) x.far_min = INF;
     return c;
   }
@@ -361,6 +368,9 @@ void dispatch_iteration(cgp_engine* en, int W, const KP& P);
 void dispatch_seed_only(cgp_engine* en, int W, const KP& P, const int32_t* d_slot_src, int nslots);
 void dispatch_seed(cgp_engine* en, int W, const KP& P, const int32_t* d_slot_src, int nslots);
 void fill_u32(hipStream_t s, void* p, size_t n, u32 v, int cus);
+// OR of the far words of a serving session of W words into h_ctl->far_union
+// (waits for the engine's stream).
+void far_union(cgp_engine* en, int W);
 // Narrow-word mask of a slot configuration (all SSSP words narrow, else 0).
 u32 narrow_mask(const Cfg& cfg, int W);
 // One batched run (all passes, WCC, output transpose); stats may be null.

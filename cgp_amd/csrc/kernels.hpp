@@ -119,7 +119,7 @@ struct alignas(256) Ctr {
 // and lane-per-query launch), and the near-far state of its SSSP improvements.
 struct alignas(256) Stripe {
   u64 adv_t1, den_t1;
-  u32 far_min;   // min value of the pairs postponed or improved to >= thr this iteration
+  u32 far_min;   // min value of the pairs put or kept in the far set this iteration
   u32 near_new;  // nonzero when this iteration produced an SSSP pair below thr
 };
 
@@ -135,8 +135,11 @@ struct Ctl {
   u32 pull_iters;
   u32 dense_mode;   // 1: advance uses fire-and-forget atomics, filter scans all vertices
   u32 dense_iters;
-  u32 thr;          // SSSP near-far threshold: frontier pairs with value >= thr are postponed
-                    // (INF: every pair expands, Bellman-Ford frontier)
+  u32 thr;          // SSSP near-far threshold: pairs lowered to a value >= thr wait in the far
+                    // set (INF: every pair expands, Bellman-Ford frontier)
+  u32 thr_old;      // ... before its last raise
+  u32 raised;       // this iteration's advance takes the far set's pairs below thr up
+  u32 far_min;      // at most the smallest value in the far set (INF: it is empty)
   u32 bumps;        // threshold raises so far
   // The running iteration as its filter sees it, written by the kernel before
   // it (advance or seeding): the filter's last workgroup moves iter and
@@ -146,6 +149,7 @@ struct Ctl {
   u32 done_verts;   // vertices that every BFS query of the pass has visited
   u32 use_done;     // the push launch looks a target up in KP::done before its record
   u64 last_union[MAXW];       // OR of the frontier words the last filter produced
+  alignas(16) u64 far_union[MAXW];  // OR of the far words, when asked for (k_far_union)
   u64 prof[NPROF];            // work counters (profile mode)
   // Device-clock launch timing (wall_clock64 ticks): start of the running
   // advance / filter (its first workgroup), and the sums over the launches of
@@ -224,6 +228,7 @@ struct KP {
   // Bit v: every BFS query of the pass has visited v (batch runs; null: not
   // kept).  512 KiB for 2^22 vertices, so it stays in every XCD's L2.
   u32* done;
+  u64* far;  // far set, bit q of word w of vertex v at v*W+w (postponing on; else null)
   int32_t bin_small;
   int32_t bin_large;
   // Vertices a full compaction scan visits: [0, scan_v).  On a symmetric

@@ -247,7 +247,7 @@ void admit(cgp_engine* en, ServeState* ss) {
     HIP_CHECK(hipMemsetAsync(&en->d_ctl->finished, 0, 4, en->s));
     ss->need_restart = false;
   }
-  dispatch_seed_only(en, ss->W, en->kp(), (const int32_t*)ss->d_src.p, ss->nslots);
+  dispatch_seed_only(en, ss->W, en->kp(ss->W), (const int32_t*)ss->d_src.p, ss->nslots);
 }
 
 cgpi::DevBuf* take_staging(ServeState* ss, size_t bytes) {
@@ -438,7 +438,7 @@ cgp_status cgp_serve_start(cgp_engine* en, const cgp_serve_opts* so) {
     ss->d_src.ensure((size_t)ss->nslots * 4);
     // Clean slot state: every value row INF, no visited bits, no pending next bits.
     fill_u32(en->s, en->vals.p, vals_elems, INF, en->cus);
-    fill_u32(en->s, en->visited.p, (size_t)V * W * 4, 0u, en->cus);  // visited + next records
+    fill_u32(en->s, en->visited.p, en->record_bytes(W) / 4, 0u, en->cus);  // records, far words
     en->next_dirty = false;
     Cfg& cfg = *en->h_cfg;
     std::memset(&cfg, 0, sizeof(Cfg));
@@ -496,7 +496,7 @@ cgp_status cgp_serve_step(cgp_engine* en, int32_t max_iterations, cgp_completion
         break;
       }
       if (max_iterations > 0 && ran >= max_iterations) break;
-      dispatch_iteration(en, W, en->kp());
+      dispatch_iteration(en, W, en->kp(W));
       HIP_CHECK(hipMemcpyAsync(en->h_ctl, en->d_ctl, CTL_HOST_BYTES, hipMemcpyDeviceToHost, en->s));
       HIP_CHECK(hipStreamSynchronize(en->s));
       ++ran;
@@ -506,9 +506,23 @@ cgp_status cgp_serve_step(cgp_engine* en, int32_t max_iterations, cgp_completion
       // once the frontier has no work left (`finished`: its remaining bits sit
       // on vertices without out-edges, and the kernels stop until restarted).
       conv.clear();
+      // With an empty far set nobody has far pairs (just before a raise its
+      // minimum is not known).
+      bool far_known = hc.far_min == INF && !hc.raised;
+      if (far_known) std::memset(en->h_ctl->far_union, 0, sizeof(hc.far_union));
       for (int k = 0; k < ss->nslots; ++k) {
         if (!ss->slots[k].busy || ss->iter < ss->slots[k].start) continue;
-        if (hc.finished || !((hc.last_union[k >> 6] >> (k & 63)) & 1ull)) conv.push_back(k);
+        const int w = k >> 6;
+        const u64 bit = 1ull << (k & 63);
+        if (!hc.finished && (hc.last_union[w] & bit)) continue;
+        // An SSSP query out of the frontier may still have pairs waiting for
+        // the near-far threshold.
+        if (!hc.finished && (en->h_cfg->val_bits[w] & bit)) {
+          if (!far_known) far_union(en, W);
+          far_known = true;
+          if (hc.far_union[w] & bit) continue;
+        }
+        conv.push_back(k);
       }
       if (hc.finished) ss->need_restart = true;
       if (!conv.empty()) retire(en, ss, conv);

@@ -136,3 +136,48 @@ def test_wcc_directed(gpu, V):
     got = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, dst.astype(np.int32))).wcc(2)
     exp = O.expected(O.G(off, dst.astype(np.int32), None), WCC, 0)
     assert np.array_equal(got[0], exp) and np.array_equal(got[1], exp)
+
+
+# Near-far: pairs at or above the threshold wait in the far set.  Small and
+# large steps, one to four mask words, BFS beside it, vertices without
+# out-edges (a frontier that is empty while pairs wait), both frontier modes.
+@pytest.mark.parametrize("delta", [1, 7, 60, 1000])
+@pytest.mark.parametrize("n", [1, 5, 70, 200])
+@pytest.mark.parametrize("opts", [dict(), dict(frontier_dense_div=1, dense_threshold=1),
+                                  dict(frontier_dense_div=1 << 20, dense_threshold=1), dict(dense_threshold=65)],
+                         ids=["default", "sparse_rows", "dense_rows", "edges"])
+def test_near_far(gpu, delta, n, opts):
+    V = 1501
+    off, idx, wt = ring_graph(V, hub_degree=200, seed=n, chords=1)
+    kinds = [SSSP] * n + [BFS] * (n // 2)
+    check(off, idx, wt, kinds, [(i * 131) % V for i in range(len(kinds))], runs=2, sssp_delta=delta, **opts)
+
+
+@pytest.mark.parametrize("delta", [1, 30])
+def test_near_far_sinks(gpu, delta):
+    # 0 -> 1..9 (sinks) at weight i, 0 -> 10 -> 11 -> ... at weight 90 each: when
+    # only sinks are near the frontier has no edges and the path still waits.
+    src = np.concatenate([np.zeros(10, np.int64), np.arange(10, 40)])
+    dst = np.concatenate([np.arange(1, 11), np.arange(11, 41)])
+    wt = np.concatenate([np.arange(1, 10), np.full(31, 90)]).astype(np.uint32)
+    off = np.zeros(42, np.int64)
+    np.add.at(off, src + 1, 1)
+    check(np.cumsum(off).astype(np.int32), dst.astype(np.int32), wt, [SSSP, SSSP, BFS], [0, 10, 0], sssp_delta=delta)
+
+
+@pytest.mark.parametrize("slots", [1, 4, 70])
+def test_near_far_serving(gpu, slots):
+    h = cgp_amd.HostCSR.grid(41, 37, p_extra=0.01, seed=3, wmin=1, wmax=1000)
+    og = O.G.of(h)
+    en = cgp_amd.Engine(cgp_amd.Graph.from_host(h), sssp_delta=300)
+    en.serve_start(max_slots=slots)
+    src = h.sample_sources(90, seed=2)
+    for i, s in enumerate(src):
+        en.serve_submit(SSSP if i % 3 else BFS, s, i, 0.0)
+    left = set(range(len(src)))
+    while left:
+        for c in en.serve_step(max_iterations=3 if slots == 4 else 0):
+            exp = O.expected(og, c["kind"], c["source"])
+            assert np.array_equal(c["result"], exp), (c["ticket"], c["kind"], c["source"])
+            left.remove(c["ticket"])
+    en.serve_stop()
