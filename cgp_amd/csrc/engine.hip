@@ -1289,7 +1289,8 @@ __device__ __forceinline__ u32 wave_fetch(u32* ctr, u32 n) {
 // Wave-level claims of the units [0, n), in NSHARD contiguous shards: shard s
 // covers [n*s/NSHARD, n*(s+1)/NSHARD) and belongs to the workgroups with
 // blockIdx % NSHARD == s, one XCD.  Each of a shard's waves owns its first
-// units without any atomic (`chunk` units by its rank); what is left is handed
+// units without any atomic (`chunk` units by its rank, and again after all of
+// the shard's waves if that covers the shard); what is left is handed
 // out through the shard's cursor, and a wave whose shard is exhausted looks at
 // all cursors with one load before it claims from another (cursors only grow).
 // A list that the first claims cover costs no atomic at all.  (Every wave used
@@ -1300,15 +1301,17 @@ __device__ __forceinline__ u32 wave_fetch(u32* ctr, u32 n) {
 struct ShardFetch {
   u32 n, chunk, wpb;
   int s;
-  bool first, strided;
-  u32 rank;  // first claim: this wave's place in its shard
+  bool strided;
+  u32 own;   // start of this wave's next own claim in its shard
+  u32 rank;
   __device__ __forceinline__ ShardFetch(u32 n_, u32 chunk_, u32 turn, bool strided_ = false)
-      : n(n_), chunk(chunk_), first(true), strided(strided_) {
+      : n(n_), chunk(chunk_), strided(strided_) {
     wpb = blockDim.x / 64u;
     s = (int)(blockIdx.x % NSHARD);
     const u32 nw = waves(s);
     rank = (blockIdx.x / NSHARD) * wpb + (u32)uniform32((int32_t)(threadIdx.x >> 6)) + turn * (nw / 4u);
     if (rank >= nw) rank -= nw;
+    own = rank * chunk;
   }
   __device__ __forceinline__ u32 waves(int sh) const { return (gridDim.x - (u32)sh + NSHARD - 1) / NSHARD * wpb; }
   __device__ __forceinline__ u32 begin(int sh) const { return (u32)(((u64)n * (u32)sh) / NSHARD); }
@@ -1317,32 +1320,37 @@ struct ShardFetch {
   }
   // Unit i of the shard the last claim was from.
   __device__ __forceinline__ u32 unit(u32 i) const { return strided ? i * NSHARD + (u32)s : begin(s) + i; }
-  // Units of a shard beyond its waves' first claims.
-  __device__ __forceinline__ u32 shared(int sh) const {
-    const u32 all = size(sh), own = waves(sh) * chunk;
-    return all > own ? all - own : 0u;
+  // Units of a shard that its waves own: all of them when that is at most
+  // two claims per wave, else one claim each.  (A 1001x777 grid with 5 SSSP at
+  // 1 / 2 / 4 / 8 claims: 5.31 / 5.26 / 5.13 / 5.12 ms, RMAT-20 64 SSSP 6.48 /
+  // 6.36 / 6.38 / 6.85, 2048^2 grid 128 SSSP 99.1 / 98.8 / 101.1 / 100.5.)
+  __device__ __forceinline__ u32 owned(int sh) const {
+    const u32 all = size(sh), round = waves(sh) * chunk;
+    return all <= 2u * round ? all : round;
   }
   __device__ __forceinline__ bool next(Ctr* cur, u32& lo, u32& hi) {
-    if (first) {
-      first = false;
-      lo = rank * chunk;
-      hi = min(size(s), lo + chunk);
-      if (lo < hi) return true;
+    {
+      const u32 mine = owned(s);  // (a wave that claims from another shard has own past its end)
+      if (own < mine) {
+        lo = own;
+        hi = min(mine, lo + chunk);
+        own += waves(s) * chunk;
+        return true;
+      }
+      own = ~0u;
     }
     while (true) {
-      const u32 sz = shared(s);
+      const u32 base = owned(s), sz = size(s) - base;
       if (sz) {
-        // Towards the end a claim is one unit: the last claims bound the
-        // launch's end.
         const u32 i = wave_fetch(&cur[s].v, chunk);
         if (i < sz) {
-          lo = waves(s) * chunk + i;
+          lo = base + i;
           hi = min(size(s), lo + chunk);
           return true;
         }
       }
       const int k = lane_id() % NSHARD;
-      const u32 szk = shared(k);
+      const u32 szk = size(k) - owned(k);
       const bool more =
           szk && __hip_atomic_load(&cur[k].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < szk;
       const u32 m = (u32)__ballot(more) & ((1u << NSHARD) - 1u);
