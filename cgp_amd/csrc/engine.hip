@@ -2334,7 +2334,7 @@ struct OutMasks {
 constexpr int OUT_VT = 64;
 __global__ __launch_bounds__(BLOCK) void k_output(const u32* vals, const u64* visited, const int32_t* inv,
                                                   int32_t V, int W, int rshift, const int32_t* qmap, OutMasks m,
-                                                  u32* out, int vec) {
+                                                  u32* out, int vec, int skip_bfs) {
   __shared__ u32 tile[64][OUT_VT + 1];
   __shared__ u64 s_vis[OUT_VT];
   __shared__ int32_t s_u[OUT_VT];
@@ -2345,6 +2345,7 @@ __global__ __launch_bounds__(BLOCK) void k_output(const u32* vals, const u64* vi
   const int nv = min(OUT_VT, V - v0);
   const int np = m.n_planes;
   const u64 bm = m.bfs[w];
+  if (skip_bfs && !m.val[w]) return;  // k_output_bfs writes this word's rows
   const u64 rd = np ? m.val[w] : (m.val[w] | bm);  // slots whose value rows are read
   if ((int)threadIdx.x < OUT_VT) {
     const int j = (int)threadIdx.x;
@@ -2434,6 +2435,72 @@ __global__ __launch_bounds__(BLOCK) void k_output(const u32* vals, const u64* vi
       const int q = t / OUT_VT, j = t % OUT_VT;
       const int32_t dst = qmap[w * 64 + q];
       if (dst >= 0 && j < nv) out[(size_t)dst * V + v0 + j] = tile[q][j];
+    }
+  }
+}
+
+// Output rows of the words whose slots are all BFS, from the visited words and
+// depth planes alone (batch runs; V % 4 == 0 and a 16-byte aligned output,
+// checked by the launcher).  A thread holds four consecutive vertices' visited
+// word and up to NP planes in registers and writes one 16-byte store per query,
+// so a wave writes 1 KiB of a row at a time and nothing goes through LDS; the
+// words of a vertex follow each other in one thread, so its record's line is
+// read once.  Part blockIdx.y of gridDim.y takes its share of each word's slots
+// (small graphs have too few vertices to fill the chip).  160 BFS on RMAT-22
+// (2.7 GB of rows): 1.01 ms through the tile, whose stores are 256-byte pieces
+// of 64 rows, 0.84 ms here, 0.78 with
+// non-temporal stores.
+typedef u32 u32x4 __attribute__((ext_vector_type(4)));
+template <int NP>
+__global__ __launch_bounds__(BLOCK) void k_output_bfs(const u64* visited, const int32_t* inv, int32_t V, int W,
+                                                      const int32_t* qmap, OutMasks m, u32* out) {
+  const int32_t v0 = (int32_t)(((int64_t)blockIdx.x * BLOCK + threadIdx.x) * 4);
+  if (v0 >= V) return;
+  const int share = 64 / (int)gridDim.y;  // gridDim.y divides 64
+  const u64 slots = (share == 64 ? ~0ull : (1ull << share) - 1ull) << (share * (int)blockIdx.y);
+  int32_t u[4] = {v0, v0 + 1, v0 + 2, v0 + 3};
+  if (inv) {
+    const int4 x = *(const int4*)(inv + v0);
+    u[0] = x.x;
+    u[1] = x.y;
+    u[2] = x.z;
+    u[3] = x.w;
+  }
+  for (int w = 0; w < W; ++w) {
+    const u64 bm = m.bfs[w] & slots;
+    if (!bm || m.val[w]) continue;  // mixed words are the tile kernel's
+    u64 vis[4], pl[4][NP];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const size_t wv = (size_t)w * (size_t)V + (size_t)u[i];
+      vis[i] = visited[(size_t)u[i] * (2 * W) + w];
+#pragma unroll
+      for (int b = 0; b < NP; ++b)
+        pl[i][b] = b < 4 ? m.plane4[(wv << 2) + b] : b < m.n_planes ? m.plane[b][wv] : 0ull;
+    }
+    // Lower, then upper 32 slots, so that a slot is a bit of 32-bit registers.
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      u32 hv[4], hp[4][NP];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        hv[i] = (u32)(vis[i] >> (32 * half));
+#pragma unroll
+        for (int b = 0; b < NP; ++b) hp[i][b] = (u32)(pl[i][b] >> (32 * half));
+      }
+      for (u32 left = (u32)(bm >> (32 * half)); left; left &= left - 1) {
+        const int q = __builtin_ctz(left);
+        u32x4 d;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          u32 x = 0;
+#pragma unroll
+          for (int b = 0; b < NP; ++b) x |= ((hp[i][b] >> q) & 1u) << b;
+          d[i] = (hv[i] >> q) & 1u ? x : INF;
+        }
+        u32* const row = out + (size_t)qmap[w * 64 + half * 32 + q] * (size_t)V;
+        __builtin_nontemporal_store(d, (u32x4*)(row + v0));  // nothing reads it here again
+      }
     }
   }
 }
@@ -3283,10 +3350,28 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
       om.n_planes = cfg.depth_planes ? en->plane_count : 0;
       om.plane4 = (const u64*)en->plane4.p;
       for (int b = 4; b < om.n_planes; ++b) om.plane[b] = (const u64*)en->plane[b].p;
+      // Words of BFS slots only, depths below 256, rows that 16-byte stores
+      // reach: from the planes alone.  The other words go through the tile.
+      bool bfs_word = false, tile_word = false;
+      for (int w = 0; w < Wused; ++w) (om.val[w] ? tile_word : bfs_word) = true;
+      const bool direct = bfs_word && om.n_planes >= 4 && om.n_planes <= 8 && (V & 3) == 0 && ((uintptr_t)dout & 15) == 0;
+      if (direct) {
+        const unsigned gx = (unsigned)((V / 4 + BLOCK - 1) / BLOCK);
+        unsigned parts = 1;
+        while (parts < 8 && gx * parts * 2 <= (unsigned)en->cus * 2) parts *= 2;
+        const dim3 grid(gx, parts);
+        if (om.n_planes == 4)
+          hipLaunchKernelGGL((k_output_bfs<4>), grid, dim3(BLOCK), 0, en->s, (const u64*)en->visited.p,
+                             (const int32_t*)g->inv, V, W, (const int32_t*)en->qmap.p, om, dout);
+        else
+          hipLaunchKernelGGL((k_output_bfs<8>), grid, dim3(BLOCK), 0, en->s, (const u64*)en->visited.p,
+                             (const int32_t*)g->inv, V, W, (const int32_t*)en->qmap.p, om, dout);
+      }
+      if (!direct || tile_word)
       hipLaunchKernelGGL(k_output, dim3((V + OUT_VT - 1) / OUT_VT, Wused), dim3(BLOCK),
                          (size_t)om.n_planes * OUT_VT * sizeof(u64), en->s, (const u32*)en->vals.p,
                          (const u64*)en->visited.p, (const int32_t*)g->inv, V, W, rshift,
-                         (const int32_t*)en->qmap.p, om, dout, vec);
+                         (const int32_t*)en->qmap.p, om, dout, vec, direct ? 1 : 0);
       HIP_CHECK(hipGetLastError());
       en->tick(CAT_OUT, false);
     };

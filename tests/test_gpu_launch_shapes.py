@@ -181,3 +181,25 @@ def test_near_far_serving(gpu, slots):
             assert np.array_equal(c["result"], exp), (c["ticket"], c["kind"], c["source"])
             left.remove(c["ticket"])
     en.serve_stop()
+
+
+# Output of words that hold only BFS slots: straight from the depth planes while
+# depths stay below 256 and V % 4 == 0 (a ring of V vertices has depths up to
+# V / 2), through the value tile otherwise; 70 SSSP leave the second word mixed.
+@pytest.mark.parametrize("V", [4, 28, 30, 400, 402, 511, 512, 600, 1028])
+@pytest.mark.parametrize("n_sssp", [0, 3, 70])
+@pytest.mark.parametrize("renumber", [False, True])
+def test_bfs_output(gpu, V, n_sssp, renumber):
+    off, idx, wt = ring_graph(V, chords=0 if V > 4 else 3)
+    kinds = [BFS] * 150 + [SSSP] * n_sssp
+    src = [(i * 7) % V for i in range(len(kinds))]
+    en = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, idx, wt, renumber=renumber))
+    og = O.G(off, idx, wt)
+    exp = np.stack([O.expected(og, k, s) for k, s in zip(kinds, src)])
+    assert np.array_equal(en.run_batch(kinds, src)[0], exp)
+    # Device outputs at every alignment of a row start.
+    buf = cgp_amd.DeviceBuffer((len(kinds) * V + 4) * 4)
+    for shift in range(4):
+        en.run_batch(kinds, src, out=buf.view(shift * 4, len(kinds) * V * 4))
+        got = buf.to_host()[shift:shift + len(kinds) * V].reshape(len(kinds), V)
+        assert np.array_equal(got, exp), shift
