@@ -3954,8 +3954,11 @@ cgp_engine_opts resolve_opts(const cgp_graph* g, const cgp_engine_opts* opts, co
     // query and for 512); small-world graphs settle in few Bellman-Ford
     // iterations and skip it.
     const double deg = g->V > 0 ? (double)g->E / (double)g->V : 0.0;
-    o.sssp_delta =
-        (g->weighted && deg <= 8.0 && g->mean_weight > 1.0) ? (int32_t)std::lround(20.0 * g->mean_weight) : 0;
+    // So are directed power-law graphs, which are as sparse (300007 vertices,
+    // 7 edges each, 11 SSSP: 2.05 ms without postponing, 2.34 with it).
+    o.sssp_delta = (g->weighted && deg <= 8.0 && g->mean_weight > 1.0 && !g->skewed)
+                       ? (int32_t)std::lround(20.0 * g->mean_weight)
+                       : 0;
   }
   // A zero threshold keeps the base's (possibly tuned) value while the
   // postponing regime it was chosen for is unchanged.

@@ -84,7 +84,7 @@ typedef struct {
                                   bit 1: device work counters -> advance_bytes */
   uint64_t hbm_budget_bytes;   /* serving: cap on per-query value memory; 0 = 64 GiB */
   int32_t dense_threshold;     /* active SSSP queries in a mask word at which the word is relaxed
-                                  lane-per-query (one wave per edge row); 0 = automatic: 6 when
+                                  lane-per-query (one wave per edge row); 0 = automatic: 5 when
                                   sssp_delta resolves to 0 (postponing off), else 8 */
   int32_t frontier_dense_div;  /* dense frontier mode (fire-and-forget atomics, filter scans all
                                   vertices) once the frontier's edges reach V / div; 0 = 8 */
@@ -107,8 +107,9 @@ typedef struct {
                                   wait; the threshold moves to the smallest waiting value + delta
                                   when nothing below it is left.  0 = no waiting (Bellman-Ford
                                   frontier); -1 (default) = automatic: 20 x mean edge weight on
-                                  weighted graphs of average degree <= 8, else 0.  Results are
-                                  identical either way. */
+                                  weighted graphs of average degree <= 8 whose largest degree
+                                  is below 32 x the mean, else 0.  Results are identical
+                                  either way. */
   int32_t dense_wide_addr;     /* 1 = the lane-per-query loop addresses value rows with 64-bit
                                   addresses even where 32-bit offsets inside one word's rows
                                   reach them (V x 256 bytes < 4 GiB); 0 (default) = only where
