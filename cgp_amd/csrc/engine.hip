@@ -1287,65 +1287,69 @@ __device__ __forceinline__ u32 wave_fetch(u32* ctr, u32 n) {
 }
 
 // Wave-level claims of the units [0, n), in NSHARD contiguous shards: shard s
-// covers [n*s/NSHARD, n*(s+1)/NSHARD) and belongs to the workgroups with
-// blockIdx % NSHARD == s, one XCD.  Each of a shard's waves owns its first
-// units without any atomic (`chunk` units by its rank, and again after all of
-// the shard's waves if that covers the shard); what is left is handed
-// out through the shard's cursor, and a wave whose shard is exhausted looks at
-// all cursors with one load before it claims from another (cursors only grow).
-// A list that the first claims cover costs no atomic at all.  (Every wave used
-// to find each shard exhausted by an atomic of its own: 16 per wave and
-// launch, 16 us at 1024 waves and 93 us at 8192 with one unit of work.)
-// Claims never cross a shard's end.  All state is wave-uniform.  `turn` (0 to 3) rotates which waves come
+// covers [n*s/NSHARD, n*(s+1)/NSHARD) (strided: every NSHARD-th unit from s) and
+// belongs to the workgroups with blockIdx % NSHARD == s, one XCD.  A shard of at
+// most own_max units per wave is shared out without atomics, in one claim per
+// wave: the units rank, rank + waves, ...  In a larger one each wave owns the
+// first `chunk` units by its rank, what is left is handed out through the
+// shard's cursor, and a wave whose shard is exhausted looks at all cursors with
+// one load before it claims from another (cursors only grow).  (Every wave used
+// to find each shard exhausted by an atomic of its own: 16 per wave and launch,
+// 16 us at 1024 waves and 93 us at 8192 with one unit of work.)
+// A claim is cnt units, lo + i * step of shard s, and never crosses a shard's
+// end.  All state is wave-uniform.  `turn` (0 to 3) rotates which waves come
 // first, so that the short lists of consecutive phases go to different waves.
 struct ShardFetch {
-  u32 n, chunk, wpb;
+  u32 n, chunk, wpb, own_max;
   int s;
-  bool strided;
-  u32 own;   // start of this wave's next own claim in its shard
+  bool strided, first;
   u32 rank;
-  __device__ __forceinline__ ShardFetch(u32 n_, u32 chunk_, u32 turn, bool strided_ = false)
-      : n(n_), chunk(chunk_), strided(strided_) {
+  u32 lo, cnt, step;  // the last claim
+  __device__ __forceinline__ ShardFetch(u32 n_, u32 chunk_, u32 own_max_, u32 turn, bool strided_ = false)
+      : n(n_), chunk(chunk_), own_max(own_max_), strided(strided_), first(true), lo(0), cnt(0), step(1) {
     wpb = blockDim.x / 64u;
     s = (int)(blockIdx.x % NSHARD);
     const u32 nw = waves(s);
     rank = (blockIdx.x / NSHARD) * wpb + (u32)uniform32((int32_t)(threadIdx.x >> 6)) + turn * (nw / 4u);
     if (rank >= nw) rank -= nw;
-    own = rank * chunk;
   }
   __device__ __forceinline__ u32 waves(int sh) const { return (gridDim.x - (u32)sh + NSHARD - 1) / NSHARD * wpb; }
   __device__ __forceinline__ u32 begin(int sh) const { return (u32)(((u64)n * (u32)sh) / NSHARD); }
   __device__ __forceinline__ u32 size(int sh) const {
     return strided ? (n + NSHARD - 1u - (u32)sh) / NSHARD : begin(sh + 1) - begin(sh);
   }
-  // Unit i of the shard the last claim was from.
-  __device__ __forceinline__ u32 unit(u32 i) const { return strided ? i * NSHARD + (u32)s : begin(s) + i; }
-  // Units of a shard that its waves own: all of them when that is at most
-  // two claims per wave, else one claim each.  (A 1001x777 grid with 5 SSSP at
-  // 1 / 2 / 4 / 8 claims: 5.31 / 5.26 / 5.13 / 5.12 ms, RMAT-20 64 SSSP 6.48 /
-  // 6.36 / 6.38 / 6.85, 2048^2 grid 128 SSSP 99.1 / 98.8 / 101.1 / 100.5.)
-  __device__ __forceinline__ u32 owned(int sh) const {
-    const u32 all = size(sh), round = waves(sh) * chunk;
-    return all <= 2u * round ? all : round;
+  // Unit i of the last claim, as an index of [0, n).
+  __device__ __forceinline__ u32 unit(u32 i) const {
+    const u32 x = lo + i * step;
+    return strided ? x * NSHARD + (u32)s : begin(s) + x;
   }
-  __device__ __forceinline__ bool next(Ctr* cur, u32& lo, u32& hi) {
-    {
-      const u32 mine = owned(s);  // (a wave that claims from another shard has own past its end)
-      if (own < mine) {
-        lo = own;
-        hi = min(mine, lo + chunk);
-        own += waves(s) * chunk;
-        return true;
+  __device__ __forceinline__ bool all_owned(int sh) const { return size(sh) <= own_max * waves(sh); }
+  // Units of a shard that its waves own.
+  __device__ __forceinline__ u32 owned(int sh) const {
+    return all_owned(sh) ? size(sh) : min(size(sh), waves(sh) * chunk);
+  }
+  __device__ __forceinline__ bool next(Ctr* cur) {
+    if (first) {
+      first = false;
+      const u32 all = size(s);
+      if (all_owned(s)) {
+        lo = rank;
+        step = waves(s);
+        cnt = lo < all ? (all - lo + step - 1) / step : 0u;
+      } else {
+        lo = rank * chunk;
+        cnt = lo < all ? min(chunk, all - lo) : 0u;
       }
-      own = ~0u;
+      if (cnt) return true;
     }
+    step = 1;
     while (true) {
       const u32 base = owned(s), sz = size(s) - base;
       if (sz) {
         const u32 i = wave_fetch(&cur[s].v, chunk);
         if (i < sz) {
           lo = base + i;
-          hi = min(size(s), lo + chunk);
+          cnt = min(chunk, sz - i);
           return true;
         }
       }
@@ -1360,6 +1364,13 @@ struct ShardFetch {
     }
   }
 };
+
+// Units per wave up to which a shard is shared out without atomics: units that
+// a claim fetches side by side (expand_units), and groups that it takes one
+// after the other.  At 2 / 8 / 32 units RMAT-16 32 BFS takes 428 / 407 / 403 us,
+// RMAT-22 one BFS and WCC 1.79 / 1.76 / 1.73 ms, 160 BFS 7.55 / 7.53 / 7.62 ms;
+// at 2 / 4 groups a 1001x777 grid with 5 SSSP 5.31 / 5.24 ms.
+constexpr u32 OWN_UNITS = 16, OWN_GROUPS = 4;
 
 // Units per claim of a list of n units on nw waves: several when every wave
 // has many to take (each claim is an atomic on a line that an eighth of the
@@ -1389,7 +1400,6 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   const u32* const done = C->use_done ? P.done : nullptr;
   if (C->raised) raise_far<W, SPARSE>(P, C->thr_old, thr, rshift, stamp, t);
   const int lane = lane_id();
-  u32 lo, hi;
   // Phase L.  A chunk is two units, or up to 32 of 128 edges while that leaves
   // every unit a wave of its own.
   const u32 nL = C->bcount[p][2].v;
@@ -1397,15 +1407,15 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
     u32 sh = 1;
     while (sh < 5 && (nL << (sh + 1)) <= nw) ++sh;
     const u32 n = nL << sh;
-    ShardFetch sf(n, claim_units(n, nw), 0, P.mix_small);
-    while (sf.next(C->shard[p][SH_L], lo, hi)) {
-      const u32 i = sf.unit(min(lo + (u32)lane, hi - 1));
+    ShardFetch sf(n, claim_units(n, nw), OWN_UNITS, 0, P.mix_small);
+    while (sf.next(C->shard[p][SH_L])) {
+      const u32 i = sf.unit(min((u32)lane, sf.cnt - 1));
       const u64 item = P.large[p][i >> sh];
       const u32 part = i & ((1u << sh) - 1u);
       const int32_t u = (int32_t)(item >> 32);
       const int32_t e0 = P.off[u] + (int32_t)((u32)item * LCHUNK + part * ((u32)LCHUNK >> sh));
       const int32_t e1 = min(P.off[u + 1], e0 + (LCHUNK >> sh));
-      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, (u32)item == 0 && part == 0, done, bfs_on, dense_t,
+      expand_units<W, SPARSE>(P, (int)sf.cnt, u, e0, e1, (u32)item == 0 && part == 0, done, bfs_on, dense_t,
                               rshift, stamp, thr, t);
     }
   }
@@ -1418,16 +1428,16 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
     u32 sh = 0;
     while (sh < 3 && (nM << (sh + 1)) <= nw) ++sh;
     const u32 n = nM << sh;
-    ShardFetch sf(n, claim_units(n, nw), 1, P.mix_small);
-    while (sf.next(C->shard[p][SH_M], lo, hi)) {
-      const u32 i = sf.unit(min(lo + (u32)lane, hi - 1));
+    ShardFetch sf(n, claim_units(n, nw), OWN_UNITS, 1, P.mix_small);
+    while (sf.next(C->shard[p][SH_M])) {
+      const u32 i = sf.unit(min((u32)lane, sf.cnt - 1));
       const int32_t u = P.medium[p][i >> sh];
       const int32_t b = P.off[u], d = P.off[u + 1] - b;
       const u32 part = i & ((1u << sh) - 1u);
       // Parts of whole 64-edge steps.
       const int32_t len = (int32_t)((((u32)d + 63u) / 64u + (1u << sh) - 1u) >> sh) * 64;
       const int32_t e0 = b + (int32_t)part * len, e1 = min(b + d, e0 + len);
-      expand_units<W, SPARSE>(P, (int)(hi - lo), u, e0, e1, part == 0, done, bfs_on, dense_t, rshift, stamp, thr, t);
+      expand_units<W, SPARSE>(P, (int)sf.cnt, u, e0, e1, part == 0, done, bfs_on, dense_t, rshift, stamp, thr, t);
     }
   }
   // Phase S.  Groups of 64 entries, halved down to 4 while that leaves every
@@ -1437,9 +1447,9 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
     u32 gsz = 64;
     while (gsz > 4 && nS <= (gsz / 2) * nw) gsz /= 2;
     const u32 ng = (nS + gsz - 1) / gsz;
-    ShardFetch sf(ng, claim_units(ng, nw), 2);
-    while (sf.next(C->shard[p][SH_S], lo, hi)) {
-      for (u32 g = lo; g < hi; ++g)
+    ShardFetch sf(ng, claim_units(ng, nw), OWN_GROUPS, 2);
+    while (sf.next(C->shard[p][SH_S])) {
+      for (u32 g = 0; g < sf.cnt; ++g)
         expand_flat_vertices<W, SPARSE>(P, P.small[p], sf.unit(g), ng, gsz, nS, done, bfs_on, dense_t, rshift, stamp, thr, t);
     }
   }
@@ -1540,9 +1550,8 @@ __global__ __launch_bounds__(BS) void k_adv_dense(KP P) {
   u32* wtab = s_wt + (TAB == 2 ? (threadIdx.x & ~63u) : 0u);
   const bool sparse = C->dense_mode == 0;
   DenseClaim dc(nD, gridDim.x * (BS / 64), P.mix_small);
-  u32 lo, hi;
-  for (ShardFetch sf(dc.nc, 1, 0, true); sf.next(C->shard[p][SH_D], lo, hi);) {
-    dc.c = sf.unit(lo);
+  for (ShardFetch sf(dc.nc, 1, 1, 0, true); sf.next(C->shard[p][SH_D]);) {
+    dc.c = sf.unit(0);
     if (sparse) expand_dense_claim<W, true, U, TAB>(P, dc, rshift, stamp, thr, tab, wtab, t);
     else expand_dense_claim<W, false, U, TAB>(P, dc, rshift, stamp, thr, tab, wtab, t);
   }
@@ -1582,10 +1591,9 @@ __global__ __launch_bounds__(BLOCK) void k_adv_narrow(KP P) {
   const int rshift = P.cfg->rshift;
   const bool sparse = C->dense_mode == 0;
   Tally t;
-  u32 lo, hi;
   DenseClaim dc(nN, gridDim.x * (BLOCK / 64), P.mix_small);
-  for (ShardFetch sf(dc.nc, 1, 0, true); sf.next(C->shard[p][SH_N], lo, hi);) {
-    dc.c = sf.unit(lo);
+  for (ShardFetch sf(dc.nc, 1, 1, 0, true); sf.next(C->shard[p][SH_N]);) {
+    dc.c = sf.unit(0);
     if (sparse) expand_flat_narrow<W, true>(P, dc, rshift, stamp, t);
     else expand_flat_narrow<W, false>(P, dc, rshift, stamp, t);
   }
@@ -1690,9 +1698,8 @@ __global__ __launch_bounds__(BLOCK) void k_pull_sssp(KP P) {
   const u32 n = (u32)P.n_pull_items;
   Tally t;
   constexpr u32 FETCH_P = 16;
-  u32 lo, hi;
-  for (ShardFetch sf(n, FETCH_P, 0); sf.next(C->shard[p][SH_P], lo, hi);) {
-    for (u32 i = lo; i < hi; ++i) {
+  for (ShardFetch sf(n, FETCH_P, FETCH_P, 0); sf.next(C->shard[p][SH_P]);) {
+    for (u32 i = 0; i < sf.cnt; ++i) {
       if (sparse) pull_sssp_item<W, true, 8>(P, P.pull_items[sf.unit(i)], rshift, stamp, t);
       else pull_sssp_item<W, false, 8>(P, P.pull_items[sf.unit(i)], rshift, stamp, t);
     }
