@@ -439,14 +439,13 @@ __device__ __forceinline__ void load_masks(const KP& P, int32_t u, bool bfs_on, 
 // with a value in [old, thr) joins the next frontier, pairs at or above thr
 // stay, and pairs below old leave the set: their value was lowered below the
 // threshold after they were put there, which put them into a frontier then.
-// No SSSP pair is expanded in this iteration, so values stand still.
-template <int W, bool SPARSE>
-__device__ __forceinline__ void raise_far(const KP& P, u32 old, u32 thr, int rshift, u32 stamp, Tally& t) {
-  for (int64_t b = (int64_t)blockIdx.x * blockDim.x; b < P.V; b += (int64_t)gridDim.x * blockDim.x) {
-    const bool have = b + threadIdx.x < P.V;
-    const int32_t v = have ? (int32_t)(b + threadIdx.x) : 0;
-    bool first = false;
-    for (int w = 0; w < W && have; ++w) {
+// No SSSP pair is expanded in this iteration, so values stand still, and the
+// frontier mode is dense (the filter that raised the threshold sees to it).
+template <int W>
+__device__ __forceinline__ void raise_far(const KP& P, u32 old, u32 thr, int rshift, Tally& t) {
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < P.V; i += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t v = (int32_t)i;
+    for (int w = 0; w < W; ++w) {
       const u64 f = P.far[(size_t)v * W + w];
       if (!f) continue;
       const size_t vb = vrow(P.V, w, v, rshift);
@@ -471,15 +470,9 @@ __device__ __forceinline__ void raise_far(const KP& P, u32 old, u32 thr, int rsh
       if (near) {
         ++t.nnear;
         ++t.nnew;
-        u64* const n = &P.next[nxt_at<W>(v, w)];
-        if (SPARSE) {
-          if (atomicOr(n, near) == 0) first = true;
-        } else {
-          atomicOr(n, near);
-        }
+        atomicOr(&P.next[nxt_at<W>(v, w)], near);
       }
     }
-    if (SPARSE) touch(P, first && claim_first<W>(P.mark, v, stamp), v, stamp);
   }
 }
 
@@ -1398,7 +1391,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   const int rshift = P.cfg->rshift, dense_t = C->sssp_pull ? 0 : P.cfg->dense_t;
   const u32 nw = gridDim.x * (BS / 64);
   const u32* const done = C->use_done ? P.done : nullptr;
-  if (C->raised) raise_far<W, SPARSE>(P, C->thr_old, thr, rshift, stamp, t);
+  if (!SPARSE && C->raised) raise_far<W>(P, C->thr_old, thr, rshift, t);
   const int lane = lane_id();
   // Phase L.  A chunk is two units, or up to 32 of 128 edges while that leaves
   // every unit a wave of its own.
