@@ -269,10 +269,13 @@ struct cgp_engine {
   }
   int grid_advance() const { return (int)((int64_t)advance_blocks() * 256 / std::max(128, opts.block_size)); }
   // Filter workgroups: no more than have vertices to look at (each looks at
-  // BLOCK * FK per step), at most four per CU.
+  // BLOCK * FK per step), at most two per CU: the scans are as fast with fewer
+  // workgroups to reserve list entries and to report (at 2 / 3 / 4 / 8 per CU
+  // RMAT-22 160 BFS takes 7.46 / 7.55 / 7.62 / 7.65 ms, a 1001x777 grid with 5
+  // SSSP 5.14 / 5.24 / 5.20 / 5.24 ms).
   int grid_filter() const {
     int64_t need = ((int64_t)g->V + BLOCK * cgpk::FK - 1) / (BLOCK * cgpk::FK);
-    return (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cus * 4));
+    return (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cus * 2));
   }
 
   // Bytes of the per-vertex done bits.
