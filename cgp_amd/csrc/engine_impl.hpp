@@ -252,20 +252,21 @@ struct cgp_engine {
   // Grid sizes: persistent-style, sized to the device, independent of the
   // frontier so the launches can be captured once and replayed.
   // Same thread count per launch for every workgroup size.
-  // Advance workgroups: `advance_blocks`, or by default one per 24576 edges
-  // between one and three per CU.  The advance launches are persistent and
-  // hand their work out, so three per CU, as many as fit (141-146 registers:
+  // Advance workgroups: `advance_blocks`, or by default one per 16384 edges
+  // between two and three per CU.  The advance launches are persistent and
+  // hand their work out, so three per CU, as many as fit (141-147 registers:
   // three waves per SIMD), is the most that helps: later ones start when the
   // work is gone and only find that out (at 256 / 512 / 768 / 1024 / 2048
   // workgroups RMAT-22 mixed 256 takes 78.5 / 51.6 / 45.8 / 47.4 / 47.2 ms and
-  // 160 BFS 10.5 / 8.4 / 8.35 / 8.9 / 8.9 ms).  Below, the frontiers are too
-  // short for more: RMAT-18 (7.5 M edges) one SSSP 844 us at 256, 889 at 512;
-  // 2048^2 grid (17 M) 128 SSSP 151 / 117.5 / 113.8 / 112.4 ms at 256 / 512 /
-  // 640 / 768; RMAT-20 (31 M) 64 SSSP 8.6 / 6.35 / 6.23 / 6.30 ms.
+  // 160 BFS 10.5 / 8.4 / 8.35 / 8.9 / 8.9 ms).  The latency of one wave per
+  // SIMD shows on small graphs too, and a wave without work costs next to
+  // nothing (at 256 / 512 / 768: RMAT-16 32 BFS 423 / 384 / 367 us, RMAT-18 one
+  // SSSP 851 / 796 / 790, RMAT-14 20 queries 902 / 904 / 924, 1001x777 grid 5
+  // SSSP 5243 / 5064 / 5150, 2048^2 grid 128 SSSP 129 / 102 / 96.6 ms, RMAT-20
+  // 64 SSSP 8.6 / 6.34 / 6.25 ms).
   int advance_blocks() const {
     if (opts.advance_blocks > 0) return opts.advance_blocks;
-    const int64_t want = g->E / 24576;
-    return (int)std::max<int64_t>(cus, std::min<int64_t>(want, (int64_t)cus * 3));
+    return (int)std::max<int64_t>((int64_t)cus * 2, std::min<int64_t>(g->E / 16384, (int64_t)cus * 3));
   }
   int grid_advance() const { return (int)((int64_t)advance_blocks() * 256 / std::max(128, opts.block_size)); }
   // Filter workgroups: no more than have vertices to look at (each looks at
