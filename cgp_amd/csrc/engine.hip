@@ -476,6 +476,14 @@ __device__ __forceinline__ void raise_far(const KP& P, u32 old, u32 thr, int rsh
   }
 }
 
+// Edges [from, from + len) of u's list, as CSR slots; empty past its end.
+__device__ __forceinline__ void edge_range(const KP& P, int32_t u, u32 from, u32 len, int32_t& e0, int32_t& e1) {
+  const int32_t b = P.off[u];
+  const u32 d = (u32)(P.off[u + 1] - b);
+  e0 = b + (int32_t)min(from, d);
+  e1 = b + (int32_t)min(from + len, d);
+}
+
 // Lane k's value of a per-lane word, as a wave-uniform scalar.
 __device__ __forceinline__ u64 lane64(u64 x, int k) {
   return ((u64)(u32)__builtin_amdgcn_readlane((int)(u32)(x >> 32), k) << 32) |
@@ -531,13 +539,13 @@ __device__ __forceinline__ void expand_units(const KP& P, int cnt, int32_t u, in
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       // Lanes past the end re-read the last edge (a line already wanted).
-      const int32_t e = eb + i * 64 + lane;
-      st.ok[i] = e < end;
-      const int32_t ec = min(e, end - 1);
+      const int32_t at = i * 64 + lane;
+      st.ok[i] = at < end - eb;
+      const int32_t ec = eb + min(at, end - eb - 1);
       st.v[i] = P.idx[ec];
       st.wv[i] = (weighted_units >> k) & 1ull ? P.wt[ec] : 1u;
     }
-    eb += 64 * N;
+    eb = end - eb > 64 * N ? eb + 64 * N : end;
     return true;
   };
   Step cur, nxt;
@@ -725,8 +733,8 @@ __device__ __forceinline__ void expand_flat_dense(const KP& P, const DenseClaim&
   const int32_t u = (int32_t)(item >> 32);
   const int w = (int)((item >> 24) & 0xFF);
   const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
-  const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
-  const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
+  int32_t e0 = 0, e1 = 0;
+  if (have) edge_range(P, u, part * dc.len(), dc.len(), e0, e1);
   const u64 sm = have ? (P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) : 0ull;
   const bool inrow = lane < R;
   // Lane offset inside a value row; every lane reads a valid address of the
@@ -897,8 +905,8 @@ __device__ __forceinline__ void expand_flat_dense_tab(const KP& P, const DenseCl
   const int32_t u = (int32_t)(item >> 32);
   const int w = (int)((item >> 24) & 0xFF);
   const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
-  const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
-  const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
+  int32_t e0 = 0, e1 = 0;
+  if (have) edge_range(P, u, part * dc.len(), dc.len(), e0, e1);
   const u64 sm = have ? (P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) : 0ull;
   const u32 dlen = sm ? (u32)(e1 - e0) : 0u;
   if (have) {
@@ -1078,8 +1086,8 @@ __device__ __forceinline__ void expand_flat_narrow(const KP& P, const DenseClaim
   const int32_t u = (int32_t)(item >> 32);
   const int w = (int)((item >> 24) & 0xFF);
   const u32 part = dc.part(at, (u32)(item & 0xFFFFFF));
-  const int32_t e0 = have ? P.off[u] + (int32_t)(part * dc.len()) : 0;
-  const int32_t e1 = have ? max(e0, min(P.off[u + 1], e0 + (int32_t)dc.len())) : 0;
+  int32_t e0 = 0, e1 = 0;
+  if (have) edge_range(P, u, part * dc.len(), dc.len(), e0, e1);
   const u32 sm = have ? (u32)(P.front[(size_t)u * W + w] & P.cfg->val_bits[w]) & 0xFFFFu : 0u;
   const u32 d = sm ? (u32)(e1 - e0) : 0u;
   if (have) {
@@ -1406,8 +1414,8 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
       const u64 item = P.large[p][i >> sh];
       const u32 part = i & ((1u << sh) - 1u);
       const int32_t u = (int32_t)(item >> 32);
-      const int32_t e0 = P.off[u] + (int32_t)((u32)item * LCHUNK + part * ((u32)LCHUNK >> sh));
-      const int32_t e1 = min(P.off[u + 1], e0 + (LCHUNK >> sh));
+      int32_t e0, e1;
+      edge_range(P, u, (u32)item * LCHUNK + part * ((u32)LCHUNK >> sh), (u32)LCHUNK >> sh, e0, e1);
       expand_units<W, SPARSE>(P, (int)sf.cnt, u, e0, e1, (u32)item == 0 && part == 0, done, bfs_on, dense_t,
                               rshift, stamp, thr, t);
     }
@@ -1425,11 +1433,12 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
     while (sf.next(C->shard[p][SH_M])) {
       const u32 i = sf.unit(min((u32)lane, sf.cnt - 1));
       const int32_t u = P.medium[p][i >> sh];
-      const int32_t b = P.off[u], d = P.off[u + 1] - b;
       const u32 part = i & ((1u << sh) - 1u);
       // Parts of whole 64-edge steps.
-      const int32_t len = (int32_t)((((u32)d + 63u) / 64u + (1u << sh) - 1u) >> sh) * 64;
-      const int32_t e0 = b + (int32_t)part * len, e1 = min(b + d, e0 + len);
+      const u32 steps = ((u32)(P.off[u + 1] - P.off[u]) + 63u) / 64u;
+      const u32 len = ((steps + (1u << sh) - 1u) >> sh) * 64u;
+      int32_t e0, e1;
+      edge_range(P, u, part * len, len, e0, e1);
       expand_units<W, SPARSE>(P, (int)sf.cnt, u, e0, e1, part == 0, done, bfs_on, dense_t, rshift, stamp, thr, t);
     }
   }
