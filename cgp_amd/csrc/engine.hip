@@ -75,23 +75,6 @@ __device__ __forceinline__ void wave_append(bool pred, T item, u32* counter, T* 
   if (pred) list[base + rank_below(m)] = item;
 }
 
-// Wave-level exclusive prefix sum of per-lane counts, with one atomicAdd per
-// wave reserving the total; returns the lane's first slot.  Every lane of the
-// wave must call it.
-__device__ __forceinline__ u32 wave_reserve(u32 cnt, u32* counter) {
-  u32 x = cnt;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    u32 y = (u32)__shfl_up((int)x, d, 64);
-    if (lane_id() >= d) x += y;
-  }
-  u32 total = (u32)__shfl((int)x, 63, 64);
-  u32 base = 0;
-  if (total != 0 && lane_id() == 0) base = atomicAdd(counter, total);
-  base = (u32)__shfl((int)base, 0, 64);
-  return base + x - cnt;
-}
-
 // Workgroup-level exclusive prefix sums of N per-thread counts, with one
 // atomicAdd per non-zero total reserving the block's range in counters[0..N);
 // at[k] is the thread's first slot for counter k.  Every thread of the
@@ -166,10 +149,6 @@ __device__ __forceinline__ bool claim_first(u32* mark, int32_t v, u32 stamp) {
 
 // A wave-uniform value held in scalar registers.
 __device__ __forceinline__ int32_t uniform32(int32_t x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ u64 uniform64(u64 x) {
-  return ((u64)(u32)__builtin_amdgcn_readfirstlane((int)(u32)(x >> 32)) << 32) |
-         (u32)__builtin_amdgcn_readfirstlane((int)(u32)x);
-}
 
 // A wave-uniform pointer into global memory pinned to scalar registers, so
 // accesses through it use the SGPR-base + 32-bit lane-offset addressing form
@@ -492,11 +471,11 @@ __device__ __forceinline__ u64 lane64(u64 x, int k) {
 
 // Expands up to 64 (vertex, edge range) units with the whole wave, lane = edge:
 // lane k < cnt holds unit k, vertex u with edges [e0, e1) (empty ranges
-// allowed), and `lead` in the part of a vertex that counts it and its queries.
-// The units' masks are fetched by their lanes in parallel
-// and each unit's are then wave-uniform, in scalar registers; N steps of 64
-// edges are relaxed together, and the columns and weights of the next step, of
-// the next unit too, are on their way while a step is relaxed.
+// allowed), and `lead` in the part of a vertex or chunk that counts it and its
+// queries.  The units' masks are fetched by their lanes in parallel and each
+// unit's are then wave-uniform, in scalar registers; N steps of 64 edges are
+// relaxed together, and the columns and weights of the next step, of the next
+// unit too, are on their way while a step is relaxed.
 template <int W, bool SPARSE>
 __device__ __forceinline__ void expand_units(const KP& P, int cnt, int32_t u, int32_t e0, int32_t e1, bool lead,
                                              const u32* done, bool bfs_on, int dense_t, int rshift, u32 stamp, u32 thr, Tally& t) {
@@ -1416,8 +1395,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
       const int32_t u = (int32_t)(item >> 32);
       int32_t e0, e1;
       edge_range(P, u, (u32)item * LCHUNK + part * ((u32)LCHUNK >> sh), (u32)LCHUNK >> sh, e0, e1);
-      expand_units<W, SPARSE>(P, (int)sf.cnt, u, e0, e1, (u32)item == 0 && part == 0, done, bfs_on, dense_t,
-                              rshift, stamp, thr, t);
+      expand_units<W, SPARSE>(P, (int)sf.cnt, u, e0, e1, part == 0, done, bfs_on, dense_t, rshift, stamp, thr, t);
     }
   }
   // Phase M.  With fewer vertices than waves, 2, 4 or 8 waves take equal parts
