@@ -1370,7 +1370,7 @@ template <int W, bool SPARSE, int BS>
 __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   Ctl* C = P.ctl;
   const u32 iter = C->iter, p = iter & 1u;
-  const bool bfs_on = C->bfs_pull == 0;
+  const bool bfs_on = C->bfs_pull == BFS_PUSH;
   const u32 stamp = C->stamp_base + iter + 1;
   const u32 thr = C->thr;
   // In an SSSP pull iteration every vertex gathers its SSSP values itself: a
@@ -1435,7 +1435,7 @@ __device__ __forceinline__ void advance_push_body(const KP& P, Tally& t) {
   }
   // Phase P: high-degree vertices one wave each (64 neighbours per step,
   // early exit on a wave-wide OR), then the rest one lane each.
-  if (!bfs_on) {
+  if (C->bfs_pull == BFS_PULL) {
     u64 bb[W];
 #pragma unroll
     for (int w = 0; w < W; ++w) bb[w] = P.cfg->bfs_bits[w];
@@ -2154,12 +2154,20 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       consumed[w] = C->last_union[w];
       C->last_union[w] = w < W ? s_tot[NSUM + w] : 0ull;
     }
-    u32 pull = 0;
-    if (fp > 0) {
-      if (cfg->pull_policy == 1) pull = 1;
+    const u32 next_iter = iter + 1u;
+    // An iteration whose advance takes up far pairs (every raise of the
+    // threshold is followed by one) expands no SSSP pair, so it does not count
+    // towards the iteration limit of the SSSP queries; BFS queries do advance
+    // in it, and stop at the limit by themselves.
+    const u32 limit = C->max_iter, raises_run = C->bumps;
+    u32 pull = BFS_PUSH;
+    if (limit != 0 && next_iter >= limit) {
+      pull = BFS_OVER;
+    } else if (fp > 0) {
+      if (cfg->pull_policy == 1) pull = BFS_PULL;
       else if (cfg->pull_policy == 2) {
-        if (cur_pull) pull = fp >= cfg->push_pairs_thr ? 1u : 0u;
-        else pull = (fp >= cfg->pull_pairs_thr || fe >= cfg->pull_edges_thr) ? 1u : 0u;
+        if (cur_pull == BFS_PULL) pull = fp >= cfg->push_pairs_thr ? BFS_PULL : BFS_PUSH;
+        else pull = (fp >= cfg->pull_pairs_thr || fe >= cfg->pull_edges_thr) ? BFS_PULL : BFS_PUSH;
       }
     }
     C->bfs_pull = pull;
@@ -2216,7 +2224,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
       if (P.iters) {
         IterRec& r = P.iters[iter % ITER_RING];
         r.iter = iter;
-        r.pull = cur_pull | (cur_spull << 1);
+        r.pull = (cur_pull == BFS_PULL ? 1u : 0u) | (cur_spull << 1);
         r.dense = scan ? 1u : 0u;
         r.frontier_items = cur_items;
         r.touched = n;
@@ -2243,12 +2251,11 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     }
     C->adv_t0 = ~0ull;
     C->den_t0 = ~0ull;
-    const u32 next_iter = iter + 1u;
     C->iter = next_iter;
-    if ((total == 0 && !raised) || (C->max_iter != 0 && next_iter >= C->max_iter)) {
+    if ((total == 0 && !raised) || (limit != 0 && next_iter - raises_run >= limit)) {
       C->finished = 1;
     } else {
-      if (pull || spull) ++C->pull_iters;
+      if (pull == BFS_PULL || spull) ++C->pull_iters;
       else ++C->push_iters;
       if (dense) ++C->dense_iters;
     }

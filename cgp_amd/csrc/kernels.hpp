@@ -60,6 +60,9 @@ constexpr int PCHUNK = 256;        // edges per SSSP pull item
 // spread over NSHARD lines instead of one.
 constexpr int NSHARD = 8;
 enum : int { SH_M = 0, SH_S, SH_L, SH_D, SH_N, SH_P, NSH };
+// Ctl::bfs_pull: top-down, bottom-up, or not at all (the iteration limit is
+// reached and only SSSP queries go on).
+enum : u32 { BFS_PUSH = 0, BFS_PULL, BFS_OVER };
 // Workgroups spread their end-of-launch atomics over NSTRIPE lines (by
 // workgroup index); the filter's last workgroup combines them.  One line takes
 // about 12 ns per atomic whoever sends it, so 2048 workgroups on one line were
@@ -127,10 +130,10 @@ struct alignas(256) Stripe {
 struct Ctl {
   u32 iter;         // iteration of the current run (0xFFFFFFFF during seeding)
   u32 stamp_base;   // mark stamp of iteration i is stamp_base + i + 1
-  u32 finished;     // set when the next frontier is empty or max_iter reached
-  u32 bfs_pull;     // BFS bits use the pull kernel this iteration
+  u32 finished;     // set when the next frontier is empty or the iteration limit reached
+  u32 bfs_pull;     // how BFS bits advance this iteration (BFS_PUSH, ...)
   u32 sssp_pull;    // SSSP words are gathered (pulled) by every vertex this iteration
-  u32 max_iter;     // 0 = unlimited
+  u32 max_iter;     // 0 = unlimited; far-set raises do not count
   u32 push_iters;
   u32 pull_iters;
   u32 dense_mode;   // 1: advance uses fire-and-forget atomics, filter scans all vertices

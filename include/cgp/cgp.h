@@ -73,7 +73,10 @@ typedef struct {
   int32_t traversal_mode;      /* cgp_traversal_mode; default CGP_HYBRID */
   double pull_frontier_ratio;  /* pull when frontier >= ratio * V (default 0.15, types.hxx:30) */
   double pull_edge_ratio;      /* pull when frontier edges >= ratio * E (default 0.20, types.hxx:31) */
-  int32_t max_iterations;      /* 0 = until convergence (types.hxx:36) */
+  int32_t max_iterations;      /* 0 = until convergence (types.hxx:36).  With postponing an iteration
+                                  in which waiting SSSP pairs are taken up relaxes no SSSP edge and
+                                  does not count for SSSP queries (cgp_run_stats.iterations counts
+                                  it); BFS queries stop at this depth all the same */
   int32_t max_words;           /* cap on 64-bit mask words per pass; 0 = tuned */
   int32_t block_size;          /* workgroup size of the advance kernel: 128, 256 or 512; 0 = default 256 */
   int32_t bin_small;           /* degree <= bin_small: 8 lanes per vertex; 0 = tuned */
