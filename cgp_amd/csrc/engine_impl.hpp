@@ -268,7 +268,10 @@ struct cgp_engine {
     if (opts.advance_blocks > 0) return opts.advance_blocks;
     return (int)std::max<int64_t>((int64_t)cus * 2, std::min<int64_t>(g->E / 16384, (int64_t)cus * 3));
   }
-  int grid_advance() const { return (int)((int64_t)advance_blocks() * 256 / std::max(128, opts.block_size)); }
+  // (One 256-thread equivalent is still a whole workgroup of 512 threads.)
+  int grid_advance() const {
+    return (int)std::max<int64_t>(1, (int64_t)advance_blocks() * 256 / std::max(128, opts.block_size));
+  }
   // Filter workgroups: no more than have vertices to look at (each looks at
   // BLOCK * FK per step), at most two per CU: the scans are as fast with fewer
   // workgroups to reserve list entries and to report (at 2 / 3 / 4 / 8 per CU

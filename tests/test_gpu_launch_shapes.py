@@ -90,6 +90,14 @@ def test_push_work_lists(gpu, hub, opts):
     check(off, idx, wt, [BFS, BFS, SSSP, SSSP], [V // 2, 0, V // 2, 5], runs=2, dense_threshold=65, **opts)
 
 
+# The smallest launch the options allow, at every workgroup size (one 256-thread
+# equivalent is half a workgroup of 512 threads).
+@pytest.mark.parametrize("block", [128, 256, 512])
+def test_smallest_advance_launch(gpu, block):
+    off, idx, wt = ring_graph(5003, hub_degree=2500)
+    check(off, idx, wt, [BFS, SSSP, SSSP], [0, 2501, 77], runs=2, advance_blocks=1, block_size=block)
+
+
 # The same lists with two and four mask words, and on a directed graph.
 @pytest.mark.parametrize("n", [5, 70, 150])
 @pytest.mark.parametrize("directed", [False, True])
