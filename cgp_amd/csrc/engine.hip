@@ -2017,6 +2017,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   const int tid = (int)threadIdx.x;
   static_assert(NSUM + MAXW <= FSTAT && FSTAT <= 64, "a statistics line is written by one wave");
   static_assert(128 + NSH * NSHARD <= BLOCK, "one thread per work cursor");
+  static_assert(12 + NSTRIPE <= 32 && 32 + MAXW <= 64, "counters reset by threads of their own");
   {
     u64 sums[NSUM] = {pairs, epairs, fedges, apairs, averts, aqedges, ndone};
 #pragma unroll
@@ -2092,6 +2093,8 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     C->done[tid - 11].v = 0;
   } else if (tid == 11 + NSTRIPE + 1) {
     C->tcount[(stamp & 1u) ^ 1u].v = 0;  // filled next; this iteration's is reset by the next filter
+  } else if (tid >= 32 && tid < 32 + MAXW) {
+    C->far_union[tid - 32] = 0;  // filled by k_far_union, if it follows
   }
   if (tid >= 64 && tid < 128) {
     // One wave combines the stripes.
@@ -2262,15 +2265,44 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
   }
 }
 
-// OR of every vertex's far words into ctl->far_union (a serving session asks
-// whether a query still has far pairs).
-__global__ __launch_bounds__(BLOCK) void k_far_union(KP P, int W) {
+// The SSSP queries with pairs waiting for the near-far threshold, into
+// ctl->far_union, for a serving session: a query that has left the frontier
+// goes on while it has any.  A pair of the far set waits while its value is at
+// or above the threshold its iteration ran with; a smaller value was expanded
+// when it was found and the pair's bit is only cleared by the next raise.
+// Queries in the frontier, and those found already, are not looked up, and a
+// workgroup adds what nobody has added before, so the pass costs the read of
+// the far words.  (With every bit counted, one atomic per thread and a readback
+// of its own in each iteration a session of 12 SSSP queries on a 1001x777 grid
+// took 31.6 ms and one of 40 staggered ones on a 501x377 grid 486 ms; 9.7 and
+// 25 ms this way.)
+__global__ __launch_bounds__(BLOCK) void k_far_union(KP P, int W, int rshift) {
+  Ctl* C = P.ctl;
+  if (C->finished) return;
+  __shared__ u64 s_found[MAXW];
+  const int tid = (int)threadIdx.x;
+  if (tid < MAXW) s_found[tid] = 0;
+  __syncthreads();
+  const u32 thr = C->raised ? C->thr_old : C->thr;
   const int64_t n = (int64_t)P.V * W, stride = (int64_t)gridDim.x * BLOCK;
-  // The stride is a multiple of every W, so a thread stays on one word.
-  u64 x = 0;
-  const int64_t i0 = (int64_t)blockIdx.x * BLOCK + threadIdx.x;
-  for (int64_t i = i0; i < n; i += stride) x |= P.far[i];
-  if (x) atomicOr(&P.ctl->far_union[i0 % W], x);
+  const int64_t i0 = (int64_t)blockIdx.x * BLOCK + tid;
+  const int w = (int)i0 & (W - 1);  // W, a power of two, divides the stride: a thread stays on one word
+  const u64 out = P.cfg->val_bits[w] & ~C->last_union[w];
+  u64 found = 0;
+  for (int64_t i = i0; i < n; i += stride) {
+    for (u64 x = P.far[i] & out & ~found; x; x &= x - 1) {
+      const size_t row = vrow(P.V, w, (int32_t)(i / W), rshift);
+      const int q = __ffsll((long long)x) - 1;
+      if (P.vals[row + q] >= thr) found |= 1ull << q;
+    }
+  }
+  if (found) __hip_atomic_fetch_or(&s_found[w], found, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  __syncthreads();
+  if (tid < W && s_found[tid]) {
+    u64* const all = &C->far_union[tid];
+    if (s_found[tid] & ~__hip_atomic_load(all, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicOr(all, s_found[tid]);
+  }
 }
 
 // ------------------------------------------------------------------ utilities
@@ -2879,14 +2911,11 @@ void dispatch_seed(cgp_engine* en, int W, const KP& P, const int32_t* src, int n
   }
 }
 
-void far_union(cgp_engine* en, int W) {
-  const KP P = en->kp(W);
-  fill_u32(en->s, en->d_ctl->far_union, MAXW * 2, 0u, en->cus);
-  hipLaunchKernelGGL(k_far_union, dim3(en->cus * 4), dim3(BLOCK), 0, en->s, P, W);
+void far_union(cgp_engine* en, int W, int rshift) {
+  const int64_t need = ((int64_t)en->g->V * W + BLOCK - 1) / BLOCK;
+  hipLaunchKernelGGL(k_far_union, dim3((unsigned)std::min<int64_t>(need, (int64_t)en->cus * 4)), dim3(BLOCK), 0,
+                     en->s, en->kp(W), W, rshift);
   HIP_CHECK(hipGetLastError());
-  HIP_CHECK(hipMemcpyAsync(en->h_ctl->far_union, en->d_ctl->far_union, sizeof(en->h_ctl->far_union),
-                           hipMemcpyDeviceToHost, en->s));
-  HIP_CHECK(hipStreamSynchronize(en->s));
 }
 
 u32 narrow_mask(const Cfg& cfg, int W) {

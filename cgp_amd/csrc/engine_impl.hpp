@@ -375,9 +375,9 @@ void dispatch_iteration(cgp_engine* en, int W, const KP& P);
 void dispatch_seed_only(cgp_engine* en, int W, const KP& P, const int32_t* d_slot_src, int nslots);
 void dispatch_seed(cgp_engine* en, int W, const KP& P, const int32_t* d_slot_src, int nslots);
 void fill_u32(hipStream_t s, void* p, size_t n, u32 v, int cus);
-// OR of the far words of a serving session of W words into h_ctl->far_union
-// (waits for the engine's stream).
-void far_union(cgp_engine* en, int W);
+// Enqueues the lookup of the queries with waiting SSSP pairs (Ctl::far_union)
+// of a serving session, behind an iteration.
+void far_union(cgp_engine* en, int W, int rshift);
 // Narrow-word mask of a slot configuration (all SSSP words narrow, else 0).
 u32 narrow_mask(const Cfg& cfg, int W);
 // One batched run (all passes, WCC, output transpose); stats may be null.

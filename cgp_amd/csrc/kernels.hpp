@@ -152,7 +152,8 @@ struct Ctl {
   u32 done_verts;   // vertices that every BFS query of the pass has visited
   u32 use_done;     // the push launch looks a target up in KP::done before its record
   u64 last_union[MAXW];       // OR of the frontier words the last filter produced
-  alignas(16) u64 far_union[MAXW];  // OR of the far words, when asked for (k_far_union)
+  u64 far_union[MAXW];        // SSSP queries out of the frontier with waiting pairs, when asked for
+                              // (k_far_union)
   u64 prof[NPROF];            // work counters (profile mode)
   // Device-clock launch timing (wall_clock64 ticks): start of the running
   // advance / filter (its first workgroup), and the sums over the launches of

@@ -49,18 +49,26 @@ __global__ __launch_bounds__(BLOCK) void k_snapshot(const u32* vals, const int32
   }
 }
 
-// Resets the listed slots' value columns to INF and clears their visited
-// bits, leaving the slots ready for their next queries; in internal vertex
-// order, so the row and record writes stream.
-__global__ __launch_bounds__(BLOCK) void k_slot_reset(u32* vals, u64* visited, int32_t V, int W, int rshift,
-                                                      SnapArgs a) {
+// Resets the listed slots' value columns to INF and clears their visited bits
+// and, with postponing, what is left of them in the far set (pairs lowered
+// below the threshold after they were put there), leaving the slots ready for
+// their next queries; in internal vertex order, so the row and record writes
+// stream.
+__global__ __launch_bounds__(BLOCK) void k_slot_reset(u32* vals, u64* visited, u64* far, int32_t V, int W,
+                                                      int rshift, SnapArgs a) {
   for (int64_t u = (int64_t)blockIdx.x * BLOCK + threadIdx.x; u < V; u += (int64_t)gridDim.x * BLOCK) {
     for (int k = 0; k < a.n; ++k) {
       const u32 e = a.ent[k];
       vals[(((size_t)(e >> 24) * (size_t)V + (size_t)u) << rshift) + ((e >> 16) & 0xFFu)] = INF;
     }
     for (int w = 0; w < W; ++w)
-      if (a.clear[w]) visited[(size_t)u * (2 * W) + w] &= ~a.clear[w];  // visited half of the record
+      if (a.clear[w]) {
+        visited[(size_t)u * (2 * W) + w] &= ~a.clear[w];  // visited half of the record
+        if (far) {
+          const u64 f = far[(size_t)u * W + w];
+          if (f & a.clear[w]) far[(size_t)u * W + w] = f & ~a.clear[w];
+        }
+      }
   }
 }
 
@@ -92,6 +100,7 @@ struct ServeState {
   int busy = 0;
   u32 iter = 0;            // device iteration counter mirror
   bool need_restart = false;
+  bool far_out = false;    // some query is out of the frontier with pairs waiting
   std::deque<cgp_completion> done;
   // WCC labels of the session (computed on the first WCC request).
   bool wcc_ready = false;
@@ -307,7 +316,7 @@ void retire(cgp_engine* en, ServeState* ss, const std::vector<int>& conv) {
       hipLaunchKernelGGL(k_snapshot, dim3(en->cus * 8), dim3(BLOCK), 0, en->s, (const u32*)en->vals.p,
                          (const int32_t*)en->g->inv, V, ss->rshift, a, (u32*)staging->p);
     hipLaunchKernelGGL(k_slot_reset, dim3(en->cus * 8), dim3(BLOCK), 0, en->s, (u32*)en->vals.p,
-                       (u64*)en->visited.p, V, ss->W, ss->rshift, a);
+                       (u64*)en->visited.p, en->kp(ss->W).far, V, ss->W, ss->rshift, a);
     HIP_CHECK(hipGetLastError());
   }
   std::vector<cgp_completion> comps((size_t)k);
@@ -497,8 +506,15 @@ cgp_status cgp_serve_step(cgp_engine* en, int32_t max_iterations, cgp_completion
       }
       if (max_iterations > 0 && ran >= max_iterations) break;
       dispatch_iteration(en, W, en->kp(W));
-      HIP_CHECK(hipMemcpyAsync(en->h_ctl, en->d_ctl, CTL_HOST_BYTES, hipMemcpyDeviceToHost, en->s));
-      HIP_CHECK(hipStreamSynchronize(en->s));
+      // While queries are out of the frontier with pairs waiting, the lookup of
+      // those goes with the iteration, ahead of its readback.
+      const bool asked = ss->far_out;
+      if (asked) far_union(en, W, ss->rshift);
+      const auto read_back = [&]() {
+        HIP_CHECK(hipMemcpyAsync(en->h_ctl, en->d_ctl, CTL_HOST_BYTES, hipMemcpyDeviceToHost, en->s));
+        HIP_CHECK(hipStreamSynchronize(en->s));
+      };
+      read_back();
       ++ran;
       const Ctl& hc = *en->h_ctl;
       ss->iter = hc.iter;
@@ -506,21 +522,26 @@ cgp_status cgp_serve_step(cgp_engine* en, int32_t max_iterations, cgp_completion
       // once the frontier has no work left (`finished`: its remaining bits sit
       // on vertices without out-edges, and the kernels stop until restarted).
       conv.clear();
-      // With an empty far set nobody has far pairs (just before a raise its
-      // minimum is not known).
-      bool far_known = hc.far_min == INF && !hc.raised;
-      if (far_known) std::memset(en->h_ctl->far_union, 0, sizeof(hc.far_union));
+      // With an empty far set nobody has waiting pairs (just before a raise its
+      // minimum is not known); else, when queries leave the frontier, they are
+      // looked up, with a readback of their own in the first such iteration.
+      bool far_known = asked || hc.finished || (hc.far_min == INF && !hc.raised);
+      ss->far_out = false;
       for (int k = 0; k < ss->nslots; ++k) {
         if (!ss->slots[k].busy || ss->iter < ss->slots[k].start) continue;
         const int w = k >> 6;
         const u64 bit = 1ull << (k & 63);
         if (!hc.finished && (hc.last_union[w] & bit)) continue;
-        // An SSSP query out of the frontier may still have pairs waiting for
-        // the near-far threshold.
         if (!hc.finished && (en->h_cfg->val_bits[w] & bit)) {
-          if (!far_known) far_union(en, W);
-          far_known = true;
-          if (hc.far_union[w] & bit) continue;
+          if (!far_known) {
+            far_union(en, W, ss->rshift);
+            read_back();
+            far_known = true;
+          }
+          if (hc.far_union[w] & bit) {
+            ss->far_out = true;
+            continue;
+          }
         }
         conv.push_back(k);
       }

@@ -46,3 +46,55 @@ def test_iteration_limit(gpu, delta, kinds, opts):
             exp = np.where(hops <= k, hops * (90 if kind == SSSP else 1), INF).astype(np.uint32)
             assert np.array_equal(got[i], exp), (k, i, kind)
             assert np.array_equal(out.to_host(shape=(len(kinds), V))[i], exp), (k, i, kind, "static")
+
+
+def serve(en, queries, slots, max_iterations=1):
+    """Completions by ticket of a session that has all queries from the start."""
+    en.serve_start(max_slots=slots)
+    for i, (kind, source) in enumerate(queries):
+        en.serve_submit(kind, source, i, 0.0)
+    done = {}
+    while len(done) < len(queries):
+        for c in en.serve_step(max_iterations=max_iterations):
+            done[c["ticket"]] = c
+    en.serve_stop()
+    return done
+
+
+# Two parts: 0 -> 2 at 100 and 0 -> 1 -> 2 at 10 each (vertex 2 is put into the
+# far set at 100 and then lowered below the threshold of 50, which leaves its
+# bit there), and a path of weight 1 whose queries stay below the threshold.  The
+# queries of the first part are done after their third or fourth iteration,
+# whoever else is running, and their slot serves the next one.
+@pytest.mark.parametrize("first", [SSSP, BFS])
+@pytest.mark.parametrize("slots", [2, 64, 128])
+def test_completion_beside_others(gpu, slots, first):
+    n = 45
+    a = np.arange(3, 3 + n)
+    off, idx, wt = csr(4 + n, np.concatenate([[0, 0, 1], a]), np.concatenate([[2, 1, 2], a + 1]),
+                       np.concatenate([[100, 10, 10], np.ones(n)]))
+    og = O.G(off, idx, wt)
+    en = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, idx, wt), sssp_delta=50)
+    queries = [(SSSP, 3), (SSSP, 0)] + [(first if i % 2 else SSSP, 0) for i in range(5)]
+    done = serve(en, queries, slots)
+    for i, (kind, source) in enumerate(queries):
+        assert np.array_equal(done[i]["result"], O.expected(og, kind, source)), i
+        if source == 0:
+            assert done[i]["iterations"] <= 4, (i, done[i]["iterations"])
+    assert done[0]["iterations"] >= n
+
+
+# Sessions of one to eight mask words on a road network: queries of every word
+# wait at the threshold while others run.
+@pytest.mark.parametrize("slots", [16, 128, 300, 512])
+@pytest.mark.parametrize("delta", [300, -1])
+def test_serving_mask_words(gpu, slots, delta):
+    h = cgp_amd.HostCSR.grid(37, 41, p_extra=0.01, seed=7, wmin=1, wmax=1000)
+    og = O.G.of(h)
+    en = cgp_amd.Engine(cgp_amd.Graph.from_host(h), sssp_delta=delta)
+    assert en.opts["sssp_delta"] > 0
+    src = h.sample_sources(min(h.V, slots + slots // 2), seed=slots)
+    queries = [(SSSP if i % 4 else BFS, int(s)) for i, s in enumerate(src)]
+    done = serve(en, queries, slots, max_iterations=0 if slots == 300 else 2)
+    for i, (kind, source) in enumerate(queries):
+        assert np.array_equal(done[i]["result"], O.expected(og, kind, source)), (i, kind, source)
