@@ -2971,6 +2971,26 @@ void fill_row_prefix(hipStream_t s, void* p, size_t nrows, int l4, u32 v, int cu
 
 static int wlog(int W) { return W == 1 ? 0 : W == 2 ? 1 : W == 4 ? 2 : 3; }
 
+// Whether a directed graph's vertices link their first two neighbours, and the
+// trees are flattened, before every edge hooks.  Hooking everything from single
+// vertices walks and rewrites long paths, and with the sample most edges find
+// both ends under one root at once.  That holds on skewed graphs of any size
+// (directed R-MAT, 1, 2 and 8 edges per vertex, us without / with the sample:
+// 248 / 113, 620 / 162 and 714 / 179 at 300007 vertices, 603 / 172, 728 / 182
+// and 855 / 218 at 2^20) unless they have fewer edges than vertices (a star of
+// 2^20: 42 / 49).  On other graphs the sample has to leave most edges for after
+// it (a grid's 2 edges per vertex: 107 / 205 at 2^17 vertices), and on uniform
+// random ones it is the sample that walks the long paths once the vertices are
+// many: 4 and 16 edges per vertex 330 / 155 and 1528 / 141 at 2^14 vertices,
+// 2480 / 1560 and 1410 / 1480 at 2^18, 1800 / 1950 and 1500 / 2350 at 2^19,
+// 1400 / 2760 and 1370 / 3140 at 2^20.  (Edges between near vertices gain at
+// every size, 1330 / 710 at 4 per vertex and 2^20, but nothing here tells the
+// two apart.)
+static bool sample_before_hooks(const cgp_graph* g) {
+  if (g->symmetric || g->V < 4096) return false;
+  return g->skewed ? g->E >= g->V : g->E >= 4 * (int64_t)g->V && g->V <= (1 << 18);
+}
+
 void compute_wcc(cgp_engine* en) {
   const cgp_graph* g = en->g;
   en->parent.ensure((size_t)g->V * 4 + 4);
@@ -2980,12 +3000,8 @@ void compute_wcc(cgp_engine* en) {
   constexpr int kSample = 2, kProbe = 1024;
   if (!g->symmetric || g->V < 4096) {
     // Directed graphs (weak components need every stored edge) and tiny
-    // graphs: a hooking pass over all edges.  On larger graphs every vertex
-    // links its first two neighbours before, and the trees are flattened, so
-    // that most edges find both ends under one root at once: hooking everything
-    // from single vertices walks and rewrites long paths (2.1 M edges of a
-    // 300007-vertex R-MAT graph: 750 us of kernels without the sample, 150 with).
-    if (g->V >= 4096) {
+    // graphs: a hooking pass over all edges.
+    if (sample_before_hooks(g)) {
       hipLaunchKernelGGL(k_wcc_sample, dim3(gb), dim3(BLOCK), 0, en->s, (const int32_t*)g->off,
                          (const int32_t*)g->idx, g->V, kSample, parent);
       hipLaunchKernelGGL(k_wcc_compress, dim3(gb), dim3(BLOCK), 0, en->s, parent, g->V);

@@ -146,6 +146,30 @@ def test_wcc_directed(gpu, V):
     assert np.array_equal(got[0], exp) and np.array_equal(got[1], exp)
 
 
+# The same where the sample's rule turns: skewed graphs from as many edges as
+# vertices on, others from four edges per vertex on and up to 2^18 vertices.
+# Edges lead within sevenths of the vertices, so there are seven parts or more.
+@pytest.mark.parametrize("V", [4096, 30011, 1 << 18, (1 << 18) + 1])
+@pytest.mark.parametrize("per_vertex", [0.9, 1.1, 3.9, 4.1])
+@pytest.mark.parametrize("hub", [False, True])
+def test_wcc_directed_sample_rule(gpu, V, per_vertex, hub):
+    rng = np.random.RandomState(V % 1000 + int(per_vertex * 10))
+    n = int(V * per_vertex * 1.02) - (V // 7 if hub else 0)
+    a = rng.randint(0, V, n).astype(np.int64)
+    b = np.minimum(V - 1, a % 7 + 7 * rng.randint(0, V // 7, n))
+    if hub:
+        a = np.concatenate([a, np.full(V // 7, 7)])
+        b = np.concatenate([b, np.arange(V // 7) * 7])
+    keep = (a != b) & (a % 7 == b % 7)
+    key = np.unique(a[keep] * V + b[keep])
+    src, dst = key // V, key % V
+    off = np.zeros(V + 1, np.int64)
+    np.add.at(off, src + 1, 1)
+    off, dst = np.cumsum(off).astype(np.int32), dst.astype(np.int32)
+    got = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, dst)).wcc(1)[0]
+    assert np.array_equal(got, O.expected(O.G(off, dst, None), WCC, 0))
+
+
 # Near-far: pairs at or above the threshold wait in the far set.  Small and
 # large steps, one to four mask words, BFS beside it, vertices without
 # out-edges (a frontier that is empty while pairs wait), both frontier modes.
