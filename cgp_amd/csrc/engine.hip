@@ -2272,7 +2272,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
 // when it was found and the pair's bit is only cleared by the next raise.
 // Queries in the frontier, and those found already, are not looked up, and a
 // workgroup adds what nobody has added before, so the pass costs the read of
-// the far words.  (With every bit counted, one atomic per thread and a readback
+// the far words (5.5 us for one word of 777 777 vertices).  (With every bit counted, one atomic per thread and a readback
 // of its own in each iteration a session of 12 SSSP queries on a 1001x777 grid
 // took 31.6 ms and one of 40 staggered ones on a 501x377 grid 486 ms; 9.7 and
 // 25 ms this way.)
@@ -2548,16 +2548,20 @@ __global__ __launch_bounds__(BLOCK) void k_fill_rows(const int32_t* off, int32_t
 enum : u32 { CSR_BAD_OFFSETS = 1, CSR_BAD_INDEX = 2, CSR_UNSORTED = 4, CSR_ASYMMETRIC = 8, CSR_ASYM_WEIGHTS = 16 };
 
 // Flags decreasing offsets and takes the largest degree (into *maxdeg).
-__global__ __launch_bounds__(BLOCK) void k_csr_check_offsets(const int32_t* off, int32_t V, u32* flags,
-                                                             u32* maxdeg) {
+__global__ __launch_bounds__(BLOCK) void k_csr_check_offsets(const int32_t* off, int32_t V, int32_t hub, u32* flags,
+                                                             u32* maxdeg, u64* hub_edges) {
   bool bad = false;
   int32_t m = 0;
+  u64 he = 0;
   for (int64_t v = (int64_t)blockIdx.x * BLOCK + threadIdx.x; v < V; v += (int64_t)gridDim.x * BLOCK) {
     const int32_t d = off[v + 1] - off[v];
     bad |= d < 0;
     m = max(m, d);
+    he += d >= hub ? (u64)d : 0ull;
   }
   if (__ballot(bad) && lane_id() == 0) atomicOr(flags, (u32)CSR_BAD_OFFSETS);
+  he = wave_sum64(he);
+  if (lane_id() == 0 && he) atomicAdd(hub_edges, he);
   for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
   if (lane_id() == 0 && m > 0) atomicMax(maxdeg, (u32)m);
 }
@@ -3708,9 +3712,16 @@ cgp_status cgp_copy_device(void* dst, const void* src, uint64_t bytes) {
   });
 }
 
-// Largest degree at least 32x the mean (power-law graphs; not meshes or grids).
-static bool is_skewed(int32_t V, int64_t E, int32_t maxd) {
-  return V > 0 && (double)maxd >= 32.0 * std::max(1.0, (double)E / (double)V);
+// Smallest degree that is at least 32x the mean: a graph with such a vertex is
+// skewed (power-law graphs are; meshes and grids are not, unless single
+// vertices have many neighbours).
+static int32_t hub_degree(int32_t V, int64_t E) {
+  return (int32_t)std::min(2147483647.0, std::ceil(32.0 * std::max(1.0, (double)E / (double)std::max(1, V))));
+}
+
+static void set_skew(cgp_graph* g, int32_t maxd, int64_t hub_edges) {
+  g->skewed = g->V > 0 && maxd >= hub_degree(g->V, g->E);
+  g->power_law = g->skewed && hub_edges * 20 >= g->E;
 }
 
 cgp_status cgp_graph_create_csr(int32_t V, int64_t E, const int32_t* off, const int32_t* idx,
@@ -3761,8 +3772,14 @@ cgp_status cgp_graph_create_csr_ex(int32_t V, int64_t E, const int32_t* off, con
     // neighbours being close already.  Results, sources and WCC labels stay
     // in the caller's numbering.
     int32_t maxd = 0;
-    for (int32_t v = 0; v < V; ++v) maxd = std::max(maxd, off[v + 1] - off[v]);
-    g->skewed = is_skewed(V, E, maxd);
+    int64_t hub_edges = 0;
+    const int32_t hub = hub_degree(V, E);
+    for (int32_t v = 0; v < V; ++v) {
+      const int32_t d = off[v + 1] - off[v];
+      maxd = std::max(maxd, d);
+      if (d >= hub) hub_edges += d;
+    }
+    set_skew(g.get(), maxd, hub_edges);
     std::vector<int32_t> perm;
     const bool auto_on = V >= (1 << 21) && g->skewed;
     if (V > 0 && (renumber == CGP_RENUMBER_ON || (renumber == CGP_RENUMBER_AUTO && auto_on)))
@@ -3857,8 +3874,8 @@ cgp_status cgp_graph_create_csr_device(int32_t V, int64_t E, const int32_t* off,
     HIP_CHECK(hipMemcpy(&ends[1], off + V, 4, hipMemcpyDeviceToHost));
     if (ends[0] != 0 || ends[1] != E) cgpi::fail(CGP_EINVAL, "cgp_graph_create_csr_device: offsets do not span [0, E]");
     // Scratch: flags, degree-list counters, weight sum.
-    HIP_CHECK(hipMalloc((void**)&own.d_tmp, 32));
-    HIP_CHECK(hipMemset(own.d_tmp, 0, 32));
+    HIP_CHECK(hipMalloc((void**)&own.d_tmp, 40));
+    HIP_CHECK(hipMemset(own.d_tmp, 0, 40));
     u32* flags = own.d_tmp;
     u32* cnt = own.d_tmp + 2;
     u64* wsum = (u64*)(own.d_tmp + 4);
@@ -3871,11 +3888,15 @@ cgp_status cgp_graph_create_csr_device(int32_t V, int64_t E, const int32_t* off,
       return f;
     };
     u32* maxdeg = own.d_tmp + 6;
-    if (V > 0) hipLaunchKernelGGL(k_csr_check_offsets, gb, dim3(BLOCK), 0, 0, off, V, flags, maxdeg);
+    u64* hubs = (u64*)(own.d_tmp + 8);
+    if (V > 0)
+      hipLaunchKernelGGL(k_csr_check_offsets, gb, dim3(BLOCK), 0, 0, off, V, hub_degree(V, E), flags, maxdeg, hubs);
     if (read_flags() & CSR_BAD_OFFSETS) cgpi::fail(CGP_EINVAL, "cgp_graph_create_csr_device: offsets not monotone");
     u32 maxd = 0;
     HIP_CHECK(hipMemcpy(&maxd, maxdeg, 4, hipMemcpyDeviceToHost));
-    g->skewed = is_skewed(V, E, (int32_t)maxd);
+    u64 hub_edges = 0;
+    HIP_CHECK(hipMemcpy(&hub_edges, hubs, 8, hipMemcpyDeviceToHost));
+    set_skew(g, (int32_t)maxd, (int64_t)hub_edges);
     HIP_CHECK(hipMalloc((void**)&g->rows, (size_t)E * 4 + 4));
     if (V > 0) hipLaunchKernelGGL(k_fill_rows, gb, dim3(BLOCK), 0, 0, off, V, g->rows);
     if (E > 0) hipLaunchKernelGGL(k_csr_check_edges, gb, dim3(BLOCK), 0, 0, (const int32_t*)g->rows, idx, E, V, flags);
@@ -3997,9 +4018,15 @@ cgp_engine_opts resolve_opts(const cgp_graph* g, const cgp_engine_opts* opts, co
     // query and for 512); small-world graphs settle in few Bellman-Ford
     // iterations and skip it.
     const double deg = g->V > 0 ? (double)g->E / (double)g->V : 0.0;
-    // So are directed power-law graphs, which are as sparse (300007 vertices,
-    // 7 edges each, 11 SSSP: 2.05 ms without postponing, 2.34 with it).
-    o.sssp_delta = (g->weighted && deg <= 8.0 && g->mean_weight > 1.0 && !g->skewed)
+    // So are sparse power-law graphs (directed, 300007 vertices, 7 edges each,
+    // 11 SSSP: 2.05 ms without postponing, 2.34 with it), which are told by the
+    // share of the edges at vertices of 32x the mean degree: 0.10 to 0.45 on
+    // R-MAT graphs of 4096 to 2^20 vertices, at most 0.001 on a road network
+    // with a depot or a few.  One such vertex does not end the long paths: a
+    // 2000x1500 grid with a vertex of degree 130, 4 SSSP, takes 51.9 ms with
+    // postponing and 70.1 without (a 700x700 grid, whose paths its random
+    // neighbours cut to a few dozen hops, 10.4 and 9.0).
+    o.sssp_delta = (g->weighted && deg <= 8.0 && g->mean_weight > 1.0 && !g->power_law)
                        ? (int32_t)std::lround(20.0 * g->mean_weight)
                        : 0;
   }

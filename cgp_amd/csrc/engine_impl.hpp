@@ -38,6 +38,7 @@ struct cgp_graph {
   bool symmetric = false;
   bool weighted = false;
   bool skewed = false;  // largest degree at least 32x the mean
+  bool power_law = false;  // the vertices of such degrees hold at least a twentieth of the edges
   bool borrowed = false;  // off / idx / wt belong to the caller (cgp_graph_create_csr_device)
   bool sym_weights = false;  // symmetric, and every edge's reverse has the same weight (pull gathers)
   double mean_weight = 1.0;  // over all edges (1 when unweighted)

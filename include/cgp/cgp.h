@@ -110,9 +110,9 @@ typedef struct {
                                   wait; the threshold moves to the smallest waiting value + delta
                                   when nothing below it is left.  0 = no waiting (Bellman-Ford
                                   frontier); -1 (default) = automatic: 20 x mean edge weight on
-                                  weighted graphs of average degree <= 8 whose largest degree
-                                  is below 32 x the mean, else 0.  Results are identical
-                                  either way. */
+                                  weighted graphs of average degree <= 8 unless vertices of at
+                                  least 32 x that degree hold a twentieth of the edges, else 0.
+                                  Results are identical either way. */
   int32_t dense_wide_addr;     /* 1 = the lane-per-query loop addresses value rows with 64-bit
                                   addresses even where 32-bit offsets inside one word's rows
                                   reach them (V x 256 bytes < 4 GiB); 0 (default) = only where

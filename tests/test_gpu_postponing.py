@@ -98,3 +98,36 @@ def test_serving_mask_words(gpu, slots, delta):
     done = serve(en, queries, slots, max_iterations=0 if slots == 300 else 2)
     for i, (kind, source) in enumerate(queries):
         assert np.array_equal(done[i]["result"], O.expected(og, kind, source)), (i, kind, source)
+
+
+# The automatic step: road networks have it, also with a vertex of many
+# neighbours (here 130 of 16 700 edges); graphs with more of their edges at such
+# vertices (1600 of 19 700, or a power law) do not.  Graphs from host and device
+# arrays agree.
+@pytest.mark.parametrize("graph,on", [("grid", True), ("hub", True), ("hubs", False), ("web", False)])
+def test_automatic_step(gpu, graph, on):
+    if graph == "web":
+        V, rng = 5000, np.random.RandomState(3)
+        key = np.unique((V * rng.rand(7 * V) ** 4).astype(np.int64) * V + rng.randint(0, V, 7 * V))
+        src, dst = key // V, key % V
+        wt = rng.randint(1, 101, len(src))
+    else:
+        h = cgp_amd.HostCSR.grid(64, 64, p_extra=0.01, seed=3, wmin=1, wmax=100)
+        V, rng = h.V, np.random.RandomState(1)
+        src, dst, wt = np.repeat(np.arange(V), np.diff(h.offsets)), h.indices, h.weights
+        for hub, degree in ([(2000, 130)] if graph == "hub" else [(7, 800), (2000, 800)] if graph == "hubs" else []):
+            leaves = rng.choice(np.arange(2001, V), degree, replace=False)
+            src = np.concatenate([src, leaves, np.full(degree, hub)])
+            dst = np.concatenate([dst, np.full(degree, hub), leaves])
+            wt = np.concatenate([wt, np.arange(2 * degree) % degree % 100 + 1])
+    off, idx, w = csr(V, src, dst, wt)
+    assert len(idx) / V <= 8
+    og = O.G(off, idx, w)
+    bufs = [cgp_amd.DeviceBuffer.from_array(x) for x in (off, idx, w)]
+    for g in (cgp_amd.Graph.from_csr(off, idx, w), cgp_amd.Graph.from_device(V, len(idx), *bufs)):
+        en = cgp_amd.Engine(g)
+        assert en.opts["sssp_delta"] == (int(round(20 * w.mean(dtype=np.float64))) if on else 0)
+        sources = [0, 2000, V - 1, 7, 5]
+        got = en.run_batch([SSSP] * 5, sources)[0]
+        for i, s in enumerate(sources):
+            assert np.array_equal(got[i], O.expected(og, SSSP, s)), (i, s)
