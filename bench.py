@@ -95,7 +95,9 @@ def host_cpu():
 def bytes_builder(w, W):
     """Algorithmic bytes of (push launch, lane-per-query launch) in this
     engine's model: each byte at its natural width, once, no line waste; an
-    SSSP relaxation reads the target's 4-byte value of every active query."""
+    SSSP relaxation reads the target's 4-byte value of every active query, and
+    a BFS edge the target's visited words unless every BFS query has visited
+    it (known from a cached bit per vertex, which is not charged)."""
     Wd = 8.0 * W
     push = (w[PUSH_ITEMS] * (8 + Wd) + w[PUSH_EDGES] * 4 + w[PUSH_WEDGES] * 4 + w[BFS_WORDS] * 8 +
             w[SSSP_PAIRS] * 4 + w[IMPROVED] * 4 + w[NEW_WORDS] * 16 + w[PULL_VERTS] * (8 + Wd) +

@@ -210,7 +210,8 @@ __device__ __forceinline__ void prof_add(const KP& P, int slot, u64 x) {
 // the near-far statistics of its SSSP improvements (flushed whenever the
 // threshold is active).
 struct Tally {
-  u32 items = 0, edges = 0, wedges = 0, bfs = 0, nnew = 0, imp = 0;
+  u32 items = 0, edges = 0, wedges = 0, nnew = 0, imp = 0;
+  int32_t bfs = 0;  // (edge, word) visited reads; a lane's own share can be negative
   u32 ditems = 0, dedges = 0, pverts = 0, pwords = 0, pedges = 0;
   u64 sssp = 0;  // (edge, query) pairs: can pass 2^32 per lane
   u32 swords = 0;  // (edge, word with sparse SSSP bits) pairs
@@ -274,6 +275,8 @@ __device__ __forceinline__ void relax_edges(const KP& P, const int32_t (&u)[N], 
         for (int w = 0; w < W; ++w) {
           nx[i][w] = 0;
           add[i][w] = ~0ull;
+          // count_edges has counted every target's visited words as read.
+          if (P.profile) t.bfs -= ok[i] && bm(i, w) ? 1 : 0;
         }
         continue;
       }
@@ -386,7 +389,7 @@ __device__ __forceinline__ void count_edges(Tally& t, const u64 (&bm)[W], const 
     nq += (u32)__popcll(sm[w]);
   }
   t.edges += d;
-  t.bfs += d * nb;
+  t.bfs += (int32_t)(d * nb);
   t.swords += d * ns;
   t.sssp += (u64)d * nq;
   if (ns && weighted) t.wedges += d;
@@ -1478,7 +1481,7 @@ __device__ __forceinline__ void flush_tally(const KP& P, const Tally& t) {
   prof_add(P, PF_PUSH_ITEMS, t.items);
   prof_add(P, PF_PUSH_EDGES, t.edges);
   prof_add(P, PF_PUSH_WEDGES, t.wedges);
-  prof_add(P, PF_BFS_WORDS, t.bfs);
+  prof_add(P, PF_BFS_WORDS, (u64)(int64_t)t.bfs);
   prof_add(P, PF_SSSP_PAIRS, t.sssp);
   prof_add(P, PF_NEW_WORDS, t.nnew);
   prof_add(P, PF_IMPROVED, t.imp);
@@ -3172,7 +3175,9 @@ static bool run_iterations(cgp_engine* en, int W, bool no_graph, const std::func
 // natural width, counted once, no cache-line waste):
 //   frontier item (vertex or chunk): 8 (offset pair) + 8 W (frontier words)
 //   edge scanned lane-per-edge: 4 (column index) [+4 weight when SSSP bits are active]
-//   (edge, active BFS word): 8 (visited word of the target)
+//   (edge, active BFS word): 8 (visited word of the target), unless the target's
+//   done bit says that every BFS query has visited it (the bits, V / 8 bytes that
+//   stay in the caches, are not charged)
 //   (edge, active SSSP query): 4 (target value) ; lowered value: 4 (store)
 //   next word gaining bits: 16 (read + write of the next-frontier word)
 //   dense item: 8 (offset pair) + 8 (frontier word); dense edge: 4 index + 4 weight

@@ -125,7 +125,8 @@ typedef enum {
   CGP_WORK_PUSH_ITEMS = 0,  /* frontier items expanded lane-per-edge (vertex or edge chunk) */
   CGP_WORK_PUSH_EDGES = 1,  /* edges scanned lane-per-edge */
   CGP_WORK_PUSH_WEDGES = 2, /* ... of which read a weight (SSSP bits active) */
-  CGP_WORK_BFS_WORDS = 3,   /* (edge, active BFS mask word) visited reads */
+  CGP_WORK_BFS_WORDS = 3,   /* (edge, active BFS mask word) visited reads; targets known to be
+                               visited by every BFS query of the pass are not read */
   CGP_WORK_SSSP_PAIRS = 4,  /* (edge, active sparse SSSP query) target value reads */
   CGP_WORK_NEW_WORDS = 5,   /* next-frontier words that gained bits (push launch) */
   CGP_WORK_IMPROVED = 6,    /* (vertex, query) values lowered (push launch) */

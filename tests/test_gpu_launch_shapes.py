@@ -235,3 +235,34 @@ def test_bfs_output(gpu, V, n_sssp, renumber):
         en.run_batch(kinds, src, out=buf.view(shift * 4, len(kinds) * V * 4))
         got = buf.to_host()[shift:shift + len(kinds) * V].reshape(len(kinds), V)
         assert np.array_equal(got, exp), shift
+
+
+# The work counter of visited words: an edge of a frontier vertex reads one word
+# per mask word with frontier bits there, unless every BFS query has visited its
+# target and more than a sixteenth of the vertices are in that state (batch runs;
+# allocation-free runs keep no such bits and read them all).
+@pytest.mark.parametrize("n_bfs,n_sssp", [(1, 0), (40, 0), (100, 3), (200, 0)])
+@pytest.mark.parametrize("div", [1, 1 << 20])
+def test_visited_words_counted(gpu, n_bfs, n_sssp, div):
+    V = 2003
+    off, idx, wt = ring_graph(V, hub_degree=900, chords=4)
+    src = [(i * 131) % V for i in range(n_bfs + n_sssp)]
+    kinds = [BFS] * n_bfs + [SSSP] * n_sssp
+    og = O.G(off, idx, wt)
+    depth = np.stack([O.expected(og, BFS, s) for s in src[:n_bfs]]).astype(np.int64)
+    word = (np.arange(n_bfs) + n_sssp) // 64  # SSSP queries take the first slots
+    owner = np.repeat(np.arange(V), np.diff(off))
+    last = depth.max(axis=0)
+    every = read = 0
+    for it in range(int(depth.max()) + 1):
+        words = sum((depth[word == w] == it).any(axis=0).astype(np.int64) for w in range(word.max() + 1))
+        done = last <= it
+        edges = words[owner]
+        every += int(edges.sum())
+        read += int(edges[~done[idx]].sum()) if done.sum() > V // 16 else int(edges.sum())
+    assert read < every
+    en = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, idx, wt), profile=2, frontier_dense_div=div)
+    out = cgp_amd.DeviceBuffer(len(kinds) * V * 4)
+    for _ in range(2):
+        assert en.run_batch(kinds, src)[1]["work"][3] == read
+    assert en.run_batch_static(kinds, src, out)["work"][3] == every
