@@ -3634,7 +3634,10 @@ void engine_run_batch_static(cgp_engine* en, const cgp_query* queries, int32_t n
   } saved{en, {}, bufs, en->wcap, en->opts.profile, en->stamp_epoch};
   for (int k = 0; k < NB; ++k) {
     saved.own[k] = *bufs[k];
-    const size_t end = k + 1 < NB ? offs[k + 1] : L.total;
+    // A region ends where the next one starts (buffers of one region share it).
+    size_t end = L.total;
+    for (size_t o : offs)
+      if (o > offs[k]) end = std::min(end, o);
     bufs[k]->p = base + offs[k];
     bufs[k]->bytes = end - offs[k];
     bufs[k]->borrowed = true;
