@@ -3383,10 +3383,8 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
       if (R < 64 || hi > 32) fill_u32(en->s, wv, (size_t)V * R, INF, en->cus);
       else fill_row_prefix(en->s, wv, (size_t)V, hi > 16 ? 3 : 2, INF, en->cus);
     }
-    // Visited + next records (2W words per vertex) start clear; the layout
-    // depends on W, so the whole region is cleared for every pass.
+    // What a pass starts with at zero, whatever the last one left there.
     fill_u32(en->s, en->visited.p, en->record_bytes(W) / 4, 0u, en->cus);
-    en->next_dirty = false;
     dispatch_seed(en, W, P, (const int32_t*)en->slot_src.p, W * 64);
     en->tick(CAT_INIT, false);
     // The pass's output: query-major rows from the value rows, visited records
@@ -3463,7 +3461,6 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
       st.dense_launches += (int64_t)hc.den_launches;
     }
     en->stamp_epoch += hc.iter + 2;
-    if (hc.max_iter != 0 && hc.iter >= hc.max_iter) en->next_dirty = true;  // truncated run
     if (!out_done) emit_output();
   }
   if (!wcc.empty()) {

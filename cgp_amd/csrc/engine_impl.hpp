@@ -166,7 +166,6 @@ struct cgp_engine {
   // Replays the engine's last pass took to finish: the next pass enqueues its
   // output behind that replay, before reading the control block back.
   int spec_replay = 0;
-  bool next_dirty = false;
   bool busy = false;
   std::mutex mu;
   // Captured iteration graphs, one per mask-word width and set of optional
@@ -286,7 +285,9 @@ struct cgp_engine {
   // Bytes of the per-vertex done bits.
   size_t done_bytes() const { return ((size_t)g->V + 127) / 128 * 16; }
   // Bytes of a pass of W words that start at zero: visited + next records, done
-  // bits, and with postponing the far words.
+  // bits, and with postponing the far words.  Every pass and every session
+  // clears them itself: the layout depends on W, and a run that was cut, or a
+  // session that was stopped, leaves bits behind.
   size_t record_bytes(int W) const {
     const size_t V = (size_t)g->V;
     return V * W * 16 + done_bytes() + (opts.sssp_delta != 0 ? V * W * 8 : 0);

@@ -376,10 +376,8 @@ void serve_free(cgp_engine* en) {
   ss->d_src.release();
   ss->wcc_lab.release();
   ss->wcc_minid.release();
-  // Stamps used by the session must not recur in later runs; slots may hold
-  // bits in next[] when stopped mid-run.
+  // Stamps used by the session must not recur in later runs.
   en->stamp_epoch += ss->iter + 2;
-  en->next_dirty = true;
   delete ss;
   en->serve = nullptr;
 }
@@ -448,7 +446,6 @@ cgp_status cgp_serve_start(cgp_engine* en, const cgp_serve_opts* so) {
     // Clean slot state: every value row INF, no visited bits, no pending next bits.
     fill_u32(en->s, en->vals.p, vals_elems, INF, en->cus);
     fill_u32(en->s, en->visited.p, en->record_bytes(W) / 4, 0u, en->cus);  // records, far words
-    en->next_dirty = false;
     Cfg& cfg = *en->h_cfg;
     std::memset(&cfg, 0, sizeof(Cfg));
     en->narrow_binned = 0;
