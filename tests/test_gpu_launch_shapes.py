@@ -266,3 +266,20 @@ def test_visited_words_counted(gpu, n_bfs, n_sssp, div):
     for _ in range(2):
         assert en.run_batch(kinds, src)[1]["work"][3] == read
     assert en.run_batch_static(kinds, src, out)["work"][3] == every
+
+
+# The same two-level count in sparse mode: one vertex touches more than 32
+# workgroups' share of vertices, fewer than the graph has, and each of those
+# leads on.
+@pytest.mark.parametrize("touched", [32 * 1024, 32 * 1024 + 1, 35000])
+@pytest.mark.parametrize("n_bfs", [3, 70])
+def test_filter_workgroups_of_a_touched_list(gpu, touched, n_bfs):
+    V = 70001
+    mid = 2 + (np.arange(touched) * 1.5).astype(np.int64)
+    src = np.concatenate([[0], np.full(touched, 1), mid])
+    dst = np.concatenate([[1], mid, mid + 1 + mid % 2 * 9000])
+    off = np.zeros(V + 1, np.int64)
+    np.add.at(off, src + 1, 1)
+    wt = ((src * 7 + dst) % 13 + 1).astype(np.uint32)
+    check(np.cumsum(off).astype(np.int32), dst.astype(np.int32), wt, [BFS] * n_bfs + [SSSP] * 2,
+          [i % 2 for i in range(n_bfs + 2)], frontier_dense_div=1)

@@ -131,3 +131,47 @@ def test_automatic_step(gpu, graph, on):
         got = en.run_batch([SSSP] * 5, sources)[0]
         for i, s in enumerate(sources):
             assert np.array_equal(got[i], O.expected(og, SSSP, s)), (i, s)
+
+
+# Allocation-free runs: the far words lie behind the records in the fixed array.
+# Wide and narrow batches in turn on one engine, several passes, an odd number of
+# vertices.
+@pytest.mark.parametrize("V", [63, 1501, 5001])
+@pytest.mark.parametrize("opts", [dict(), dict(max_words=1), dict(frontier_dense_div=1, dense_threshold=1)],
+                         ids=["default", "passes", "rows"])
+def test_static_runs(gpu, V, opts):
+    rng = np.random.RandomState(V)
+    a, b = np.arange(V), np.roll(np.arange(V), -1)
+    a, b = np.concatenate([a, rng.randint(0, V, V)]), np.concatenate([b, rng.randint(0, V, V)])
+    w = rng.randint(1, 98, len(a))
+    off, idx, wt = csr(V, np.concatenate([a, b]), np.concatenate([b, a]), np.concatenate([w, w]))
+    og = O.G(off, idx, wt)
+    en = cgp_amd.Engine(cgp_amd.Graph.from_csr(off, idx, wt), sssp_delta=60, **opts)
+    out = cgp_amd.DeviceBuffer(150 * V * 4)
+    for n in (150, 3, 70, 1, 150):
+        kinds = [SSSP if i % 3 else BFS for i in range(n)]
+        src = [(i * 31 + n) % V for i in range(n)]
+        en.run_batch_static(kinds, src, out)
+        got = out.to_host(shape=(150, V))
+        for i, (k, s) in enumerate(zip(kinds, src)):
+            assert np.array_equal(got[i], O.expected(og, k, s)), (n, i, k, s)
+
+
+# The push launch, which takes up the far set, on a second stream beside the
+# lane-per-query launch; captured, launched directly, and in a session.
+@pytest.mark.parametrize("n", [5, 40, 150])
+@pytest.mark.parametrize("opts", [dict(), dict(use_hip_graph=0), dict(dense_threshold=1)],
+                         ids=["graph", "direct", "rows"])
+def test_concurrent_advance(gpu, n, opts):
+    h = cgp_amd.HostCSR.grid(45, 51, p_extra=0.01, seed=9, wmin=1, wmax=1000)
+    og = O.G.of(h)
+    en = cgp_amd.Engine(cgp_amd.Graph.from_host(h), sssp_delta=700, concurrent_advance=1, **opts)
+    src = [int(s) for s in h.sample_sources(n, seed=n)]
+    queries = [(BFS if i % 5 == 4 else SSSP, s) for i, s in enumerate(src)]
+    exp = [O.expected(og, k, s) for k, s in queries]
+    for _ in range(2):
+        got = en.run_batch([k for k, _ in queries], src)[0]
+        assert np.array_equal(got, np.stack(exp))
+    done = serve(en, queries, 64)
+    for i in range(n):
+        assert np.array_equal(done[i]["result"], exp[i]), i
