@@ -236,11 +236,12 @@ __device__ __forceinline__ void note_improved(Tally& t, u32 c, u32 thr) {
 //
 // In dense mode edges without BFS bits (any_b false) read no record: their
 // improved SSSP bits go to next by a fire-and-forget atomicOr, so the record's
-// line is touched only for an improvement, not for every edge scanned.  (A
-// per-vertex byte of "BFS words every running query has visited", kept by the
-// filter to skip the record read too, cut the visited tests of the RMAT-22
-// mixed batch by 39 % but not its traffic: the skipped records were cache
-// hits, and the extra dependent load made 160 BFS 0.5 ms slower.)
+// line is touched only for an improvement, not for every edge scanned.  Targets
+// whose bit in `done` says that every BFS query has visited them need no record
+// either.  (The lookup is a load before the others, so it has to be cheap and
+// rarely in vain: a byte per vertex looked up from the first iteration on made
+// 160 BFS on RMAT-22 0.5 ms slower; one bit, in every XCD's L2, looked up from
+// a sixteenth of the vertices on, makes it 0.4 ms faster.)
 //
 // The step is as much bound by instruction issue as by memory (a 64-edge step
 // of a BFS scan of RMAT-22 has about 1600 cycles of its SIMD, and 100 vector
@@ -256,7 +257,6 @@ __device__ __forceinline__ void relax_edges(const KP& P, const int32_t (&u)[N], 
   // nx: bits that next[v] already has; add: bits to set there.
   u64 nx[N][W], add[N][W];
   if (SPARSE || any_b) {
-    // Targets that every BFS query has visited need no record.
     u32 dn[N];
     if (done) {
 #pragma unroll
@@ -3417,11 +3417,12 @@ void engine_run_batch(cgp_engine* en, const cgp_query* queries, int32_t n, uint3
           hipLaunchKernelGGL((k_output_bfs<8>), grid, dim3(BLOCK), 0, en->s, (const u64*)en->visited.p,
                              (const int32_t*)g->inv, V, W, (const int32_t*)en->qmap.p, om, dout);
       }
-      if (!direct || tile_word)
-      hipLaunchKernelGGL(k_output, dim3((V + OUT_VT - 1) / OUT_VT, Wused), dim3(BLOCK),
-                         (size_t)om.n_planes * OUT_VT * sizeof(u64), en->s, (const u32*)en->vals.p,
-                         (const u64*)en->visited.p, (const int32_t*)g->inv, V, W, rshift,
-                         (const int32_t*)en->qmap.p, om, dout, vec, direct ? 1 : 0);
+      if (!direct || tile_word) {
+        hipLaunchKernelGGL(k_output, dim3((V + OUT_VT - 1) / OUT_VT, Wused), dim3(BLOCK),
+                           (size_t)om.n_planes * OUT_VT * sizeof(u64), en->s, (const u32*)en->vals.p,
+                           (const u64*)en->visited.p, (const int32_t*)g->inv, V, W, rshift,
+                           (const int32_t*)en->qmap.p, om, dout, vec, direct ? 1 : 0);
+      }
       HIP_CHECK(hipGetLastError());
       en->tick(CAT_OUT, false);
     };

@@ -44,20 +44,23 @@ constexpr int MAXW = 8;          // mask words per pass (512 slots)
 constexpr int MAXPLANES = 32;    // BFS depth bit planes (depths below 2^32)
 constexpr u32 INF = 0xFFFFFFFFu;
 constexpr int BLOCK = 256;       // workgroup size of every kernel (4 waves)
-constexpr int LCHUNK = 4096;     // edges per large-bin workgroup item
-// Edges per dense lane-per-query wave item.  A wave claims 64 items at a
-// time, so the chunk bounds the work of the last claims of a launch: on
-// RMAT-22 (80 SSSP) 1024 / 512 / 256 / 128 / 64 edges measured 37.2 / 32.1 /
-// 29.6 / 28.8 / 30.0 ms of lane-per-query time per batch.
+constexpr int LCHUNK = 4096;     // edges per large-bin item, which two to 32 waves share
+// Edges per dense lane-per-query item.  A wave claims up to 64 items at a time
+// (fewer on short lists, down to an eighth of one), so the chunk bounds the work
+// of the last claims of a launch: on RMAT-22 (80 SSSP) 1024 / 512 / 256 / 128 /
+// 64 edges measured 37.2 / 32.1 / 29.6 / 28.8 / 30.0 ms of lane-per-query time
+// per batch.
 constexpr int DCHUNK = 128;
 constexpr int NPROF = 18;
 constexpr int PULL_WAVE_DEG = 64;  // pull: vertices above this degree get a whole wave
 constexpr int PCHUNK = 256;        // edges per SSSP pull item
-// Work lists are split into NSHARD contiguous shards, one per XCD of the
-// MI355X (workgroups are placed on the XCDs round-robin), each with its own
-// cursor: a wave takes work from its own XCD's shard first, so the shard's
-// CSR rows and source rows stay in that XCD's L2, and the cursors' atomics
-// spread over NSHARD lines instead of one.
+// Work lists are split into NSHARD shards, one per XCD of the MI355X (workgroups
+// are placed on the XCDs round-robin), each with its own cursor: a wave takes
+// work from its own XCD's shard first, and the cursors' atomics spread over
+// NSHARD lines instead of one.  Shards are contiguous where neighbouring units
+// share CSR rows and value rows, which then stay in that XCD's L2; on skewed
+// graphs the push launch's large and medium lists, and the lane-per-query claims
+// always, go to the shards in turn, so that each has its part of the heavy units.
 constexpr int NSHARD = 8;
 enum : int { SH_M = 0, SH_S, SH_L, SH_D, SH_N, SH_P, NSH };
 // Ctl::bfs_pull: top-down, bottom-up, or not at all (the iteration limit is

@@ -79,8 +79,9 @@ typedef struct {
                                   it); BFS queries stop at this depth all the same */
   int32_t max_words;           /* cap on 64-bit mask words per pass; 0 = tuned */
   int32_t block_size;          /* workgroup size of the advance kernel: 128, 256 or 512; 0 = default 256 */
-  int32_t bin_small;           /* degree <= bin_small: 8 lanes per vertex; 0 = tuned */
-  int32_t bin_large;           /* degree > bin_large: one workgroup per vertex; 0 = tuned */
+  int32_t bin_small;           /* degree <= bin_small: up to 64 vertices per wave; 0 = tuned */
+  int32_t bin_large;           /* degree > bin_large: 4096-edge chunks, several waves each; between
+                                  the two a wave, or a part of one, per vertex; 0 = tuned */
   int32_t use_hip_graph;       /* capture iterations into a hipGraph (default 1) */
   int32_t graph_iterations;    /* iterations per captured graph launch (default 8) */
   int32_t profile;             /* bit 0: per-launch HIP events (also inside graph replays);
@@ -106,10 +107,10 @@ typedef struct {
                                   postponing off (sssp_delta 0) */
   int32_t advance_blocks;      /* workgroups of the advance launches (256-thread equivalents);
                                   0 = one per 16384 edges, between 2 and 3 per CU */
-  int32_t sssp_delta;          /* SSSP near-far step: frontier pairs whose value is >= a threshold
-                                  wait; the threshold moves to the smallest waiting value + delta
-                                  when nothing below it is left.  0 = no waiting (Bellman-Ford
-                                  frontier); -1 (default) = automatic: 20 x mean edge weight on
+  int32_t sssp_delta;          /* SSSP near-far step: pairs lowered to a value >= a threshold wait
+                                  outside the frontier; the threshold moves to the smallest waiting
+                                  value + delta when nothing below it is left.  0 = no waiting
+                                  (Bellman-Ford frontier); -1 (default) = automatic: 20 x mean edge weight on
                                   weighted graphs of average degree <= 8 unless vertices of at
                                   least 32 x that degree hold a twentieth of the edges, else 0.
                                   Results are identical either way. */
