@@ -2165,7 +2165,7 @@ __global__ __launch_bounds__(BLOCK) void k_filter(KP P) {
     // threshold is followed by one) expands no SSSP pair, so it does not count
     // towards the iteration limit of the SSSP queries; BFS queries do advance
     // in it, and stop at the limit by themselves.
-    const u32 limit = C->max_iter, raises_run = C->bumps;
+    const u32 limit = C->max_iter, raises_run = limit ? C->bumps : 0u;
     u32 pull = BFS_PUSH;
     if (limit != 0 && next_iter >= limit) {
       pull = BFS_OVER;
